@@ -17,15 +17,16 @@
 // mod 2^64.
 //
 // Tiling.  One MFMA v_mfma_i32_32x32x32_i8 covers 32 "digit rows" = 4 share
-// rows x 8 digits, ordered so that the 16 accumulator registers of a lane hold
-// all 8 digits of 2 share rows for its column (32x32 accumulator layout: lane l,
-// register r -> column l%32, row 8(r/4) + 4(l/32) + r%4).  The digit sum is
-// therefore formed in registers with no cross-lane traffic.  A workgroup of 4
-// waves computes 32 share rows x 128 columns; each wave 16 rows x 64 columns
-// (8 MFMAs per 32-wide K step).  Shares are staged in LDS as 8 digit planes
-// (byte transpose with v_perm), weights as int8 rows; both with an 80-byte row
-// pitch so the 16-byte operand reads are bank-conflict free.
+// rows x 8 digits (32x32 accumulator layout: lane l, register r -> column l%32,
+// row 8(r/4) + 4(l/32) + r%4), so that a lane holds, for its column, four
+// digits of each share row and the digit sum is formed in registers with one
+// exchange across the wave's halves.  Large products run as 32-row x 128- or
+// 192-column tiles (LDS DMA, or staged through registers), products of few
+// rows on a kernel that splits K over the waves of a workgroup.
 #include "kernels.hpp"
+#include "praghip.h"
+
+#include <vector>
 
 namespace praghip {
 
@@ -63,171 +64,39 @@ struct TileRegs {
   uint32_t wb[8];
 };
 
-template <int WB>
 __device__ __forceinline__ void load_tile(TileRegs& tr, const uint64_t* __restrict__ xrow, bool x_row_ok,
-                                          const void* __restrict__ wv, size_t wrow_off, bool w_row_ok, int k0, int K,
-                                          int ak, int wk, int wdigit, int w_vec) {
+                                          const int8_t* __restrict__ wrow, bool w_row_ok, int k0, int K, int ak, int wk,
+                                          int w_vec) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int kk = k0 + ak + e;
     tr.xs[e] = (x_row_ok && kk < K) ? xrow[kk] : 0;
   }
   const int kk = k0 + wk;
-  if (WB == 8) {
-    const int8_t* wrow = static_cast<const int8_t*>(wv) + wrow_off;
-    if (w_row_ok && kk + 32 <= K && w_vec) {
-      const uint4 a = *reinterpret_cast<const uint4*>(wrow + kk);
-      const uint4 b = *reinterpret_cast<const uint4*>(wrow + kk + 16);
-      tr.wb[0] = a.x; tr.wb[1] = a.y; tr.wb[2] = a.z; tr.wb[3] = a.w;
-      tr.wb[4] = b.x; tr.wb[5] = b.y; tr.wb[6] = b.z; tr.wb[7] = b.w;
-    } else {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        uint32_t word = 0;
-#pragma unroll
-        for (int bb = 0; bb < 4; ++bb) {
-          const int kq = kk + 4 * q + bb;
-          const uint32_t byte = (w_row_ok && kq < K) ? uint8_t(wrow[kq]) : 0u;
-          word |= byte << (8 * bb);
-        }
-        tr.wb[q] = word;
-      }
-    }
+  if (w_row_ok && kk + 32 <= K && w_vec) {
+    const uint4 a = *reinterpret_cast<const uint4*>(wrow + kk);
+    const uint4 b = *reinterpret_cast<const uint4*>(wrow + kk + 16);
+    tr.wb[0] = a.x; tr.wb[1] = a.y; tr.wb[2] = a.z; tr.wb[3] = a.w;
+    tr.wb[4] = b.x; tr.wb[5] = b.y; tr.wb[6] = b.z; tr.wb[7] = b.w;
   } else {
-    const int32_t* wrow = static_cast<const int32_t*>(wv) + wrow_off;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       uint32_t word = 0;
 #pragma unroll
       for (int bb = 0; bb < 4; ++bb) {
         const int kq = kk + 4 * q + bb;
-        const int wvv = (w_row_ok && kq < K) ? wrow[kq] : 0;
-        word |= uint32_t(uint8_t(weight_digit(wvv, wdigit))) << (8 * bb);
+        const uint32_t byte = (w_row_ok && kq < K) ? uint8_t(wrow[kq]) : 0u;
+        word |= byte << (8 * bb);
       }
       tr.wb[q] = word;
     }
   }
 }
 
-// Two workgroups per CU (two waves per SIMD, accumulators in VGPRs): while
-// one waits on memory the other runs MFMAs.  Within a workgroup the next K
-// step's global loads are issued before the current step's MFMAs.
-template <int WB>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    share_gemm_kernel(const uint64_t* __restrict__ x, const void* __restrict__ wv, const int8_t* __restrict__ shifts,
-                      uint64_t* __restrict__ y, int M, int K, int N, uint64_t mask, int wdigit, int accumulate,
-                      int w_vec) {
-  __shared__ __attribute__((aligned(16))) uint8_t a_lds[8][kBM][kPitch];
-  __shared__ __attribute__((aligned(16))) uint8_t w_lds[kBN][kPitch];
-  __shared__ int csum[kThreads];
-
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
-
-  // share-tile loader: row ar, 8 consecutive k from ak
-  const int ar = t >> 3, ak = (t & 7) * 8;
-  // weight-tile loader: row wr, 32 consecutive k from wk
-  const int wr = t >> 1, wk = (t & 1) * 32;
-  int colsum = 0;
-
-  // MFMA operand coordinates of this lane
-  const int i = lane & 31, khalf = lane >> 5;
-  const int a_row_in_block = 2 * ((i >> 2) & 1) + (i >> 4);
-  const int a_digit = 4 * ((i >> 3) & 1) + (i & 3);
-
-  v16i acc[4][2];
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = v16i{0};
-
-  const bool x_row_ok = (m0 + ar) < M;
-  const bool w_row_ok = (n0 + wr) < N;
-  const uint64_t* xrow = x + size_t(m0 + ar) * K;
-  const size_t wrow_off = size_t(n0 + wr) * K;
-
-  TileRegs tr;
-  load_tile<WB>(tr, xrow, x_row_ok, wv, wrow_off, w_row_ok, 0, K, ak, wk, wdigit, w_vec);
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    // ---- shares -> 8 offset-binary digit planes
-    uint32_t d[16];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      d[2 * e] = uint32_t(tr.xs[e]) ^ 0x80808080u;
-      d[2 * e + 1] = uint32_t(tr.xs[e] >> 32) ^ 0x80808080u;
-    }
-    uint32_t o[4][4];
-    transpose4(d[0], d[2], d[4], d[6], o[0][0], o[0][1], o[0][2], o[0][3]);      // digits 0-3, k 0-3
-    transpose4(d[8], d[10], d[12], d[14], o[1][0], o[1][1], o[1][2], o[1][3]);   // digits 0-3, k 4-7
-    transpose4(d[1], d[3], d[5], d[7], o[2][0], o[2][1], o[2][2], o[2][3]);      // digits 4-7, k 0-3
-    transpose4(d[9], d[11], d[13], d[15], o[3][0], o[3][1], o[3][2], o[3][3]);   // digits 4-7, k 4-7
-#pragma unroll
-    for (int dg = 0; dg < 4; ++dg) {
-      *reinterpret_cast<uint2*>(&a_lds[dg][ar][ak]) = make_uint2(o[0][dg], o[1][dg]);
-      *reinterpret_cast<uint2*>(&a_lds[dg + 4][ar][ak]) = make_uint2(o[2][dg], o[3][dg]);
-    }
-    // ---- weights (digit `wdigit` of each) -> int8 rows
-#pragma unroll
-    for (int q = 0; q < 8; ++q) colsum = __builtin_amdgcn_sdot4(int(tr.wb[q]), 0x01010101, colsum, false);
-    *reinterpret_cast<uint4*>(&w_lds[wr][wk]) = make_uint4(tr.wb[0], tr.wb[1], tr.wb[2], tr.wb[3]);
-    *reinterpret_cast<uint4*>(&w_lds[wr][wk + 16]) = make_uint4(tr.wb[4], tr.wb[5], tr.wb[6], tr.wb[7]);
-    __syncthreads();
-    // ---- next step's loads, in flight during the MFMAs
-    if (k0 + kBK < K) load_tile<WB>(tr, xrow, x_row_ok, wv, wrow_off, w_row_ok, k0 + kBK, K, ak, wk, wdigit, w_vec);
-
-    // ---- MFMA over the two 32-wide K steps
-#pragma unroll
-    for (int ks = 0; ks < kBK / 32; ++ks) {
-      const int kb = ks * 32 + khalf * 16;
-      v4i bop[2];
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) bop[cb] = *reinterpret_cast<const v4i*>(&w_lds[wn * 64 + cb * 32 + i][kb]);
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb) {
-        const v4i aop = *reinterpret_cast<const v4i*>(&a_lds[a_digit][wm * 16 + rb * 4 + a_row_in_block][kb]);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-          acc[rb][cb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, bop[cb], acc[rb][cb], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- epilogue: column sums, digit recombination, shift, mask
-  csum[t] = colsum;
-  __syncthreads();
-  const int shift_e = 8 * wdigit;
-#pragma unroll
-  for (int cb = 0; cb < 2; ++cb) {
-    const int cl = wn * 64 + cb * 32 + i;
-    const int col = n0 + cl;
-    if (col >= N) continue;
-    const int64_t s_n = int64_t(csum[2 * cl]) + int64_t(csum[2 * cl + 1]);
-    const uint64_t corr = 0x8080808080808080ull * uint64_t(s_n);
-    const int sh = shift_e + (shifts ? int(shifts[col]) : 0);
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const int row = m0 + wm * 16 + rb * 4 + 2 * khalf + a;
-        if (row >= M) continue;
-        uint64_t v = corr;
-#pragma unroll
-        for (int dg = 0; dg < 8; ++dg) v += uint64_t(int64_t(acc[rb][cb][8 * a + dg])) << (8 * dg);
-        v = sh < 64 ? (v << sh) : 0;
-        uint64_t* dst = y + size_t(row) * N + col;
-        if (accumulate) v += *dst;
-        *dst = v & mask;
-      }
-    }
-  }
-}
-
 // ------------------------------------------------------------- VALU form
 // The same product with VALU dot products instead of the matrix cores: the
-// tiles are staged exactly as in share_gemm_kernel (digit planes of the
-// offset-binary share bytes, int8 weight rows), and each thread forms a 4 x 4
+// tiles are staged as digit planes of the offset-binary share bytes (byte
+// transpose with v_perm) and int8 weight rows, and each thread forms a 4 x 4
 // block of outputs with v_dot4_i32_i8, one per (row, column, digit) and four
 // k.  It exists as the measured alternative to the MFMA kernels (int8
 // weights).
@@ -252,9 +121,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       for (int d = 0; d < 8; ++d) acc[i][j][d] = 0;
   const bool x_row_ok = (m0 + ar) < M, w_row_ok = (n0 + wr) < N;
   const uint64_t* xrow = x + size_t(m0 + ar) * K;
-  const size_t wrow_off = size_t(n0 + wr) * K;
+  const int8_t* wrow = w + size_t(n0 + wr) * K;
   TileRegs tr;
-  load_tile<8>(tr, xrow, x_row_ok, w, wrow_off, w_row_ok, 0, K, ak, wk, 0, w_vec);
+  load_tile(tr, xrow, x_row_ok, wrow, w_row_ok, 0, K, ak, wk, w_vec);
   for (int k0 = 0; k0 < K; k0 += kBK) {
     uint32_t d[16];
 #pragma unroll
@@ -295,7 +164,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     __syncthreads();
     // the next step's tile is loaded after the dot products (the 128
     // accumulators leave no registers to hold it during them)
-    if (k0 + kBK < K) load_tile<8>(tr, xrow, x_row_ok, w, wrow_off, w_row_ok, k0 + kBK, K, ak, wk, 0, w_vec);
+    if (k0 + kBK < K) load_tile(tr, xrow, x_row_ok, wrow, w_row_ok, k0 + kBK, K, ak, wk, w_vec);
   }
   csum[t] = colsum;
   __syncthreads();
@@ -409,26 +278,10 @@ __device__ __forceinline__ void dma_issue(const DmaCtx& c, int k0, RAW& raw, WT&
   for (int j = 0; j < CB; ++j) dma16(c.wsrc[j] + k0, &wt[(16 * (CB * c.wave + j)) * kBK]);
 }
 
-// Three stages: step s computes on stage s % 3 while the DMAs of steps s + 1
-// (issued one step earlier) and s + 2 (issued here, into the stage step s - 1
-// read) are in flight.
-template <int CB, class RAW, class WT, class RAWN, class WTN>
-__device__ __forceinline__ void dma_step(const DmaCtx& c, bool ahead, bool next, int k_next, const RAW& raw,
-                                         const WT& wt, RAWN& raw_n, WTN& wt_n, int (&colsum)[CB],
-                                         v16i (&acc)[4][CB]) {
-  // this wave's DMAs for this step are done: loads complete in order, and
-  // `ahead` says whether the next step's 4 + CB are still allowed in flight;
-  // after the barrier every wave's are, and every wave has finished reading
-  // the stage the new DMAs overwrite
-  if (ahead) {
-    if (CB == 2)
-      asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(7)\n\ts_barrier" ::: "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  }
-  if (next) dma_issue<CB>(c, k_next, raw_n, wt_n);
+// One K step of MFMAs on stage buffers (raw, wt).
+template <int CB, class RAW, class WT>
+__device__ __forceinline__ void mfma_step(const DmaCtx& c, const RAW& raw, const WT& wt, int (&colsum)[CB],
+                                          v16i (&acc)[4][CB]) {
   // ---- every operand of the step first (16 transpose reads, 2 CB weight
   // reads), so that the MFMAs then issue back to back behind one LDS wait
   v4i aop[kBK / 32][4], bop[kBK / 32][CB];
@@ -469,6 +322,29 @@ __device__ __forceinline__ void dma_step(const DmaCtx& c, bool ahead, bool next,
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) colsum[cb] = __builtin_amdgcn_sdot4(bop[ks][cb][e], 0x01010101, colsum[cb], false);
+}
+
+// Three stages: step s computes on stage s % 3 while the DMAs of steps s + 1
+// (issued one step earlier) and s + 2 (issued here, into the stage step s - 1
+// read) are in flight.
+template <int CB, class RAW, class WT, class RAWN, class WTN>
+__device__ __forceinline__ void dma_step(const DmaCtx& c, bool ahead, bool next, int k_next, const RAW& raw,
+                                         const WT& wt, RAWN& raw_n, WTN& wt_n, int (&colsum)[CB],
+                                         v16i (&acc)[4][CB]) {
+  // this wave's DMAs for this step are done: loads complete in order, and
+  // `ahead` says whether the next step's 4 + CB are still allowed in flight;
+  // after the barrier every wave's are, and every wave has finished reading
+  // the stage the new DMAs overwrite
+  if (ahead) {
+    if (CB == 2)
+      asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(7)\n\ts_barrier" ::: "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  if (next) dma_issue<CB>(c, k_next, raw_n, wt_n);
+  mfma_step<CB>(c, raw, wt, colsum, acc);
 }
 
 // Software-pipelined form (CB = 3, one wave per SIMD): each step runs as two
@@ -558,7 +434,7 @@ __device__ __forceinline__ int64_t mad_i64(int a, int m, int64_t c) {
   return r;
 }
 
-// Tile (tm, tn) of this workgroup in the gridDim.y x gridDim.x tile grid.
+// Tile (tm, tn) of workgroup t in a TM x TN tile grid.
 // Workgroups go to the 8 XCDs round robin (linear id mod 8), so when the grid
 // holds a multiple of 8 tiles XCD x is given the contiguous range
 // [x nt/8, (x+1) nt/8) of a grouped order (8 tile rows at a time, column by
@@ -566,9 +442,8 @@ __device__ __forceinline__ int64_t mad_i64(int a, int m, int64_t c) {
 // weight columns stay in that XCD's L2 (512 x 3072 in 32 x 192 tiles: each
 // XCD 8 x 4 tiles, 2 MiB of shares and 768 KiB of weights).  Any bijection
 // is correct; this one only places the reuse.
-__device__ __forceinline__ void tile_of(int& tm, int& tn) {
-  const int TN = int(gridDim.x), TM = int(gridDim.y), nt = TN * TM;
-  int t = int(blockIdx.y) * TN + int(blockIdx.x);
+__device__ __forceinline__ void tile_of(int& tm, int& tn, int TN, int TM, int t) {
+  const int nt = TN * TM;
   if (nt % 8 == 0) t = (t % 8) * (nt / 8) + t / 8;
   constexpr int G = 8;
   const int group = t / (G * TN), first = group * G, rows = min(G, TM - first);
@@ -624,30 +499,10 @@ __device__ __forceinline__ uint64_t column_correction(int colsum) {
   return 0x8080808080808080ull * uint64_t(int64_t(int(cs[0])) + int64_t(int(cs[1])));
 }
 
-// Weight planes: w holds `planes` int8 matrices [planes][N][K], plane e the
-// signed byte of weight digit e (planes = 1: int8 weights; 3: the pre-split
-// f12 weights).  Workgroup z takes plane z / splits and K split z % splits;
-// plane e's products enter y shifted by 8e.  CB = 2: 128-column tiles, two
-// workgroups (two waves per SIMD) per CU, whose waits overlap; CB = 3:
-// 192-column tiles, one workgroup per CU, 12 accumulator tiles per wave, so
-// that every MFMA takes fewer operand bytes from L2 and LDS.
+// Operand coordinates of this lane (everything of DmaCtx but the DMA sources).
 template <int CB>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CB == 2 ? 2 : 1, CB == 2 ? 2 : 1)))
-    share_gemm_dma_kernel(const uint64_t* __restrict__ x, const int8_t* __restrict__ w,
-                          const int8_t* __restrict__ shifts, uint64_t* __restrict__ y, int M, int K, int N,
-                          uint64_t mask, int k_split, int splits) {
-  constexpr int BN = 64 * CB;
-  const int plane = int(blockIdx.z) / splits, split_z = int(blockIdx.z) % splits;
-  w += size_t(plane) * size_t(N) * size_t(K);
-  __shared__ __attribute__((aligned(16))) uint8_t raw0[kBM * kRawRow];
-  __shared__ __attribute__((aligned(16))) uint8_t raw1[kBM * kRawRow];
-  __shared__ __attribute__((aligned(16))) uint8_t raw2[kBM * kRawRow];
-  __shared__ __attribute__((aligned(16))) uint8_t wt0[BN * kBK];
-  __shared__ __attribute__((aligned(16))) uint8_t wt1[BN * kBK];
-  __shared__ __attribute__((aligned(16))) uint8_t wt2[BN * kBK];
-
+__device__ __forceinline__ void lane_context(DmaCtx& c) {
   const int t = threadIdx.x, lane = t & 63;
-  DmaCtx c;
   c.wave = t >> 6;
   c.wm = c.wave >> 1;
   c.wn = c.wave & 1;
@@ -668,9 +523,27 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(C
     for (int ks = 0; ks < 2; ++ks)
       c.w_off[ks] = (c.wn * 32 * CB + c.i) * kBK + 16 * (2 * (ks ^ (f >> 1)) + (c.khalf ^ (f & 1)));
   }
-  int tm, tn;
-  tile_of(tm, tn);
-  const int m0 = tm * kBM, n0 = tn * BN;
+}
+
+// The tile at (m0, n0) over the K steps [k_begin, k_begin + 64 steps) of one
+// weight plane (w: its [N][K] bytes; its products enter y shifted by 8 plane).
+// split: the result is added into y by 64-bit atomics, unmasked.
+template <int CB>
+__device__ __forceinline__ void dma_tile(const uint64_t* __restrict__ x, const int8_t* __restrict__ w,
+                                         const int8_t* __restrict__ shifts, uint64_t* __restrict__ y, int M, int K,
+                                         int N, uint64_t mask, int m0, int n0, int k_begin, int steps, int plane,
+                                         bool split) {
+  constexpr int BN = 64 * CB;
+  __shared__ __attribute__((aligned(16))) uint8_t raw0[kBM * kRawRow];
+  __shared__ __attribute__((aligned(16))) uint8_t raw1[kBM * kRawRow];
+  __shared__ __attribute__((aligned(16))) uint8_t raw2[kBM * kRawRow];
+  __shared__ __attribute__((aligned(16))) uint8_t wt0[BN * kBK];
+  __shared__ __attribute__((aligned(16))) uint8_t wt1[BN * kBK];
+  __shared__ __attribute__((aligned(16))) uint8_t wt2[BN * kBK];
+
+  DmaCtx c;
+  lane_context<CB>(c);
+  const int lane = threadIdx.x & 63;
   // DMA sources of this lane: 4 raw-share instructions (2 rows of 512 B each)
   // and CB weight instructions (16 rows of 64 B each) per wave and step.
 #pragma unroll
@@ -696,11 +569,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(C
     for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = v16i{0};
   }
 
-  // split-K: workgroup z takes K steps [z k_split, (z+1) k_split); with more
-  // than one split the partial products are added into y (zeroed first) by
-  // 64-bit atomics, exact mod 2^64 in any order
-  const int k_begin = split_z * k_split;
-  const int steps = min(k_split, K - k_begin) / kBK;
   if constexpr (CB == 3) {
     auto raw_of = [&](int q) { return q == 0 ? raw0 : (q == 1 ? raw1 : raw2); };
     auto wt_of = [&](int q) { return q == 0 ? wt0 : (q == 1 ? wt1 : wt2); };
@@ -729,8 +597,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(C
     if (s + 2 < steps) dma_step<CB>(c, s + 3 < steps, s + 4 < steps, kn + 2 * kBK, raw2, wt2, raw1, wt1, colsum, acc);
   }
   }
-  const bool split = gridDim.z > 1;
-
   // ---- epilogue: column sums, digit recombination, shift, mask
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
@@ -740,6 +606,370 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(C
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
       store_tile(acc[rb][cb], m0 + c.wm * 16 + rb * 4, col, c.khalf, corr, sh, split, mask, y, M, N);
+  }
+}
+
+// Weight planes: w holds `planes` int8 matrices [planes][N][K], plane e the
+// signed byte of weight digit e (planes = 1: int8 weights; 3: the pre-split
+// f12 weights).  Workgroup z takes plane z / splits and K split z % splits;
+// plane e's products enter y shifted by 8e.  CB = 2: 128-column tiles, two
+// workgroups (two waves per SIMD) per CU, whose waits overlap; CB = 3:
+// 192-column tiles, one workgroup per CU, 12 accumulator tiles per wave, so
+// that every MFMA takes fewer operand bytes from L2 and LDS.
+// split-K: workgroup z takes K steps [z k_split, (z+1) k_split); with more
+// than one split the partial products are added into y (zeroed first) by
+// 64-bit atomics, exact mod 2^64 in any order.
+template <int CB>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CB == 2 ? 2 : 1, CB == 2 ? 2 : 1)))
+    share_gemm_dma_kernel(const uint64_t* __restrict__ x, const int8_t* __restrict__ w,
+                          const int8_t* __restrict__ shifts, uint64_t* __restrict__ y, int M, int K, int N,
+                          uint64_t mask, int k_split, int splits) {
+  const int plane = int(blockIdx.z) / splits, k_begin = (int(blockIdx.z) % splits) * k_split;
+  int tm, tn;
+  tile_of(tm, tn, int(gridDim.x), int(gridDim.y), int(blockIdx.y * gridDim.x + blockIdx.x));
+  dma_tile<CB>(x, w + size_t(plane) * size_t(N) * size_t(K), shifts, y, M, K, N, mask, tm * kBM, tn * 64 * CB, k_begin,
+               min(k_split, K - k_begin) / kBK, plane, gridDim.z > 1);
+}
+
+// ------------------------------------------------------- products of a batch
+// The tiles of up to kGroupMax independent products in one launch: workgroup
+// g takes tile g - first of the product whose range [first, first + tiles)
+// holds g.  Apart, each product pays its own launch, ring fill, epilogue and
+// last round of tiles (about 10 us of the 26 us of a 512-row Qwen3 product);
+// in one grid a CU's next tile, of whatever product, starts as soon as one of
+// its two workgroups ends, so fills and epilogues run beside other tiles'
+// MFMAs, and no product needs its K split (and the clear and the atomics of
+// one) to fill the chip.
+constexpr int kGroupMax = 32;
+struct GemmGroup {
+  struct Item {
+    const uint64_t* x;
+    const int8_t* w;
+    const int8_t* shifts;
+    uint64_t* y;
+    int M, K, N;
+    int mask_bits;
+    int tiles_n, tiles_m;
+    unsigned first;  // index of its first tile in the grid
+    int pad;
+  } item[kGroupMax];
+  int count;
+};
+__device__ __forceinline__ const GemmGroup::Item& group_item(const GemmGroup& g, unsigned tile) {
+  int lo = 0, hi = g.count;  // the last item whose first tile is at or below `tile`
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (g.item[mid].first <= tile)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  return g.item[lo];
+}
+__device__ __forceinline__ uint64_t group_mask(int bits) { return bits >= 64 ? ~0ull : (1ull << bits) - 1; }
+
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    share_gemm_group_kernel(GemmGroup g) {
+  const GemmGroup::Item& it = group_item(g, blockIdx.x);
+  int tm, tn;
+  tile_of(tm, tn, it.tiles_n, it.tiles_m, int(blockIdx.x - it.first));
+  dma_tile<2>(it.x, it.w, it.shifts, it.y, it.M, it.K, it.N, group_mask(it.mask_bits), tm * kBM, tn * kBN, 0,
+              it.K / kBK, 0, false);
+}
+
+// ------------------------------------------------- any K, any weight form
+// Weight forms of the kernels below: int8 rows, three int8 planes [3][N][K],
+// or int32 words in [-0x808080, 0x7F7F7F].  For those
+//   w + 0x808080 = sum_e b_e 256^e (bytes b_e),  w = sum_e (b_e - 128) 256^e,
+// so balanced digit e is byte e of w + 0x808080 with its top bit flipped.
+enum { kW8 = 0, kWPlanes = 1, kW32 = 2 };
+
+// 16 bytes from any address (one global_load_dwordx4: gfx950 loads need no
+// alignment).
+__device__ __forceinline__ uint4 load16(const void* p) {
+  uint4 v;
+  __builtin_memcpy(&v, (const __attribute__((address_space(1))) char*)(p), 16);
+  return v;
+}
+
+// Share words k, k + 1 of a row of K; zero past K.  Nothing past K is read.
+__device__ __forceinline__ uint4 load_x2(const uint64_t* row, int k, int K) {
+  if (k + 2 <= K) return load16(row + k);
+  if (k < K) {
+    const uint64_t v = row[k];
+    return make_uint4(uint32_t(v), uint32_t(v >> 32), 0, 0);
+  }
+  return make_uint4(0, 0, 0, 0);
+}
+
+// Weight bytes k .. k + 15 of a row of K; zero past K.  Nothing past K is
+// read: a piece that K cuts is taken from the 16 bytes that end at K.
+__device__ __forceinline__ uint4 load_w16(const int8_t* row, int k, int K) {
+  if (k + 16 <= K) return load16(row + k);
+  unsigned __int128 v = 0;
+  if (k < K) {
+    if (K >= 16) {
+      const uint4 t = load16(row + K - 16);
+      v = ((unsigned __int128)((uint64_t(t.w) << 32) | t.z) << 64) | ((uint64_t(t.y) << 32) | t.x);
+      v >>= 8 * (k + 16 - K);
+    } else {
+      for (int b = k; b < K; ++b) v |= (unsigned __int128)(uint8_t(row[b])) << (8 * (b - k));
+    }
+  }
+  const uint64_t lo = uint64_t(v), hi = uint64_t(v >> 64);
+  return make_uint4(uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32));
+}
+
+// int32 weights k .. k + 3 of a row of K; zero past K.
+__device__ __forceinline__ uint4 load_w4(const int32_t* row, int k, int K) {
+  if (k + 4 <= K) return load16(row + k);
+  return make_uint4(k < K ? row[k] : 0, k + 1 < K ? row[k + 1] : 0, k + 2 < K ? row[k + 2] : 0, 0);
+}
+
+// ------------------------------------------------------ register-staged tile
+// The 32 x 128 tile of the DMA kernel for operands its LDS DMA cannot take: K
+// not a multiple of 64, weight rows off 16 bytes, int32 weights.  The next K
+// step's words are loaded into registers during the current step's MFMAs and
+// written to the other of two LDS stages, in the DMA path's swizzled layout;
+// the MFMA part is the same.  One barrier per step: a stage is rewritten two
+// steps after it was read.  Workgroup z as in the DMA kernel.
+template <int WT>
+struct RegTile {
+  uint4 x[4], w[WT == kW32 ? 8 : 2];
+};
+
+template <int WT>
+__device__ __forceinline__ void reg_load(RegTile<WT>& r, const uint64_t* const (&xrow)[4], const void* const (&wrow)[2],
+                                         int kx, int kw, int K) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r.x[j] = load_x2(xrow[j], kx, K);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if constexpr (WT == kW32) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) r.w[4 * j + q] = load_w4(static_cast<const int32_t*>(wrow[j]), kw + 4 * q, K);
+    } else {
+      r.w[j] = load_w16(static_cast<const int8_t*>(wrow[j]), kw, K);
+    }
+  }
+}
+
+// Balanced digit e of four int32 weights as four bytes (sel: byte e of both
+// v_perm operands).
+__device__ __forceinline__ uint32_t digit4(uint4 w, uint32_t sel) {
+  const uint32_t o = 0x808080u;
+  const uint32_t lo = __builtin_amdgcn_perm(w.y + o, w.x + o, sel), hi = __builtin_amdgcn_perm(w.w + o, w.z + o, sel);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ 0x80808080u;
+}
+
+template <int WT>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    share_gemm_reg_kernel(const uint64_t* __restrict__ x, const void* __restrict__ wv,
+                          const int8_t* __restrict__ shifts, uint64_t* __restrict__ y, int M, int K, int N,
+                          uint64_t mask, int k_split, int splits) {
+  constexpr int CB = 2;
+  __shared__ __attribute__((aligned(16))) uint8_t raw[2][kBM * kRawRow];
+  __shared__ __attribute__((aligned(16))) uint8_t wt[2][kBN * kBK];
+  const int plane = int(blockIdx.z) / splits, k_begin = (int(blockIdx.z) % splits) * k_split;
+  const int k_end = min(k_begin + k_split, K);
+  int tm, tn;
+  tile_of(tm, tn, int(gridDim.x), int(gridDim.y), int(blockIdx.y * gridDim.x + blockIdx.x));
+  const int m0 = tm * kBM, n0 = tn * kBN;
+  DmaCtx c;
+  lane_context<CB>(c);
+  const int lane = threadIdx.x & 63, xc = lane & 31, wc = lane & 3;
+  const uint64_t* xrow[4];
+  const void* wrow[2];
+  int x_at[4], w_at[2];  // this lane's LDS slots
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = 2 * (4 * c.wave + j) + (lane >> 5);
+    xrow[j] = x + size_t(min(m0 + row, M - 1)) * K;  // rows past M: any valid row, results dropped
+    x_at[j] = row * kRawRow + ((xc ^ (4 * (row & 7))) << 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = 16 * (2 * c.wave + j) + (lane >> 2);
+    const size_t off = size_t(min(n0 + row, N - 1)) * K;
+    wrow[j] = WT == kW32 ? static_cast<const void*>(static_cast<const int32_t*>(wv) + off)
+                         : static_cast<const void*>(static_cast<const int8_t*>(wv) + off + size_t(plane) * N * K);
+    w_at[j] = row * kBK + ((wc ^ wt_swizzle(row)) << 4);
+  }
+  const uint32_t sel = 0x0c0c0400u + 0x0101u * unsigned(plane);
+  int colsum[CB];
+  v16i acc[4][CB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    colsum[cb] = 0;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = v16i{0};
+  }
+  RegTile<WT> r;
+  reg_load<WT>(r, xrow, wrow, k_begin + 2 * xc, k_begin + 16 * wc, k_end);
+  const auto step = [&](uint8_t* rs, uint8_t* ws, int k) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(rs + x_at[j]) = r.x[j];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (WT == kW32)
+        *reinterpret_cast<uint4*>(ws + w_at[j]) = make_uint4(digit4(r.w[4 * j], sel), digit4(r.w[4 * j + 1], sel),
+                                                             digit4(r.w[4 * j + 2], sel), digit4(r.w[4 * j + 3], sel));
+      else
+        *reinterpret_cast<uint4*>(ws + w_at[j]) = r.w[j];
+    }
+    __syncthreads();
+    const int kn = k + kBK;
+    if (kn < k_end) reg_load<WT>(r, xrow, wrow, kn + 2 * xc, kn + 16 * wc, k_end);
+    mfma_step<CB>(c, static_cast<const uint8_t*>(rs), static_cast<const uint8_t*>(ws), colsum, acc);
+  };
+  for (int k = k_begin; k < k_end; k += 2 * kBK) {
+    step(raw[0], wt[0], k);
+    if (k + kBK < k_end) step(raw[1], wt[1], k + kBK);
+  }
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const int col = n0 + c.wn * 32 * CB + cb * 32 + c.i;
+    const uint64_t corr = column_correction(colsum[cb]);
+    const int sh = 8 * plane + (shifts && col < N ? int(shifts[col]) : 0);
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+      store_tile(acc[rb][cb], m0 + c.wm * 16 + rb * 4, col, c.khalf, corr, sh, gridDim.z > 1, mask, y, M, N);
+  }
+}
+
+// ---------------------------------------------------------------- few rows
+// Products of few share rows (decoding, short prompts) read every weight once
+// and have little to compute: what counts is how many bytes are in flight and
+// how many launches there are.  A workgroup of eight waves takes 4 RB share
+// rows x 32 columns over the whole K: wave v takes the 128-wide K chunks v, v +
+// 8, ..., so that the workgroup reads K/128 chunks at once, and the waves' sums
+// meet in LDS at the end: one launch, no clear, no atomics, no mask pass, and
+// eight times the waves of a 128-column tile grid.  Any K and weight form.
+//
+// Weights go from memory straight into the MFMA's B registers: lane l holds 64
+// bytes of column l % 32, the chunk's half l / 32, and MFMA j of a chunk takes
+// bytes 16 j .. 16 j + 15 of both halves (any assignment of k to MFMAs is
+// exact, as long as A follows the same).  Shares go through a wave-private LDS
+// buffer of 4 rows x 128 words and are read as digits by the transpose read, as
+// in the DMA kernel.  LDS operations of one wave complete in order, so the
+// buffer needs no barrier.  Pre-split and int32 weights keep one accumulator
+// set per plane, so the shares are staged once for all three.
+constexpr int kFewWaves = 8, kFewChunk = 128, kFewCols = 32;
+constexpr int kFewRow = kFewChunk * 8;  // bytes of one staged share row
+
+template <int WT>
+constexpr int few_planes() { return WT == kW8 ? 1 : 3; }
+
+template <int RB, int WT>
+__global__ void __launch_bounds__(64 * kFewWaves) __attribute__((amdgpu_waves_per_eu(2)))
+    share_gemm_few_kernel(GemmGroup g) {
+  constexpr int P = few_planes<WT>();
+  constexpr int kStage = kFewWaves * 4 * kFewRow, kSums = kFewWaves * RB * 4 * 64 * 8;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kStage > kSums ? kStage : kSums];
+  const GemmGroup::Item& it = group_item(g, blockIdx.x);
+  const int M = it.M, K = it.K, N = it.N;
+  const int tile = int(blockIdx.x - it.first), m0 = (tile / it.tiles_n) * 4 * RB, n0 = (tile % it.tiles_n) * kFewCols;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5;
+  const size_t col = size_t(min(n0 + (lane & 31), N - 1)) * K;  // columns past N: any valid one, results dropped
+  const int8_t* w8 = it.w + col;
+  const int32_t* w32 = reinterpret_cast<const int32_t*>(it.w) + col;
+  const size_t plane_step = size_t(N) * K;
+  uint8_t* buf = lds + wave * 4 * kFewRow;
+  // transpose-read source: row tr_row, words 64 half + 16 j + tr_k (+ 8)
+  const int tr_row = 2 * ((lane >> 4) & 1) + (lane & 1), tr_k = (lane >> 1) & 7;
+  v16i acc[P][RB];
+  int colsum[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    colsum[p] = 0;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[p][rb] = v16i{0};
+  }
+  for (int k0 = wave * kFewChunk; k0 < K; k0 += kFewWaves * kFewChunk) {
+    const int kw = k0 + 64 * half;
+    v4i b[P][4];
+    if constexpr (WT == kW32) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint4 v = load_w4(w32, kw + 16 * j + 4 * q, K);
+#pragma unroll
+          for (int p = 0; p < P; ++p) b[p][j][q] = int(digit4(v, 0x0c0c0400u + 0x0101u * unsigned(p)));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint4 v = load_w16(w8 + p * plane_step, kw + 16 * j, K);
+          b[p][j] = v4i{int(v.x), int(v.y), int(v.z), int(v.w)};
+        }
+    }
+    uint4 xv[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        xv[rb][r] = load_x2(it.x + size_t(min(m0 + 4 * rb + r, M - 1)) * K, k0 + 2 * lane, K);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) *reinterpret_cast<uint4*>(buf + r * kFewRow + ((lane ^ (4 * r)) << 4)) = xv[rb][r];
+      __builtin_amdgcn_wave_barrier();
+      v4i a[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = 64 * half + 16 * j + tr_k;
+        const v2i lo = tr8(buf, tr_row * kFewRow + (((k >> 1) ^ (4 * tr_row)) << 4) + ((k & 1) << 3));
+        const v2i hi = tr8(buf, tr_row * kFewRow + ((((k + 8) >> 1) ^ (4 * tr_row)) << 4) + ((k & 1) << 3));
+        a[j] = v4i{lo.x, lo.y, hi.x, hi.y} ^ int(0x80808080u);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          acc[p][rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j], b[p][j], acc[p][rb], 0, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) colsum[p] = __builtin_amdgcn_sdot4(b[p][j][e], 0x01010101, colsum[p], false);
+  }
+  // this lane's part of rows 4 rb + gq: digits 4 half .. 4 half + 3 and its
+  // half of the column's offset correction
+  __syncthreads();
+  uint64_t* sums = reinterpret_cast<uint64_t*>(lds);  // [wave][row][lane]
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      uint64_t v = 0;
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const v16i& a = acc[p][rb];
+        const int64_t d = mad_i64(a[4 * gq + 3], 16777216,
+                                  mad_i64(a[4 * gq + 2], 65536, mad_i64(a[4 * gq + 1], 256, int64_t(a[4 * gq]))));
+        v += ((uint64_t(d) << (32 * half)) + 0x8080808080808080ull * uint64_t(int64_t(colsum[p]))) << (8 * p);
+      }
+      sums[(wave * 4 * RB + 4 * rb + gq) * 64 + lane] = v;
+    }
+  __syncthreads();
+  const int row = t >> 5, cl = t & 31;
+  if (row < 4 * RB && m0 + row < M && n0 + cl < N) {
+    uint64_t v = 0;
+#pragma unroll
+    for (int w = 0; w < kFewWaves; ++w) {
+      const uint64_t* s = sums + (w * 4 * RB + row) * 64 + cl;
+      v += s[0] + s[32];
+    }
+    const int sh = it.shifts ? int(it.shifts[n0 + cl]) : 0;
+    v = sh < 64 ? (v << sh) : 0;
+    it.y[size_t(m0 + row) * N + n0 + cl] = v & group_mask(it.mask_bits);
   }
 }
 
@@ -769,97 +999,207 @@ hipError_t launch_weight_split(const int32_t* w, int8_t* planes, size_t count, h
 
 // Zero several outputs in one launch (a batch's split-K products): blockIdx.y
 // names the buffer.
+constexpr int kGemmClearMax = 64;
+struct GemmClearList {
+  uint64_t* ptr[kGemmClearMax];
+  size_t words[kGemmClearMax];
+  int count;
+};
 __global__ void __launch_bounds__(256) gemm_clear_list_kernel(GemmClearList l) {
   uint64_t* y = l.ptr[blockIdx.y];
   const size_t n = l.words[blockIdx.y];
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) y[i] = 0;
 }
 
-hipError_t launch_gemm_clear_list(const GemmClearList& l, hipStream_t s) {
-  if (l.count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(gemm_clear_list_kernel, dim3(512, unsigned(l.count)), dim3(256), 0, s, l);
+// The few-row kernel's workgroups each read 4 rb share rows and 32 weight
+// columns whole, so what it moves through L2 grows with M N K, while a tile
+// kernel pays a clear, a mask pass and a ring fill.  Measured (us, few-row /
+// tile kernel, int8): 1x1024x4096 11.9 / 17.5 and 64x1024x4096 12.0 / 17.7
+// (both at the host's issue rate), 100x1024x3001 15.5 / 17.7 (108 MB),
+// 32x4096x8192 26.4 / 22.4 (335 MB), 100x3072x4096 35.1 / 25.9 (440 MB); three
+// planes: 64x3072x1024 15.3 / 18.2 (126 MB), 77x3072x1024 28.2 / 21.2 (157 MB);
+// int32: 13x1024x3001 12.7 / 18.7 (37 MB), 13x3072x4096 32.9 / 29.5 (151 MB).
+constexpr size_t kFewBytes = size_t(128) << 20;
+static int few_rb(int w_bits, int M) { return M <= 4 ? 1 : (M <= 8 || w_bits != 8) ? 2 : 4; }
+static size_t few_bytes(int w_bits, int M, int K, int N) {
+  const size_t rb = size_t(few_rb(w_bits, M)), wgs = (size_t(M) + 4 * rb - 1) / (4 * rb) * ((size_t(N) + 31) / 32);
+  return wgs * size_t(K) * 32 * (rb + (w_bits == 8 ? 1 : w_bits == 24 ? 3 : 4));
+}
+
+// Which kernel a product takes, and how its K is split.
+enum GemmKernel { kGemmFew, kGemmDma2, kGemmDma3, kGemmReg };
+struct GemmChoice {
+  GemmKernel kernel;
+  int rb;               // kGemmFew: 4-row blocks per workgroup
+  int k_split, splits;  // K words per workgroup, K splits (tile kernels)
+  int planes;
+  bool adds;  // the workgroups of one tile add into y (atomics): y is zeroed first, masked after
+};
+
+static GemmChoice gemm_choice(const void* x, const void* w, int w_bits, int M, int K, int N,
+                              size_t few_limit = kFewBytes) {
+  GemmChoice c{};
+  c.planes = w_bits == 8 ? 1 : 3;
+  c.rb = few_rb(w_bits, M);
+  if (few_bytes(w_bits, M, K, N) <= few_limit) {
+    c.kernel = kGemmFew;
+    return c;
+  }
+  // LDS DMA: whole 64-wide K steps, 16-byte aligned rows
+  const bool dma = w_bits != 32 && K % kBK == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  // 128-column tiles (CB = 2, up to two workgroups per CU), K split while
+  // the tiles fill fewer than 256 workgroups and each split keeps >= 8
+  // steps.  192-column tiles (CB = 3, one workgroup per CU) only where
+  // they fill the 256 CUs in one round while the 128-column grid would
+  // leave the CUs unevenly loaded (between one and two workgroups each):
+  // 512 x 1024 x 3072 int8 runs 21.4 us against 22.8 us; every other
+  // Qwen3 shape and the f12 planes run faster with CB = 2 (measured).
+  const int ksteps = (K + kBK - 1) / kBK;
+  const long tiles2 = long((N + 127) / 128) * long((M + kBM - 1) / kBM);
+  const long tiles3 = long((N + 191) / 192) * long((M + kBM - 1) / kBM);
+  int splits = 1;
+  while (splits < 4 && tiles2 * splits < 256 && ksteps / (splits * 2) >= 8) splits *= 2;
+  const long wg2 = tiles2 * splits * c.planes;
+  c.kernel = !dma ? kGemmReg : (splits == 1 && c.planes == 1 && wg2 > 256 && wg2 < 512 && tiles3 <= 256) ? kGemmDma3 : kGemmDma2;
+  c.k_split = (ksteps + splits - 1) / splits * kBK;
+  c.splits = (K + c.k_split - 1) / c.k_split;
+  c.adds = c.splits * c.planes > 1;
+  return c;
+}
+
+static GemmGroup::Item group_entry(const uint64_t* x, const void* w, const int8_t* shifts, uint64_t* y, int M, int K,
+                                   int N, int mask_bits, int tile_m, int tile_n, unsigned first) {
+  return GemmGroup::Item{x, static_cast<const int8_t*>(w), shifts, y, M, K, N, mask_bits,
+                         (N + tile_n - 1) / tile_n, (M + tile_m - 1) / tile_m, first, 0};
+}
+
+static hipError_t launch_few(const GemmGroup& g, int rb, int w_bits, unsigned tiles, hipStream_t s) {
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(tiles), dim3(64 * kFewWaves), 0, s, g); };
+  if (w_bits == 8)
+    rb == 1 ? go(share_gemm_few_kernel<1, kW8>) : rb == 2 ? go(share_gemm_few_kernel<2, kW8>) : go(share_gemm_few_kernel<4, kW8>);
+  else if (w_bits == 24)
+    rb == 1 ? go(share_gemm_few_kernel<1, kWPlanes>) : go(share_gemm_few_kernel<2, kWPlanes>);
+  else
+    rb == 1 ? go(share_gemm_few_kernel<1, kW32>) : go(share_gemm_few_kernel<2, kW32>);
   return hipGetLastError();
 }
 
-// Split-K products add their partial products into y with atomics, so y must
-// be zero first; true when this product takes that path.
-bool share_gemm_adds_into_y(const void* x, const void* w, int w_bits, int M, int K, int N) {
-  if (w_bits != 8 && w_bits != 24) return false;
-  const int w_vec = (K % 16 == 0) && (reinterpret_cast<uintptr_t>(w) % 16 == 0);
-  if (!(K % kBK == 0 && w_vec && reinterpret_cast<uintptr_t>(x) % 16 == 0)) return false;
-  const int planes = w_bits == 8 ? 1 : 3, ksteps = K / kBK;
-  const long tiles2 = long((N + 127) / 128) * long((M + kBM - 1) / kBM);
-  int splits = 1;
-  while (splits < 4 && tiles2 * splits < 256 && ksteps / (splits * 2) >= 8) splits *= 2;
-  const int k_split = (ksteps + splits - 1) / splits * kBK;
-  return ((K + k_split - 1) / k_split) * planes > 1;
+static hipError_t run_share_gemm(const uint64_t* x, const void* w, int w_bits, const int8_t* shifts, uint64_t* y,
+                                 int M, int K, int N, int mask_bits, hipStream_t s, bool y_zero) {
+  const uint64_t mask = mask_bits >= 64 ? ~0ull : ((1ull << mask_bits) - 1);
+  const GemmChoice c = gemm_choice(x, w, w_bits, M, K, N);
+  if (c.kernel == kGemmFew) {
+    GemmGroup g;
+    g.count = 1;
+    g.item[0] = group_entry(x, w, shifts, y, M, K, N, mask_bits, 4 * c.rb, kFewCols, 0);
+    return launch_few(g, c.rb, w_bits, unsigned(g.item[0].tiles_m) * unsigned(g.item[0].tiles_n), s);
+  }
+  const size_t words = size_t(M) * N;
+  const unsigned fgrid = unsigned(std::min<size_t>((words + 255) / 256, 4096));
+  // several planes or K splits add their partial products into y
+  if (c.adds && !y_zero) {
+    hipLaunchKernelGGL(gemm_clear_kernel, dim3(fgrid), dim3(256), 0, s, y, words, 0ull);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  const dim3 block(kThreads);
+  const unsigned gy = unsigned((M + kBM - 1) / kBM), gz = unsigned(c.splits * c.planes);
+  const dim3 grid2(unsigned((N + kBN - 1) / kBN), gy, gz);
+  const auto reg = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid2, block, 0, s, x, w, shifts, y, M, K, N, mask, c.k_split, c.splits);
+  };
+  if (c.kernel == kGemmReg)
+    w_bits == 32 ? reg(share_gemm_reg_kernel<kW32>) : reg(share_gemm_reg_kernel<kW8>);
+  else if (c.kernel == kGemmDma2)
+    hipLaunchKernelGGL(share_gemm_dma_kernel<2>, grid2, block, 0, s, x, static_cast<const int8_t*>(w), shifts, y, M, K,
+                       N, mask, c.k_split, c.splits);
+  else
+    hipLaunchKernelGGL(share_gemm_dma_kernel<3>, dim3(unsigned((N + 191) / 192), gy, gz), block, 0, s, x,
+                       static_cast<const int8_t*>(w), shifts, y, M, K, N, mask, c.k_split, c.splits);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && c.adds && mask != ~0ull) {
+    hipLaunchKernelGGL(gemm_clear_kernel, dim3(fgrid), dim3(256), 0, s, y, words, mask);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t launch_share_gemm(const uint64_t* x, const void* w, int w_bits, const int8_t* shifts, uint64_t* y,
-                             int M, int K, int N, int mask_bits, hipStream_t s, bool y_zero) {
-  const uint64_t mask = mask_bits >= 64 ? ~0ull : ((1ull << mask_bits) - 1);
-  const dim3 grid((N + kBN - 1) / kBN, (M + kBM - 1) / kBM), block(kThreads);
-  // 16-byte weight loads need 16-byte aligned rows
-  const int w_vec = (K % 16 == 0) && (reinterpret_cast<uintptr_t>(w) % 16 == 0);
-  if (w_bits == 8 || w_bits == 24) {
-    const int planes = w_bits == 8 ? 1 : 3;
-    if (K % kBK == 0 && w_vec && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
-      // 128-column tiles (CB = 2, up to two workgroups per CU), K split while
-      // the tiles fill fewer than 256 workgroups and each split keeps >= 8
-      // steps.  192-column tiles (CB = 3, one workgroup per CU) only where
-      // they fill the 256 CUs in one round while the 128-column grid would
-      // leave the CUs unevenly loaded (between one and two workgroups each):
-      // 512 x 1024 x 3072 int8 runs 21.4 us against 22.8 us; every other
-      // Qwen3 shape and the f12 planes run faster with CB = 2 (measured).
-      const int ksteps = K / kBK;
-      const long tiles2 = long((N + 127) / 128) * long((M + kBM - 1) / kBM);
-      const long tiles3 = long((N + 191) / 192) * long((M + kBM - 1) / kBM);
-      int best_splits = 1;
-      while (best_splits < 4 && tiles2 * best_splits < 256 && ksteps / (best_splits * 2) >= 8) best_splits *= 2;
-      const long wg2 = tiles2 * best_splits * planes;
-      const int best_cb = (best_splits == 1 && planes == 1 && wg2 > 256 && wg2 < 512 && tiles3 <= 256) ? 3 : 2;
-      const int k_split = (ksteps + best_splits - 1) / best_splits * kBK;
-      const int splits = (K + k_split - 1) / k_split;
-      const size_t words = size_t(M) * N;
-      const unsigned fgrid = unsigned(std::min<size_t>((words + 255) / 256, 4096));
-      // several planes or K splits add their partial products into y
-      const bool atomic = splits * planes > 1;
-      if (atomic && !y_zero) {
-        hipLaunchKernelGGL(gemm_clear_kernel, dim3(fgrid), dim3(256), 0, s, y, words, 0ull);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-      }
-      const unsigned gy = unsigned((M + kBM - 1) / kBM), gz = unsigned(splits * planes);
-      if (best_cb == 2)
-        hipLaunchKernelGGL(share_gemm_dma_kernel<2>, dim3(unsigned((N + 127) / 128), gy, gz), block, 0, s, x,
-                           static_cast<const int8_t*>(w), shifts, y, M, K, N, mask, k_split, splits);
-      else
-        hipLaunchKernelGGL(share_gemm_dma_kernel<3>, dim3(unsigned((N + 191) / 192), gy, gz), block, 0, s, x,
-                           static_cast<const int8_t*>(w), shifts, y, M, K, N, mask, k_split, splits);
-      hipError_t e = hipGetLastError();
-      if (e == hipSuccess && atomic && mask != ~0ull) {
-        hipLaunchKernelGGL(gemm_clear_kernel, dim3(fgrid), dim3(256), 0, s, y, words, mask);
-        e = hipGetLastError();
-      }
-      return e;
+                             int M, int K, int N, int mask_bits, hipStream_t s) {
+  return run_share_gemm(x, w, w_bits, shifts, y, M, K, N, mask_bits, s, false);
+}
+
+// Products whose order does not matter: the int8 ones in launches of up to
+// kGroupMax, those of few rows by their row blocks and the DMA path's as
+// 128-column tiles, longest K first (the last round of tiles is then one of
+// short ones); the rest one by one, the outputs they add into zeroed together.
+// A grid of many products fills the chip with either kernel, and then the bytes
+// per product decide: for every 32 columns and k a tile moves 96, the few-row
+// kernel 64 (up to 4 rows), 96 or 160.  56 products of 16 rows: tiles 85 us,
+// few-row 142 us; of one row: 77 and 60 us.
+hipError_t launch_share_gemm_group(const praghip_gemm_desc* list, size_t count, hipStream_t s) {
+  std::vector<const praghip_gemm_desc*> few[3], dma, rest, adds;
+  hipError_t e = hipSuccess;
+  size_t moved = 0;
+  for (size_t i = 0; i < count; ++i)
+    if (list[i].m && list[i].n && list[i].w_bits == 8)
+      moved += few_bytes(8, int(list[i].m), int(list[i].k), int(list[i].n));
+  for (size_t i = 0; i < count; ++i) {
+    const praghip_gemm_desc& d = list[i];
+    if (d.m == 0 || d.n == 0) continue;
+    GemmChoice c = gemm_choice(d.x, d.w, d.w_bits, int(d.m), int(d.k), int(d.n));
+    if (d.w_bits == 8 && c.kernel == kGemmFew && d.m > 4 && moved > kFewBytes) {
+      const GemmChoice t = gemm_choice(d.x, d.w, 8, int(d.m), int(d.k), int(d.n), 0);
+      if (t.kernel == kGemmDma2 || t.kernel == kGemmDma3) c = t;
     }
-    // register-staged kernel, one launch per plane (plane e shifted by 8e,
-    // accumulated into y after the first)
-    for (int e = 0; e < planes; ++e) {
-      const int8_t* we = static_cast<const int8_t*>(w) + size_t(e) * size_t(N) * size_t(K);
-      hipLaunchKernelGGL((share_gemm_kernel<8>), grid, block, 0, s, x, we, shifts, y, M, K, N, mask, e, e > 0,
-                         w_vec);
-      const hipError_t err = hipGetLastError();
-      if (err != hipSuccess) return err;
+    const size_t tiles = ((d.m + 3) / 4) * ((d.n + kFewCols - 1) / kFewCols);
+    if (d.w_bits == 8 && c.kernel == kGemmFew && tiles < (1u << 24))
+      few[c.rb >> 1].push_back(&d);
+    else if (d.w_bits == 8 && (c.kernel == kGemmDma2 || c.kernel == kGemmDma3) && tiles < (1u << 24))
+      dma.push_back(&d);
+    else {
+      rest.push_back(&d);
+      if (c.adds) adds.push_back(&d);
     }
-    return hipSuccess;
   }
-  for (int e = 0; e < 3; ++e) {
-    hipLaunchKernelGGL((share_gemm_kernel<32>), grid, block, 0, s, x, w, shifts, y, M, K, N, mask, e, e > 0, 0);
-    const hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  const bool together = adds.size() > 1;
+  for (size_t a0 = 0; together && a0 < adds.size() && e == hipSuccess; a0 += kGemmClearMax) {
+    GemmClearList l{};
+    for (size_t a = a0; a < adds.size() && l.count < kGemmClearMax; ++a) {
+      l.ptr[l.count] = adds[a]->y;
+      l.words[l.count++] = adds[a]->m * adds[a]->n;
+    }
+    hipLaunchKernelGGL(gemm_clear_list_kernel, dim3(512, unsigned(l.count)), dim3(256), 0, s, l);
+    e = hipGetLastError();
   }
-  return hipSuccess;
+  for (size_t i = 0; i < rest.size() && e == hipSuccess; ++i) {
+    const praghip_gemm_desc& d = *rest[i];
+    e = run_share_gemm(d.x, d.w, d.w_bits, d.shifts, d.y, int(d.m), int(d.k), int(d.n), d.mask_bits, s, together);
+  }
+  std::stable_sort(dma.begin(), dma.end(), [](auto* a, auto* b) { return a->k > b->k; });
+  const auto run = [&](const std::vector<const praghip_gemm_desc*>& v, int tile_m, int tile_n, auto&& launch) {
+    for (size_t i0 = 0; i0 < v.size() && e == hipSuccess; i0 += kGroupMax) {
+      GemmGroup g;
+      g.count = int(std::min<size_t>(kGroupMax, v.size() - i0));
+      unsigned tiles = 0;
+      for (int i = 0; i < g.count; ++i) {
+        const praghip_gemm_desc& d = *v[i0 + size_t(i)];
+        g.item[i] = group_entry(d.x, d.w, d.shifts, d.y, int(d.m), int(d.k), int(d.n), d.mask_bits, tile_m, tile_n, tiles);
+        tiles += unsigned(g.item[i].tiles_m) * unsigned(g.item[i].tiles_n);
+      }
+      e = launch(g, tiles);
+    }
+  };
+  for (int i = 0; i < 3; ++i) {
+    const int rb = 1 << i;
+    run(few[i], 4 * rb, kFewCols, [&](const GemmGroup& g, unsigned tiles) { return launch_few(g, rb, 8, tiles, s); });
+  }
+  run(dma, kBM, kBN, [&](const GemmGroup& g, unsigned tiles) {
+    hipLaunchKernelGGL(share_gemm_group_kernel, dim3(tiles), dim3(kThreads), 0, s, g);
+    return hipGetLastError();
+  });
+  return e;
 }
 
 }  // namespace praghip

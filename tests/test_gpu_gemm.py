@@ -198,3 +198,78 @@ def test_gemm_batch_split_k_outputs_cleared_together(gpu):
     np.testing.assert_array_equal(from_dev(y1), oracle.share_gemm(xb, w1))
     np.testing.assert_array_equal(from_dev(B), oracle.share_gemm(x2, w2))
     np.testing.assert_array_equal(from_dev(y0), oracle.share_gemm(x2, w2))
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 15, 1), (1, 17, 33), (3, 127, 31), (4, 128, 32), (5, 129, 33), (8, 1023, 65),
+                                   (9, 1025, 64), (16, 2049, 95), (17, 63, 130), (33, 1000, 129), (40, 4097, 257),
+                                   (129, 130, 1)])
+@pytest.mark.parametrize("wdt", ["i8", "i32", "i32split"])
+def test_gemm_any_k_and_alignment(gpu, m, k, n, wdt):
+    """Few-row and register-staged kernels around their edges: rows about the
+    4-row blocks and the 32-row tile, K about the 128-wide chunks and 64-wide
+    steps (odd K puts every weight row at another alignment), columns about 32
+    and 128; the operands start 8 bytes (x) and one element (w) off 16 bytes.
+    Whole-number arithmetic: exact."""
+    import torch
+    print(f"[gemm] m={m} k={k} n={n} {wdt}", flush=True)
+    x = oracle.fill_u64(m * k, 11000 + m).reshape(m, k)
+    if wdt == "i8":
+        w = oracle.fill_i8(n * k, 12000 + n).reshape(n, k)
+        w.flat[0] = -128
+    else:
+        w = ((oracle.fill_u64(n * k, 13000 + n) % np.uint64(0x7F7F7F + 0x808080 + 1)).astype(np.int64)
+             - 0x808080).astype(np.int32).reshape(n, k)
+    sh = oracle.fill_shift(n, 14000 + k)
+    tx = torch.zeros(m * k + 1, dtype=torch.int64, device="cuda")[1:].view(m, k)
+    tx.copy_(to_dev(x))
+    tw = torch.from_numpy(w).cuda()
+    if wdt == "i32split":
+        tw = praghip.split_weights(tw)
+    off = torch.zeros(tw.numel() + 1, dtype=tw.dtype, device="cuda")[1:].view(tw.shape)
+    off.copy_(tw)
+    for shifts, mask in ((None, 64), (sh, 59)):
+        ts = None if shifts is None else torch.from_numpy(shifts).cuda()
+        y = praghip.share_gemm(tx, off, shifts=ts, mask_bits=mask)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(from_dev(y), oracle.share_gemm(x, w, shifts, mask))
+
+
+def test_gemm_batch_forms(gpu):
+    """A batch mixing few-row, tiled, ragged-K and pre-split products, once
+    with separate operands (run together) and once with an output that a later
+    product reads (run in list order)."""
+    import ctypes
+
+    import torch
+    from praghip._lib import GemmDesc, check, lib
+    specs = [(3, 256, 70, 8, 64), (40, 128, 300, 8, 59), (300, 192, 520, 8, 64), (20, 100, 33, 8, 64),
+             (5, 1000, 64, 24, 59), (64, 64, 128, 24, 64), (1, 64, 4096, 8, 64), (40, 320, 129, 8, 64)] * 5
+    # one batch: product 1 reads product 0's output
+    chain = [(40, 128, 320, 8, 64), (40, 320, 129, 8, 64)]
+    for chained, rows in ((False, specs), (True, chain)):
+        descs, keep, want = [], [], []
+        prev = None
+        for i, (m, k, n, bits, mask) in enumerate(rows):
+            x = oracle.fill_u64(m * k, 15000 + i).reshape(m, k)
+            tx = to_dev(x)
+            if chained and prev is not None:
+                x, tx = want[-1], prev
+            if bits == 8:
+                w = oracle.fill_i8(n * k, 16000 + i).reshape(n, k)
+                tw = torch.from_numpy(w).cuda()
+            else:
+                w = ((oracle.fill_u64(n * k, 16000 + i) % np.uint64(1 << 21)).astype(np.int64) - (1 << 20)).astype(np.int32).reshape(n, k)
+                tw = praghip.split_weights(torch.from_numpy(w).cuda())
+            sh = oracle.fill_shift(n, 17000 + i)
+            ts = torch.from_numpy(sh).cuda()
+            y = torch.full((m, n), -1, dtype=torch.int64, device="cuda")
+            prev = y
+            want.append(oracle.share_gemm(x, w, sh, mask))
+            keep.append((tx, tw, ts, y))
+            descs.append(GemmDesc(tx.data_ptr(), tw.data_ptr(), ts.data_ptr(), y.data_ptr(), m, k, n, bits, mask))
+        arr = (GemmDesc * len(descs))(*descs)
+        check(lib().praghip_share_gemm_batch(0, ctypes.cast(arr, ctypes.c_void_p), len(descs),
+                                             torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        for i, (_, _, _, y) in enumerate(keep):
+            np.testing.assert_array_equal(from_dev(y), want[i], err_msg=f"product {i} {rows[i]}")
