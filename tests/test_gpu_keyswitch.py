@@ -273,3 +273,31 @@ def test_keyswitch_wide_special_prime_three_phase(gpu, bits, dnum):
     tin, tout, tk = to_dev(ct), to_dev(np.zeros_like(ct)), to_dev(keys)
     sw.keyswitch(tin, tout, keys=tk, key_stride=sw.key_words, galois=3)
     np.testing.assert_array_equal(from_dev(tout), want)
+
+
+@pytest.mark.parametrize("log_n,kind,L,dnum,batch", [
+    (12, "50", 6, 6, 1), (12, "locked", 6, 4, 3), (12, "locked", 5, 2, 40), (12, "50", 2, 2, 70), (12, "50", 5, 3, 130),
+    (13, "locked", 6, 6, 1), (13, "50", 6, 4, 2), (13, "50", 5, 2, 17), (13, "locked", 3, 2, 66),
+    (14, "50", 6, 5, 1), (14, "locked", 6, 4, 1), (14, "locked", 5, 2, 4), (14, "50", 5, 2, 3), (14, "50", 3, 2, 33),
+    (14, "locked", 4, 3, 22), (14, "50", 5, 4, 17), (14, "locked", 6, 5, 14)])
+def test_keyswitch_rows_shapes(gpu, log_n, kind, L, dnum, batch):
+    """The three-phase kernels over their sizes, unequal digits and batches on
+    both sides of every launch rule (targets spread over threads, digits over
+    wave pairs, the special prime's columns formed by each data prime), with the
+    largest words in the first ciphertext and key; exact."""
+    n = 1 << log_n
+    q = (cf.primes_below(50, n, L) + cf.primes_below(60, n, 1)) if kind == "50" else \
+        list(cf.LOCKED_PRIMES[:L]) + [cf.LOCKED_PRIMES[6]]
+    print(f"[ks] N={n} {kind} L={L} dnum={dnum} batch={batch}", flush=True)
+    ct = oracle.fill_residues(batch * 2 * L, n, q[:L], 0x77 + batch).reshape(batch, 2, L, n)
+    ct[0, 1] = np.array(q[:L], dtype=np.uint64)[:, None] - np.uint64(1)
+    keys = oracle.fill_residues(2 * dnum * 2 * (L + 1), n, q, 0x78 + L).reshape(2, dnum, 2, L + 1, n)
+    keys[0] = (np.array(q, dtype=np.uint64) - np.uint64(1))[None, None, :, None]
+    sw = praghip.Switch(q, log_n, dnum, max_batch=batch)
+    tin, tout, tk = to_dev(ct), to_dev(np.zeros_like(ct)), to_dev(keys)
+    for k, g in ((0, 3), (1, 2 * n - 1), (1, 1)):
+        sw.keyswitch(tin, tout, keys=tk[k].contiguous(), key_stride=0, galois=g)
+        got = from_dev(tout)
+        for b in sorted({0, batch // 2, batch - 1}):
+            want = oracle.keyswitch(ct[b:b + 1], keys[k], q, dnum, log_n, g)[0]
+            np.testing.assert_array_equal(got[b], want, err_msg=f"key {k} galois {g} ciphertext {b}")
