@@ -100,11 +100,11 @@ uint64_t minimal_root(uint64_t q, uint64_t two_n) {
     if (powmod(c, two_n / 2, q) == q - 1) g = c;
   }
   if (!g) return 0;
-  const uint64_t g2 = mulmod(g, g, q);
+  const uint64_t g2 = mulmod(g, g, q), g2_q = shoup_q(g2, q);
   uint64_t cur = g, best = g;
   for (uint64_t i = 0; i < two_n; i += 2) {
     best = cur < best ? cur : best;
-    cur = mulmod(cur, g2, q);
+    cur = mul_shoup(cur, g2, g2_q, q);
   }
   return best;
 }
@@ -119,15 +119,19 @@ bool make_tables(uint64_t q, unsigned log_n, uint64_t* fwd, uint64_t* inv, uint6
   fwd[1] = shoup_q(1, q);
   inv[0] = 1;
   inv[1] = shoup_q(1, q);
+  // powers by Shoup products and quotients from the Barrett ratio: no 128-bit
+  // division per entry
+  const uint64_t psi_q = shoup_q(psi, q), psi_inv_q = shoup_q(psi_inv, q);
+  const Barrett m = barrett_of(q);
   uint64_t p = psi, pi = psi_inv;
   for (uint64_t i = 1; i < n; ++i) {
     const uint64_t f = bitrev(i, log_n), r = bitrev(i - 1, log_n) + 1;
     fwd[2 * f] = p;
-    fwd[2 * f + 1] = shoup_q(p, q);
+    fwd[2 * f + 1] = shoup_quotient(p, m);
     inv[2 * r] = pi;
-    inv[2 * r + 1] = shoup_q(pi, q);
-    p = mulmod(p, psi, q);
-    pi = mulmod(pi, psi_inv, q);
+    inv[2 * r + 1] = shoup_quotient(pi, m);
+    p = mul_shoup(p, psi, psi_q, q);
+    pi = mul_shoup(pi, psi_inv, psi_inv_q, q);
   }
   const uint64_t ni = invmod(n % q, q);
   invn[0] = ni;
@@ -190,6 +194,26 @@ void release_all(int device, Buffers& buf, hipStream_t& stream, hipEvent_t* even
 }
 
 
+// One integer form serves a plan.  ArPM needs pm_bits of every prime that some
+// kernel takes on the integer path: the primes of 50 bits and more, the last
+// one (a keyswitch's special prime) in any case, and - a keyswitch with one
+// data prime on the integer path has them all there - no float prime among
+// integer ones before it.
+bool pm_plan(const uint64_t* q, size_t P) {
+  size_t wide = 0;
+  for (size_t p = 0; p + 1 < P; ++p) {
+    if (q[p] >> 50) {
+      if (!pm_bits(q[p])) return false;
+      ++wide;
+    }
+  }
+  return (wide == 0 || wide + 1 == P) && q[P - 1] >> 50 && pm_bits(q[P - 1]);
+}
+// (w, its Shoup quotient) as ArPM's pair
+ulonglong2 pm_pair(uint64_t w, uint64_t wq, uint64_t q) {
+  return make_ulonglong2(pm_split(w), pm_split(mul_shoup(1ull << 32, w, wq, q)));
+}
+
 // Builds the per-prime constants and device-format tables of a prime set.
 int build_ntt_host(const uint64_t* q, size_t P, unsigned log_n, const uint64_t* fwd_in, const uint64_t* inv_in,
                    const uint64_t* invn_in, NttHost& h) {
@@ -200,6 +224,7 @@ int build_ntt_host(const uint64_t* q, size_t P, unsigned log_n, const uint64_t* 
   h.fwd_f.resize(P * n);
   h.inv_f.resize(P * n);
   std::vector<uint64_t> fwd(2 * n), inv(2 * n), invn(2);
+  h.pm = P && pm_plan(q, P);
   for (size_t p = 0; p < P; ++p) {
     const uint64_t qq = q[p];
     if (qq < 3 || qq >= (1ull << 62) || !is_prime(qq) || (qq - 1) % (2 * n))
@@ -228,9 +253,16 @@ int build_ntt_host(const uint64_t* q, size_t P, unsigned log_n, const uint64_t* 
     pr.qinv = 1.0 / double(qq);
     pr.ninv_f = double(invn[0]);
     pr.last_f = double(last);
+    pr.pm_bits = h.pm ? pm_bits(qq) : 0;
+    const auto pair = [&](uint64_t w, uint64_t wq) {
+      return pr.pm_bits ? pm_pair(w, wq, qq) : make_ulonglong2(w, wq);
+    };
+    const ulonglong2 ni = pair(pr.ninv, pr.ninv_q), la = pair(pr.last, pr.last_q);
+    pr.ninv = ni.x, pr.ninv_q = ni.y;
+    pr.last = la.x, pr.last_q = la.y;
     for (size_t i = 0; i < n; ++i) {
-      h.fwd_u[p * n + i] = make_ulonglong2(fwd[2 * i], fwd[2 * i + 1]);
-      h.inv_u[p * n + i] = make_ulonglong2(inv[2 * i], inv[2 * i + 1]);
+      h.fwd_u[p * n + i] = pair(fwd[2 * i], fwd[2 * i + 1]);
+      h.inv_u[p * n + i] = pair(inv[2 * i], inv[2 * i + 1]);
       h.fwd_f[p * n + i] = double(fwd[2 * i]);
       h.inv_f[p * n + i] = double(inv[2 * i]);
     }
@@ -242,6 +274,7 @@ hipError_t upload_ntt(const NttHost& h, unsigned log_n, Buffers& buf, NttDevice&
   const size_t P = h.primes.size(), n = size_t(1) << log_n;
   d.log_n = int(log_n);
   d.P = int(P);
+  d.pm_u64 = h.pm ? 1 : 0;
   hipError_t e;
   if ((e = buf.alloc((void**)&d.primes, P * sizeof(NttPrime), false)) != hipSuccess) return e;
   if ((e = buf.alloc((void**)&d.tw_fwd_u, P * n * 16, false)) != hipSuccess) return e;
@@ -668,6 +701,14 @@ int build_ks_const(const uint64_t* q, size_t L, size_t dnum, unsigned log_n, KsC
     const uint64_t nr = mulmod(invn[0], r, q[t]), lr = mulmod(inv[2 * (n - 1)], nr, q[t]);
     kc.ninv_r[t] = Shoup{nr, shoup_q(nr, q[t])};
     kc.last_r[t] = Shoup{lr, shoup_q(lr, q[t])};
+  }
+  kc.pm = kc.lazy && pm_plan(q, K) ? 1 : 0;
+  for (size_t t = 0; kc.pm && t < K; ++t) {
+    if (!pm_bits(q[t])) continue;  // a float-path prime
+    for (Shoup* c : {&kc.ninv_r[t], &kc.last_r[t]}) {
+      const ulonglong2 w = pm_pair(c->w, c->wq, q[t]);
+      *c = Shoup{w.x, w.y};
+    }
   }
   return PRAGHIP_OK;
 }

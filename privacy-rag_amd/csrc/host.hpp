@@ -93,6 +93,7 @@ struct NttHost {
   std::vector<NttPrime> primes;
   std::vector<ulonglong2> fwd_u, inv_u;
   std::vector<double> fwd_f, inv_f;
+  bool pm = false;  // integer tables in ArPM's form
 };
 
 int build_ntt_host(const uint64_t* q, size_t P, unsigned log_n, const uint64_t* fwd_in, const uint64_t* inv_in,

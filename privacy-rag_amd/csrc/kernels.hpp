@@ -14,7 +14,7 @@ namespace praghip {
 struct NttDevice {
   int log_n = 0, P = 0;
   NttPrime* primes = nullptr;        // [P]
-  ulonglong2* tw_fwd_u = nullptr;    // [P][N] (w, floor(w 2^64/q))
+  ulonglong2* tw_fwd_u = nullptr;    // [P][N] (w, floor(w 2^64/q)), or ArPM's pairs
   ulonglong2* tw_inv_u = nullptr;    // [P][N]
   double* tw_fwd_f = nullptr;        // [P][N] w as a double, for q < 2^50
   double* tw_inv_f = nullptr;        // [P][N]
@@ -23,6 +23,7 @@ struct NttDevice {
   int* sel_u64 = nullptr;            // device [n_u64]
   int n_f64 = 0, n_u64 = 0;
   int host_sel_f64[64] = {}, host_sel_u64[64] = {};
+  int pm_u64 = 0;    // every integer-path prime just below a power of two: ArPM, and tables in its form
   int lazy_u64 = 1;  // every integer-path prime below 2^60: the lazy integer transforms (ArU64L)
 };
 
@@ -50,6 +51,7 @@ struct KsConst {
   uint64_t neg_qinv[kMaxKeyPrimes];      // -q_t^-1 mod 2^64
   Shoup ninv_r[kMaxKeyPrimes];           // N^-1 2^64 mod q_t
   Shoup last_r[kMaxKeyPrimes];           // w_last N^-1 2^64 mod q_t (w_last = inv[N-1])
+  int pm;                                // ArPM on the integer path (ninv_r, last_r in its form)
 };
 
 struct KsArgs {

@@ -268,12 +268,12 @@ __device__ __forceinline__ void ks_item_f64(const KsFused& f, const KsConst& kc,
   }
 }
 
-// Integer path item (special prime, primes of 50 bits or more): both running
-// sums go through the workgroup's slot.
-template <int LOGN>
+// Integer path item (special prime, primes of 50 bits or more; A = ArPM when
+// the plan's tables have its form): both running sums go through the
+// workgroup's slot.
+template <int LOGN, class A>
 __device__ __forceinline__ void ks_item_u64(const KsFused& f, const KsConst& kc, unsigned b, int t, uint64_t* lds,
                                             uint64_t* slot) {
-  using A = ArU64;
   constexpr unsigned TH = ntt_threads<LOGN>();
   const NttPrime pr = f.primes[t];
   const A ar(pr);
@@ -341,7 +341,7 @@ __device__ __forceinline__ void ks_item_u64(const KsFused& f, const KsConst& kc,
 // The last workgroup to leave zeroes the counters for the next launch.  Every
 // workgroup exits once its ticket passes the item count, so the loop always
 // ends.
-template <int LOGN>
+template <int LOGN, class AU>
 __global__ void __launch_bounds__(ntt_threads<LOGN>()) ks_fused_kernel(KsFused f) {
   __shared__ __attribute__((aligned(16))) uint64_t lds[(1 << LOGN) + (1 << LOGN) / 16];
   __shared__ unsigned ticket;
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>()) ks_fused_kernel(KsFused f
     if (f.data_f64 && t < L)
       ks_item_f64<LOGN>(f, kc, b, int(t), lds, slot);
     else
-      ks_item_u64<LOGN>(f, kc, b, int(t), lds, slot);
+      ks_item_u64<LOGN, AU>(f, kc, b, int(t), lds, slot);
   }
   if (threadIdx.x == 0) {
     __threadfence();
@@ -385,7 +385,7 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>()) ks_fused_kernel(KsFused f
 
 static unsigned grid_for(size_t work) { return unsigned(std::min<size_t>((work + 255) / 256, 1u << 20)); }
 
-template <int LOGN>
+template <int LOGN, class AU>
 static unsigned fused_grid() {
   static unsigned grid = 0;
   if (!grid) {
@@ -393,7 +393,7 @@ static unsigned fused_grid() {
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ks_fused_kernel<LOGN>, ntt_threads<LOGN>(), 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (ks_fused_kernel<LOGN, AU>), ntt_threads<LOGN>(), 0) !=
             hipSuccess ||
         per_cu < 1)
       per_cu = 1;
@@ -402,32 +402,32 @@ static unsigned fused_grid() {
   return grid;
 }
 
-#define PH_LOGN_SWITCH(EXPR)      \
+#define PH_LOGN_SWITCH(...)       \
   switch (log_n) {                \
-    case 4: { constexpr int LG = 4; EXPR; } \
-    case 5: { constexpr int LG = 5; EXPR; } \
-    case 6: { constexpr int LG = 6; EXPR; } \
-    case 7: { constexpr int LG = 7; EXPR; } \
-    case 8: { constexpr int LG = 8; EXPR; } \
-    case 9: { constexpr int LG = 9; EXPR; } \
-    case 10: { constexpr int LG = 10; EXPR; } \
-    case 11: { constexpr int LG = 11; EXPR; } \
-    case 12: { constexpr int LG = 12; EXPR; } \
-    case 13: { constexpr int LG = 13; EXPR; } \
-    case 14: { constexpr int LG = 14; EXPR; } \
+    case 4: { constexpr int LG = 4; __VA_ARGS__; } \
+    case 5: { constexpr int LG = 5; __VA_ARGS__; } \
+    case 6: { constexpr int LG = 6; __VA_ARGS__; } \
+    case 7: { constexpr int LG = 7; __VA_ARGS__; } \
+    case 8: { constexpr int LG = 8; __VA_ARGS__; } \
+    case 9: { constexpr int LG = 9; __VA_ARGS__; } \
+    case 10: { constexpr int LG = 10; __VA_ARGS__; } \
+    case 11: { constexpr int LG = 11; __VA_ARGS__; } \
+    case 12: { constexpr int LG = 12; __VA_ARGS__; } \
+    case 13: { constexpr int LG = 13; __VA_ARGS__; } \
+    case 14: { constexpr int LG = 14; __VA_ARGS__; } \
     default: break;               \
   }
 
 unsigned ks_acc_slots(int log_n) {
-  PH_LOGN_SWITCH(return fused_grid<LG>());
+  PH_LOGN_SWITCH(return (std::max(fused_grid<LG, ArU64>(), fused_grid<LG, ArPM>())));
   return 0;
 }
 
-template <int LOGN>
+template <int LOGN, class AU>
 static hipError_t launch_fused_n(KsFused f, hipStream_t s) {
-  const unsigned blocks = std::min(f.items, std::min(fused_grid<LOGN>(), f.acc_slots));
+  const unsigned blocks = std::min(f.items, std::min(fused_grid<LOGN, AU>(), f.acc_slots));
   f.xcd = (f.batch % kQueueGroups == 0 && blocks % kQueueGroups == 0) ? 1 : 0;
-  hipLaunchKernelGGL((ks_fused_kernel<LOGN>), dim3(blocks), dim3(ntt_threads<LOGN>()), 0, s, f);
+  hipLaunchKernelGGL((ks_fused_kernel<LOGN, AU>), dim3(blocks), dim3(ntt_threads<LOGN>()), 0, s, f);
   return hipGetLastError();
 }
 
@@ -460,7 +460,7 @@ hipError_t launch_keyswitch(const KsArgs& a, const KsConst* kc_dev, const KsCons
   hipError_t e = hipErrorInvalidValue;
   const int log_n = kc.log_n;
   if (a.phase_events) (void)hipEventRecord(a.phase_events[0], s);
-  PH_LOGN_SWITCH(e = launch_fused_n<LG>(f, s); break);
+  PH_LOGN_SWITCH(e = d.pm_u64 ? launch_fused_n<LG, ArPM>(f, s) : launch_fused_n<LG, ArU64>(f, s); break);
   if (e != hipSuccess) return e;
   if (a.phase_events) {
     (void)hipEventRecord(a.phase_events[1], s);

@@ -69,6 +69,9 @@ template <class A>
 struct TypeTag {
   using type = A;
 };
+// Policies whose key products are Montgomery products (every key prime below 2^60)
+template <class A>
+constexpr bool mont_keys = std::is_same<A, ArU64L>::value || std::is_same<A, ArPM>::value;
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint64_t bits_of(double x) { return (uint64_t)__double_as_longlong(x); }
@@ -551,9 +554,9 @@ __device__ __forceinline__ void row_passes_fwd_lds(typename A::T (&v)[E], typena
 
 // Item (ciphertext bl, prime t, row) on the two waves of the workgroup
 // (thread t2 < 128).  Policy A:
-//   ArU64L    - every key prime below 2^60: Montgomery key products x k 2^-64
-//               of the transformed digit word (x < 12q after stage 13) and
-//               the canonical key words (x k < 12 q^2 < q 2^64, each product
+//   ArPM, ArU64L - every key prime below 2^60: Montgomery key products x k 2^-64
+//               of the transformed digit word (any x < 2^64) and
+//               the canonical key words (x k < q 2^64, each product
 //               below 2q), added without reduction from zero and reduced by 8q
 //               after every fourth digit, so the sums stay below 16q; the last
 //               inverse stage multiplies the factor 2^64 back in
@@ -573,7 +576,7 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
   using T = typename A::T;
   constexpr int E = 1 << kRowLE;
   constexpr bool kF64 = std::is_same<T, double>::value;
-  constexpr bool kMont = std::is_same<A, ArU64L>::value;
+  constexpr bool kMont = mont_keys<A>;
   const unsigned dnum = unsigned(kc.dnum), K = unsigned(kc.K);
   const unsigned b = f.b0 + bl;
   const NttPrime pr = f.primes[t];
@@ -651,7 +654,7 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
           a0[rr] += ar.mul(v[rr], ArF64::from_u64(w0));
           a1[rr] += ar.mul(v[rr], ArF64::from_u64(w1));
         } else if constexpr (kMont) {
-          // x < 12q after stage 13, canonical key words: each product < 2q
+          // any x < 2^64, canonical key words: each product < 2q
           a0[rr] += mul_mont(v[rr], w0, ar.q, kc.neg_qinv[t]);
           a1[rr] += mul_mont(v[rr], w1, ar.q, kc.neg_qinv[t]);
         } else {
@@ -737,9 +740,10 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
     __syncthreads();
   }
   uint64_t* pb = f.prod + ((size_t(b) * 2 * K + t) << LOG) + (row << kRowLog);
-  // the integer paths' inverse passes with the compiler's Shoup product
+  // the integer paths' inverse passes on Shoup tables with the compiler's product
   // (ArU64LC, ArU64C)
-  using AI = std::conditional_t<kMont, ArU64LC, std::conditional_t<std::is_same<A, ArU64>::value, ArU64C, A>>;
+  using AI = std::conditional_t<std::is_same<A, ArU64L>::value, ArU64LC,
+                                std::conditional_t<std::is_same<A, ArU64>::value, ArU64C, A>>;
   const AI ari(pr);
   if constexpr (SPLIT) {
     if (g == 1) {
@@ -836,7 +840,7 @@ __device__ __forceinline__ void top_inv(typename A::T (&v)[kColE<LOG>], const ty
 template <class A>
 __device__ __forceinline__ NttPrime product_prime(const KsRows& f, const KsConst& kc, int t) {
   NttPrime r = f.primes[t];
-  if constexpr (std::is_same<A, ArU64L>::value) {
+  if constexpr (mont_keys<A>) {
     r.ninv = kc.ninv_r[t].w;
     r.ninv_q = kc.ninv_r[t].wq;
     r.last = kc.last_r[t].w;
@@ -890,7 +894,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 // fewer for chunks of few ciphertexts, at L times the special prime's columns.
 template <int LOG, class A, class AU, bool SELF>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(SELF ? 2 : std::is_same<typename A::T, double>::value ? 3 : 4)))
+    __attribute__((amdgpu_waves_per_eu(SELF ? 2 : std::is_same<typename A::T, double>::value || std::is_same<A, ArPM>::value ? 3 : 4)))
     ks_cols_inv_kernel(KsRows f) {
   const KsConst& kc = *f.kc;
   const unsigned K = unsigned(kc.K), L = unsigned(kc.L);
@@ -1086,7 +1090,9 @@ hipError_t run_keyswitch_rows(const KsArgs& a, const KsConst* kc_dev, const KsCo
     // products (KsConst::lazy); else Harvey's bounds and Shoup key products
     // phase events only when the whole batch is one chunk
     hipEvent_t* ev = a.batch <= a.inter_cts ? a.phase_events : nullptr;
-    if (kc.lazy)
+    if (kc.pm)
+      launch_chunk<LOG, ArPM>(f, kc, s, ev);
+    else if (kc.lazy)
       launch_chunk<LOG, ArU64L>(f, kc, s, ev);
     else if constexpr (LOG == 14)
       launch_chunk<LOG, ArU64>(f, kc, s, ev);

@@ -145,6 +145,55 @@ PH_HD uint64_t sub_mod(uint64_t a, uint64_t b, uint64_t q) {
   return x >= q ? x - q : x;
 }
 
+// Products modulo a prime just below a power of two.  For q = 2^b - c with
+// 50 <= b <= 60 let M = q 2^(60-b) = 2^60 - c' (c' = c 2^(60-b)); then
+// 2^61 == 2c' (mod q).  A constant w < q is held as w and v = w 2^32 mod q, both
+// split at 29 bits (pm_split: low part in the low word), and for any
+// a = a1 2^32 + a0
+//   X = a0 w + a1 v < 2^93 == a w (mod q),
+//   l = a0 w_lo + a1 v_lo < 2^62,  h = a0 w_hi + a1 v_hi + (l >> 29) = X >> 29 < 2^64,
+//   r = (X mod 2^61) + (X >> 61) 2c',   X >> 61 = h >> 32:
+// five 32 x 32 + 64 multiply-adds and four shifts and masks, where the Shoup
+// product takes seven multiply-adds, three low products and four additions or
+// moves.  Measured with four waves per SIMD, multiply-adds, low products,
+// 64-bit additions and shifts issue one per 4.2 to 4.4 cycles and 32-bit
+// shifts, masks and moves one per 2.5, which makes this product about 35
+// cycles and the Shoup one about 62.  The split at 29 puts the fold at a word
+// boundary of h.  With c < 2^27 and 2c' < 2^32
+// (pm_bits) X < 2^33 q gives (X >> 61) 2c' <= 2^33 c < 2^60, so r < 3 * 2^60 -
+// 2^33 < 3M.
+constexpr uint64_t kPmLow = (1ull << 29) - 1;
+PH_HD uint64_t pm_split(uint64_t w) { return (w & kPmLow) | ((w >> 29) << 32); }
+// b when the products above apply to q, else 0.
+PH_HD int pm_bits(uint64_t q) {
+  int b = 0;
+  while (b < 64 && (q >> b)) ++b;
+  if (b < 50 || b > 60) return 0;
+  const uint64_t c = (1ull << b) - q;
+  return c < (1ull << 27) - 1 && (c << (60 - b)) < (1ull << 31) ? b : 0;
+}
+PH_HD uint64_t mul_pm(uint64_t a, uint64_t w, uint64_t v, uint32_t c2) {
+  const uint32_t a0 = uint32_t(a), a1 = uint32_t(a >> 32);
+  const uint64_t l = uint64_t(a1) * uint32_t(v) + uint64_t(a0) * uint32_t(w);
+  uint64_t h = uint64_t(a0) * uint32_t(w >> 32) + (l >> 29);
+#if defined(__HIP_DEVICE_COMPILE__)
+  h = pin_pair(h);  // one chain of multiply-adds: reassociated, it takes an addition more
+#endif
+  h += uint64_t(a1) * uint32_t(v >> 32);
+  const uint32_t hl = uint32_t(h), lo = (uint32_t(l) & uint32_t(kPmLow)) | (hl << 29);
+  return uint64_t(uint32_t(h >> 32)) * c2 + ((uint64_t(hl >> 3) << 32) | lo);
+}
+// x mod 2^60 + (x >> 60) c' == x (mod q), below 2^60 + 2^35 < 2M for any x.
+PH_HD uint64_t fold_pm(uint64_t x, uint32_t c1) {
+  return uint64_t(uint32_t(x >> 32) >> 28) * c1 + (x & 0x0fffffffffffffffull);
+}
+// Canonical residue of any x < 2^64: x mod 2^b + (x >> b) c < q + 2^32.
+PH_HD uint64_t canon_pm(uint64_t x, uint64_t q, uint32_t c, unsigned sh) {  // sh = b - 32
+  const uint32_t hi = uint32_t(x >> 32);
+  const uint64_t r = uint64_t(hi >> sh) * c + ((uint64_t(hi & ((1u << sh) - 1)) << 32) | uint32_t(x));
+  return r >= q ? r - q : r;
+}
+
 // a*b mod q by Barrett reduction of the 128-bit product x = xh 2^64 + xl with
 // the ratio R = floor((2^128-1)/q) = r1 2^64 + r0 (the reduction SEAL uses,
 // which the reference's kernels call at switch.cu:30-45).  The quotient

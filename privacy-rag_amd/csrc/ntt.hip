@@ -192,7 +192,8 @@ struct TypeTag {
 template <int LOGN>
 static hipError_t launch_ntt_n(bool inverse, uint64_t* data, size_t limbs, const NttDevice& d,
                                hipStream_t s) {
-  // integer-path primes all below 2^60: the lazy transforms (ArU64L)
+  // integer-path primes all just below a power of two: ArPM; all below 2^60:
+  // the lazy transforms (ArU64L)
   const auto u64 = [&](auto tag, bool inv) {
     using A = typename decltype(tag)::type;
     return inv ? launch_subset<LOGN, true, A>(data, limbs, d, d.tw_inv_u, d.sel_u64, d.host_sel_u64, d.n_u64, s)
@@ -203,7 +204,7 @@ static hipError_t launch_ntt_n(bool inverse, uint64_t* data, size_t limbs, const
     e = launch_subset<LOGN, true, ArF64T>(data, limbs, d, d.tw_inv_f, d.sel_f64, d.host_sel_f64, d.n_f64, s);
   else
     e = launch_subset<LOGN, false, ArF64T>(data, limbs, d, d.tw_fwd_f, d.sel_f64, d.host_sel_f64, d.n_f64, s);
-  if (e == hipSuccess && d.n_u64) e = d.lazy_u64 ? u64(TypeTag<ArU64L>{}, inverse) : u64(TypeTag<ArU64>{}, inverse);
+  if (e == hipSuccess && d.n_u64) e = d.pm_u64 ? u64(TypeTag<ArPM>{}, inverse) : d.lazy_u64 ? u64(TypeTag<ArU64L>{}, inverse) : u64(TypeTag<ArU64>{}, inverse);
   return e;
 }
 
@@ -211,10 +212,11 @@ template <int LOGN>
 static hipError_t launch_ntt_lift_n(const uint64_t* ring, size_t width, uint64_t* out, size_t limbs,
                                     const NttDevice& d, hipStream_t s) {
   const NttLift lift{ring, width};
-  return d.lazy_u64 ? launch_subset<LOGN, false, ArU64L, true>(out, limbs, d, d.tw_fwd_u, d.sel_u64, d.host_sel_u64,
-                                                               d.n_u64, s, lift)
-                    : launch_subset<LOGN, false, ArU64, true>(out, limbs, d, d.tw_fwd_u, d.sel_u64, d.host_sel_u64,
-                                                              d.n_u64, s, lift);
+  const auto go = [&](auto tag) {
+    return launch_subset<LOGN, false, typename decltype(tag)::type, true>(out, limbs, d, d.tw_fwd_u, d.sel_u64,
+                                                                          d.host_sel_u64, d.n_u64, s, lift);
+  };
+  return d.pm_u64 ? go(TypeTag<ArPM>{}) : d.lazy_u64 ? go(TypeTag<ArU64L>{}) : go(TypeTag<ArU64>{});
 }
 
 // Every prime on the integer path: the lift is done by the transform's loads.

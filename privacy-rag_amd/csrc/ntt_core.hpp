@@ -20,10 +20,12 @@
 // Arithmetic policies:
 //   ArU64 - any q < 2^62: Harvey's lazy butterflies (forward values in [0,4q),
 //           inverse in [0,2q)) over Shoup twiddle pairs, canonical at the end;
+//   ArPM  - primes just below a power of two: a product with two fixed words
+//           per twiddle and no quotient;
 //   ArF64 - q < 2^50: residues as exact integers in doubles, products with an
 //           error-free FMA split, values re-centred every fourth forward /
 //           third inverse stage.
-// Both produce the canonical residue of the same transform, so the result is
+// All produce the canonical residue of the same transform, so the result is
 // bit-identical to the reference whatever the path.
 #pragma once
 #include "modarith.hpp"
@@ -33,13 +35,14 @@ namespace praghip {
 // Per-prime constants of a plan (device copy).
 struct NttPrime {
   uint64_t q, q2;             // q, 2q
-  uint64_t ninv, ninv_q;      // N^-1 mod q (Shoup pair)
-  uint64_t last, last_q;      // w_last * N^-1 (Shoup pair), w_last = inv[N-1]
+  uint64_t ninv, ninv_q;      // N^-1 mod q (pair of the prime's table form)
+  uint64_t last, last_q;      // w_last * N^-1 (likewise), w_last = inv[N-1]
   double qd, qinv;            // q and 1/q as doubles (float path)
   double ninv_f, last_f;      // N^-1 and w_last * N^-1 as doubles
   uint64_t one_q;             // floor(2^64 / q), the Shoup quotient of 1
   int use_f64;                // q < 2^50: the float path is exact
-  int pad;
+  int pm_bits;                // ArPM: bit length of q; the integer tables and pairs hold (w, w 2^32) split at
+                              // 29 bits instead of (w, Shoup quotient).  0: Shoup pairs
 };
 
 // lift59_residue with the prime's Shoup quotient of 1 instead of a division
@@ -111,7 +114,7 @@ struct ArU64 {
   template <bool UNI = false>
   __device__ __forceinline__ void fwd_at(int, T& x, T& y, TW w) const { fwd<UNI>(x, y, w); }
   template <bool UNI = false>
-  __device__ __forceinline__ void inv(T& x, T& y, TW w) const {  // GS, values in [0,2q)
+  __device__ __forceinline__ void inv_at(int, T& x, T& y, TW w) const {  // GS, values in [0,2q)
     T s = x + y;
     s = s >= q2 ? s - q2 : s;
     const T d = x - y + q2;
@@ -157,7 +160,7 @@ struct ArU64L : ArU64 {
     y = a - t + q2;
   }
   template <bool UNI = false>
-  __device__ __forceinline__ void inv(T& x, T& y, TW w) const {
+  __device__ __forceinline__ void inv_at(int, T& x, T& y, TW w) const {
     T s = x + y;
     s = s >= q4 ? s - q4 : s;
     const T d = x - y + q4;
@@ -184,7 +187,7 @@ struct ArU64L : ArU64 {
 struct ArU64C : ArU64 {
   __device__ explicit ArU64C(const NttPrime& p) : ArU64(p) {}
   template <bool = false>
-  __device__ __forceinline__ void inv(T& x, T& y, TW w) const {
+  __device__ __forceinline__ void inv_at(int, T& x, T& y, TW w) const {
     T s = x + y;
     s = s >= q2 ? s - q2 : s;
     const T d = x - y + q2;
@@ -195,13 +198,70 @@ struct ArU64C : ArU64 {
 struct ArU64LC : ArU64L {
   __device__ explicit ArU64LC(const NttPrime& p) : ArU64L(p) {}
   template <bool = false>
-  __device__ __forceinline__ void inv(T& x, T& y, TW w) const {
+  __device__ __forceinline__ void inv_at(int, T& x, T& y, TW w) const {
     T s = x + y;
     s = s >= q4 ? s - q4 : s;
     const T d = x - y + q4;
     x = s;
     y = mul_shoup_lazy(d, w.x, w.y, q);
   }
+};
+
+// The integer path for primes just below a power of two (pm_bits: the locked
+// primes and every NTT prime of the usual way of choosing them, the largest of
+// their size): butterflies on mul_pm.  What bounds the integer kernels is
+// VALU issue, and a forward butterfly takes about 53 issue cycles here, 79
+// with ArU64L.  Bounds, with M = q 2^(60-b) and products T < 3M:
+//   forward - X + T and X - T + 3M add at most 3 * 2^60, and X is folded
+//             (fold_pm: back to 2^60 + 2^35) at stages 4, 8 and 12, so values
+//             stay below 13 * 2^60 + 2^35;
+//   inverse - before an even stage values are below 4M, before an odd one
+//             below 8M: differences get 8M (below 16M < 2^64), sums are
+//             folded after odd stages only.
+// Measured (us, ArU64L -> ArPM): 32 limbs at N = 4096, forward and inverse,
+// 19.5 -> 15.9; one rotation with six locked one-prime digits 40.6 -> 36.0; the
+// rows of 32 pairs of the packing tree 270 -> 231; 7,296 lifted limbs at
+// N = 16384 729 -> 660.
+struct ArPM {
+  using T = uint64_t;
+  using TW = ulonglong2;  // (w, w 2^32 mod q), each split at 29 bits
+  static constexpr bool kAhead = false;
+  uint64_t q, q4, q8, m3, m8;
+  uint32_t c1, c2, c;
+  unsigned sh;
+  PH_HD explicit ArPM(const NttPrime& p) : q(p.q), q4(4 * p.q), q8(8 * p.q) {
+    const uint64_t m = p.q << (60 - p.pm_bits);
+    m3 = 3 * m;
+    m8 = 8 * m;
+    c1 = uint32_t((1ull << 60) - m);
+    c2 = 2 * c1;
+    c = c1 >> (60 - p.pm_bits);
+    sh = unsigned(p.pm_bits) - 32;
+  }
+  PH_HD T from_u64(uint64_t x) const { return x; }
+  PH_HD uint64_t to_u64_fwd(T x) const { return canon_pm(x, q, c, sh); }
+  PH_HD uint64_t to_u64_inv(T x) const { return canon_pm(x, q, c, sh); }
+  template <bool = false>
+  PH_HD void fwd_at(int s, T& x, T& y, TW w) const {
+    const T a = s > 0 && s % 4 == 0 ? fold_pm(x, c1) : x;
+    const T t = mul_pm(y, w.x, w.y, c2);
+    x = a + t;
+    y = a + m3 - t;
+  }
+  template <bool = false>
+  PH_HD void inv_at(int l, T& x, T& y, TW w) const {
+    const T s = x + y, d = x + m8 - y;
+    x = l % 2 ? fold_pm(s, c1) : s;
+    y = mul_pm(d, w.x, w.y, c2);
+  }
+  PH_HD void inv_last(T& x, T& y, const NttPrime& p) const {
+    const T s = x + y, d = x + m8 - y;
+    x = mul_pm(s, p.ninv, p.ninv_q, c2);
+    y = mul_pm(d, p.last, p.last_q, c2);
+  }
+  PH_HD void settle(T&) const {}
+  static constexpr bool settle_fwd(int) { return false; }
+  static constexpr bool settle_inv(int) { return false; }
 };
 
 // Float path bounds (q < 2^50, |x| <= M q, mul_f64 gives |t| <= (1/2 + 3A/8) q
@@ -243,7 +303,7 @@ struct ArF64 {
   template <bool = false>
   __device__ __forceinline__ void fwd_at(int, T& x, T& y, TW w) const { fwd(x, y, w); }
   template <bool = false>
-  __device__ __forceinline__ void inv(T& x, T& y, TW w) const {
+  __device__ __forceinline__ void inv_at(int, T& x, T& y, TW w) const {
     const T s = x + y, d = x - y;
     x = s;
     y = mul(d, w);
@@ -477,7 +537,7 @@ __device__ __forceinline__ void inv_pass(typename A::T (&v)[E], const typename A
           if (l == LOGN - 1)  // last stage: one group, twiddle and N^-1 folded
             ar.inv_last(v[j0], v[j1], pr);
           else
-            ar.template inv<UNI>(v[j0], v[j1], w[n]);
+            ar.template inv_at<UNI>(l, v[j0], v[j1], w[n]);
         }
       }
       if (A::settle_inv(l) && l != LOGN - 1) {

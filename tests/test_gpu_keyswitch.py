@@ -14,6 +14,16 @@ pytestmark = pytest.mark.gpu
 P16384_SWITCH = cf.primes_below(50, 16384, 6) + cf.primes_below(60, 16384, 1)
 
 
+def _primes_under(top, n, count):
+    """The largest primes == 1 mod 2n below `top`."""
+    out, v = [], (top - 2) // (2 * n) * 2 * n + 1
+    while len(out) < count:
+        if cf.is_prime(v):
+            out.append(v)
+        v -= 2 * n
+    return out
+
+
 def test_keyswitch_golden_fixtures(gpu, golden_dir):
     data = np.load(os.path.join(golden_dir, "keyswitch_small.npz"))
     tags = sorted({k.rsplit("_", 1)[0] for k in data.files})
@@ -280,7 +290,7 @@ def test_keyswitch_wide_special_prime_three_phase(gpu, bits, dnum):
     (13, "locked", 6, 6, 1), (13, "50", 6, 4, 2), (13, "50", 5, 2, 17), (13, "locked", 3, 2, 66),
     (14, "50", 6, 5, 1), (14, "locked", 6, 4, 1), (14, "locked", 5, 2, 4), (14, "50", 5, 2, 3), (14, "50", 3, 2, 33),
     (14, "locked", 4, 3, 22), (14, "50", 5, 4, 17), (14, "locked", 6, 5, 14)])
-def test_keyswitch_rows_shapes(gpu, log_n, kind, L, dnum, batch):
+def test_keyswitch_rows_sizes_and_digits(gpu, log_n, kind, L, dnum, batch):
     """The three-phase kernels over their sizes, unequal digits and batches on
     both sides of every launch rule (targets spread over threads, digits over
     wave pairs, the special prime's columns formed by each data prime), with the
@@ -301,3 +311,23 @@ def test_keyswitch_rows_shapes(gpu, log_n, kind, L, dnum, batch):
         for b in sorted({0, batch // 2, batch - 1}):
             want = oracle.keyswitch(ct[b:b + 1], keys[k], q, dnum, log_n, g)[0]
             np.testing.assert_array_equal(got[b], want, err_msg=f"key {k} galois {g} ciphertext {b}")
+
+
+@pytest.mark.parametrize("log_n,L,dnum,batch", [(14, 4, 4, 2), (14, 3, 1, 1), (13, 3, 2, 1), (12, 2, 2, 40), (11, 3, 3, 2)])
+def test_keyswitch_primes_off_a_power_of_two(gpu, log_n, L, dnum, batch):
+    """Integer primes below 2^60 but not just below a power of two: Shoup tables
+    and butterflies (the locked and the largest primes of a size take the
+    two-word products), on the three-phase and the whole-limb kernels; exact."""
+    n = 1 << log_n
+    q = _primes_under(3 << 57, n, L) + cf.primes_below(60, n, 1)
+    print(f"[ks] off-power primes N={n} L={L} dnum={dnum} batch={batch}", flush=True)
+    ct = oracle.fill_residues(batch * 2 * L, n, q[:L], 0x79 + batch).reshape(batch, 2, L, n)
+    ct[0, 1] = np.array(q[:L], dtype=np.uint64)[:, None] - np.uint64(1)
+    key = oracle.fill_residues(dnum * 2 * (L + 1), n, q, 0x7a + L).reshape(dnum, 2, L + 1, n)
+    key[0] = (np.array(q, dtype=np.uint64) - np.uint64(1))[None, :, None]
+    sw = praghip.Switch(q, log_n, dnum, max_batch=batch)
+    tin, tout, tk = to_dev(ct), to_dev(np.zeros_like(ct)), to_dev(key)
+    sw.keyswitch(tin, tout, keys=tk, key_stride=0, galois=3)
+    got = from_dev(tout)
+    for b in sorted({0, batch - 1}):
+        np.testing.assert_array_equal(got[b], oracle.keyswitch(ct[b:b + 1], key, q, dnum, log_n, 3)[0])

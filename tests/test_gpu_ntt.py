@@ -223,3 +223,19 @@ def test_device_binding_by_uuid_and_pci(gpu, monkeypatch):
     t = to_dev(a)
     plan.forward(t)
     np.testing.assert_array_equal(from_dev(t), oracle.ntt(a, oracle.Tables(q, 10)))
+
+
+@pytest.mark.parametrize("log_n", [4, 5, 8, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("bits", [0, 51, 54, 57, 60])
+def test_ntt_integer_prime_forms(gpu, log_n, bits):
+    """The integer transforms by prime: just below 2^bits (two-word twiddles,
+    alone and with a float-path prime before the last), and with 0 far from
+    every power of two (Shoup twiddles); words at q - 1 among them; exact."""
+    n = 1 << log_n
+    if bits:
+        q = cf.primes_below(bits, n, 2)
+        _roundtrip_case([cf.primes_below(50, n, 1)[0], q[1]], log_n, 5, 0x99 + log_n, gpu)
+    else:
+        top = (3 << 57) // (2 * n) * 2 * n + 1
+        q = [v for v in range(top - 600 * 2 * n, top, 2 * n) if cf.is_prime(v)][-2:]
+    _roundtrip_case(q, log_n, 7, 0x98 + log_n, gpu)
