@@ -28,6 +28,11 @@ struct NttDevice {
 };
 
 hipError_t launch_ntt(bool inverse, uint64_t* data, size_t limbs, const NttDevice& d, hipStream_t s);
+// Inverse transform of [slots][2][P][N] with the token path's finish on the way
+// to out: scaled[slot][p] added to coefficient width - 1 of component 0, then
+// the limb times x^-(width-1).  data is used up.
+hipError_t launch_ntt_finish(uint64_t* data, const uint64_t* scaled, uint64_t* out, size_t slots, size_t width,
+                             const NttDevice& d, hipStream_t s);
 hipError_t launch_dyadic_shoup(uint64_t* data, const ulonglong2* key, const NttDevice& d, size_t words,
                                hipStream_t s);
 
@@ -136,8 +141,6 @@ constexpr size_t kNoAllocSlots = 64;
 hipError_t local_dot_scratch(int device, uint64_t** address);
 
 // Token-resident path and packing tree (token.hip).
-hipError_t launch_token_finish(const uint64_t* in, const uint64_t* scaled, uint64_t* out, size_t slots,
-                               const PrimeList& pl, int log_n, size_t width, hipStream_t s);
 // out[c][l][N] = sum_b in[b][l] (.) w[c][b][l % P] over `coords` weight
 // columns sharing the resident inputs in [blocks][limbs][N]; w is
 // [coords][blocks][P][N], out [coords][limbs][N].

@@ -23,7 +23,7 @@ namespace praghip {
 // no registers to spare and load each limb at the top of its turn.
 //
 // LIFT (forward only): limb l = b P + k is not read from data but formed on
-// load from ring block b, lift59_residue mod q_k (ring[b][z] when width = 0;
+// load from ring block b, lift_word mod q_k (ring[b][z] when width = 0;
 // ring[b][width-1-z] for z < width and 0 above otherwise), so the lifted limbs
 // never pass through memory.
 struct NttLift {
@@ -31,13 +31,39 @@ struct NttLift {
   size_t width = 0;
 };
 
-template <int LOGN, bool INV, class A, bool LIFT = false>
+// FINISH (inverse only): limb l = (slot * 2 + c) P + p is not stored in place but
+// finished on the way out (resident.cu:54-59 add_shift): in component 0
+// scaled[slot][p] is added to coefficient `lift`, and the limb times x^-lift
+// goes to out, so the products are not read and written once more (64 columns
+// of 4 slots, us: 271 for the transform and 176 for the finish as a pass of its
+// own -> 293 together).
+struct NttFinish {
+  uint64_t* out = nullptr;
+  const uint64_t* scaled = nullptr;
+  unsigned lift = 0;
+};
+
+// The signed value of ring word v (bit 58 the sign) as a forward transform's
+// input: canonical, or for ArPM below M by one masked addition of M - 2^59 (M is
+// a multiple of q above 2^59 whatever q's size).
+template <class A>
+__device__ __forceinline__ uint64_t lift_word(const A& ar, uint64_t v, const NttPrime& pr) {
+  if constexpr (std::is_same<A, ArPM>::value)
+    return v + (((ar.m8 >> 3) - (1ull << 59)) & (0ull - (v >> 58)));
+  else
+    return lift59_residue(v, pr);
+}
+
+template <int LOGN, bool INV, class A, bool LIFT = false, bool FINISH = false>
 __global__ void __launch_bounds__(ntt_threads<LOGN>())
     ntt_kernel(uint64_t* __restrict__ data, size_t count, const NttPrime* __restrict__ primes,
-               const typename A::TW* __restrict__ tw, int P, const int* __restrict__ sel, int C, NttLift lift) {
+               const typename A::TW* __restrict__ tw, int P, const int* __restrict__ sel, int C, NttLift lift,
+               NttFinish fin) {
   __shared__ __attribute__((aligned(16))) uint64_t lds[(1 << LOGN) + (1 << LOGN) / 16];
   using T = typename A::T;
-  const unsigned t = threadIdx.x;
+  // with FINISH recomputed per limb (v < 2^40): the output indices would
+  // otherwise be kept in registers across the loop and spill
+  unsigned t = threadIdx.x;
   const auto limb_of = [&](size_t v) { return (v / unsigned(C)) * unsigned(P) + unsigned(sel[v % unsigned(C)]); };
   const auto in_index = [&](int j) { return INV ? inv_in_index<LOGN>(t, j) : fwd_in_index<LOGN>(t, j); };
   // the input words of limb `limb` in the first pass's register layout (with
@@ -62,15 +88,26 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
       for (int j = 0; j < kE; ++j) raw[j] = x[in_index(j)];
     }
   };
-  const auto lifted = [&](uint64_t v, const NttPrime& pr) {
+  const auto lifted = [&](uint64_t v, const A& ar, const NttPrime& pr) {
     if constexpr (LIFT)
-      return lift59_residue(v, pr);
+      return lift_word(ar, v, pr);
     else
       return v;
   };
-  const auto store = [&](const A& ar, T (&x)[kE], size_t limb) {
-    uint64_t* out = data + (limb << LOGN);
-    if (!INV) {
+  const auto store = [&](const A& ar, T (&x)[kE], size_t limb, const NttPrime& pr) {
+    uint64_t* out = (FINISH ? fin.out : data) + (limb << LOGN);
+    if constexpr (FINISH) {
+      const size_t row = limb / unsigned(P), slot = row >> 1;  // row = slot * 2 + component
+      const uint64_t add = row & 1 ? 0 : fin.scaled[slot * unsigned(P) + limb % unsigned(P)];
+#pragma unroll
+      for (int j = 0; j < kE; ++j) {
+        const unsigned z = inv_out_index<LOGN>(t, j);
+        uint64_t v = ar.to_u64_inv(x[j]);
+        if (z == fin.lift) v = add_mod(v, add, pr.q);
+        out[(z - fin.lift) & ((1u << LOGN) - 1)] = z < fin.lift && v ? pr.q - v : v;
+        if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else if (!INV) {
 #pragma unroll
       for (int j = 0; j < kE; j += 2)
         *reinterpret_cast<ulonglong2*>(out + fwd_out_index<LOGN>(t, j)) =
@@ -92,12 +129,12 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
       const A ar(pr);
       T x[kE];
 #pragma unroll
-      for (int j = 0; j < kE; ++j) x[j] = ar.from_u64(lifted(raw[j], pr));
+      for (int j = 0; j < kE; ++j) x[j] = ar.from_u64(lifted(raw[j], ar, pr));
       const size_t vn = v + gridDim.x;
       ntt_regs<LOGN, INV>(x, reinterpret_cast<T*>(lds), t, tw + (size_t(p) << LOGN), ar, pr, [&] {
         if (vn < count) load(raw, limb_of(vn));
       });
-      store(ar, x, limb);
+      store(ar, x, limb, pr);
     }
   } else if constexpr (std::is_same<T, double>::value && INV) {
     // the next limb's first-pass twiddles are loaded before this limb's
@@ -125,11 +162,12 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
       run_passes<LOGN, INV, 0>(x, reinterpret_cast<T*>(lds), t, tw + (size_t(p) << LOGN), ar, pr, w0, [] {});
       const size_t vn = v + gridDim.x;
       if (vn < count) load_pass_twiddles<LOGN, INV, 0>(w0, t, tw + ((limb_of(vn) % unsigned(P)) << LOGN));
-      store(ar, x, limb);
+      store(ar, x, limb, pr);
       if (vn < count) load(raw, limb_of(vn));
     }
   } else {
     for (size_t v = blockIdx.x; v < count; v += gridDim.x) {
+      if constexpr (FINISH) t = threadIdx.x + unsigned(v >> 40);
       const size_t limb = limb_of(v);
       const int p = int(limb % unsigned(P));
       const NttPrime pr = primes[p];
@@ -138,15 +176,15 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
       load(raw, limb);
       T x[kE];
 #pragma unroll
-      for (int j = 0; j < kE; ++j) x[j] = ar.from_u64(lifted(raw[j], pr));
+      for (int j = 0; j < kE; ++j) x[j] = ar.from_u64(lifted(raw[j], ar, pr));
       ntt_regs<LOGN, INV>(x, reinterpret_cast<T*>(lds), t, tw + (size_t(p) << LOGN), ar, pr);
-      store(ar, x, limb);
+      store(ar, x, limb, pr);
     }
   }
 }
 
 // Resident workgroups per CU times the CU count, cached per kernel.
-template <int LOGN, bool INV, class A, bool LIFT>
+template <int LOGN, bool INV, class A, bool LIFT, bool FINISH>
 static unsigned persistent_grid() {
   static unsigned grid = 0;
   if (!grid) {
@@ -154,7 +192,8 @@ static unsigned persistent_grid() {
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ntt_kernel<LOGN, INV, A, LIFT>, ntt_threads<LOGN>(), 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (ntt_kernel<LOGN, INV, A, LIFT, FINISH>), ntt_threads<LOGN>(),
+                                                     0) !=
             hipSuccess ||
         per_cu < 1)
       per_cu = 1;
@@ -171,16 +210,17 @@ static size_t subset_count(size_t limbs, int P, const int* host_sel, int C) {
   return count;
 }
 
-template <int LOGN, bool INV, class A, bool LIFT = false>
+template <int LOGN, bool INV, class A, bool LIFT = false, bool FINISH = false>
 static hipError_t launch_subset(uint64_t* data, size_t limbs, const NttDevice& d, const typename A::TW* tw,
-                                const int* sel_dev, const int* sel_host, int C, hipStream_t s, NttLift lift = {}) {
+                                const int* sel_dev, const int* sel_host, int C, hipStream_t s, NttLift lift = {},
+                                NttFinish fin = {}) {
   if (!C) return hipSuccess;
   const size_t count = subset_count(limbs, d.P, sel_host, C);
   if (!count) return hipSuccess;
   const dim3 block{unsigned(ntt_threads<LOGN>())};
-  const dim3 grid{unsigned(std::min<size_t>(count, persistent_grid<LOGN, INV, A, LIFT>()))};
-  hipLaunchKernelGGL((ntt_kernel<LOGN, INV, A, LIFT>), grid, block, 0, s, data, count, d.primes, tw, d.P, sel_dev, C,
-                     lift);
+  const dim3 grid{unsigned(std::min<size_t>(count, persistent_grid<LOGN, INV, A, LIFT, FINISH>()))};
+  hipLaunchKernelGGL((ntt_kernel<LOGN, INV, A, LIFT, FINISH>), grid, block, 0, s, data, count, d.primes, tw, d.P,
+                     sel_dev, C, lift, fin);
   return hipGetLastError();
 }
 
@@ -208,13 +248,103 @@ static hipError_t launch_ntt_n(bool inverse, uint64_t* data, size_t limbs, const
   return e;
 }
 
+// The lifted transform at N = 16384 by half limbs.  A whole limb's exchange
+// buffer (136 KiB) leaves one workgroup on a CU, whose loads, stages and stores
+// follow one another; two half-limb workgroups (68 KiB, 512 threads) fill the
+// same registers and run each other's gaps.  Stage 0 pairs the halves, so each
+// workgroup forms it from the ring words of both and keeps its own side - the
+// ring is not written, so there is no order between the two.  When the ring
+// block reaches half the limb at most (kReversedLow) the upper half is
+// zero, the stage changes nothing and costs nothing.  Every limb half of a ring
+// block runs on one XCD (workgroup % 8), whose L2 then holds the block.
+// 7,296 limbs (19 blocks x 64 columns x 6 primes), width 8192: 660 us by whole
+// limbs, 601 here (VALU issue bounds both).
+constexpr int kHalfLog = 13;
+enum HalfInput { kPlain, kReversed, kReversedLow };  // width 0, above N / 2, up to N / 2
+template <class A, HalfInput IN>
+__global__ void __launch_bounds__(1 << (kHalfLog - kLogE)) __attribute__((amdgpu_waves_per_eu(4)))
+    ntt_lift_half_kernel(uint64_t* __restrict__ out, size_t blocks, const NttPrime* __restrict__ primes,
+                         const typename A::TW* __restrict__ tw, int P, const int* __restrict__ sel, int C,
+                         NttLift lift) {
+  constexpr unsigned kHalf = 1u << kHalfLog;
+  __shared__ __attribute__((aligned(16))) uint64_t lds[kHalf + kHalf / 16];
+  const unsigned items = 2 * unsigned(C);
+  const size_t total = (blocks + 7) / 8 * 8 * items;
+  for (size_t v = blockIdx.x; v < total; v += gridDim.x) {  // gridDim is a multiple of 8
+    const size_t seq = v >> 3, b = seq / items * 8 + (v & 7);
+    if (b >= blocks) continue;
+    const unsigned t = threadIdx.x + unsigned(v >> 40);  // recomputed per item: no index kept across the loop
+    const unsigned sub = unsigned(seq % items), h = sub & 1u, p = unsigned(sel[sub >> 1]);
+    const NttPrime pr = primes[p];
+    const A ar(pr);
+    // coefficient z is ring[b][z], or ring[b][width - 1 - z] and zero from width on
+    const typename A::TW* tab = tw + (size_t(p) << (kHalfLog + 1));
+    const unsigned z0 = fwd_in_index<kHalfLog>(t, 0), width = unsigned(lift.width);
+    const uint64_t* first = IN == kPlain ? lift.ring + (b << (kHalfLog + 1)) + z0
+                                         : lift.ring + b * lift.width + lift.width - 1 - (long long)z0;
+    const auto word = [&](unsigned d) {  // of coefficient z0 + d
+      if constexpr (IN == kPlain)
+        return first[d];
+      else
+        return z0 + d < width ? *(first - d) : 0;
+    };
+    uint64_t x[kE];
+#pragma unroll
+    for (int j = 0; j < kE; ++j) x[j] = word(PassMap<kHalfLog, false, 0>::reg_field(j));
+#pragma unroll
+    for (int j = 0; j < kE; ++j) x[j] = ar.from_u64(lift_word(ar, x[j], pr));
+    if constexpr (IN != kReversedLow) {
+      const typename A::TW w = load_invariant(tab + 1);
+#pragma unroll
+      for (int j = 0; j < kE; ++j) {
+        uint64_t y = ar.from_u64(lift_word(ar, word(PassMap<kHalfLog, false, 0>::reg_field(j) + kHalf), pr));
+        ar.template fwd_at<true>(0, x[j], y, w);
+        x[j] = h ? y : x[j];
+        if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four words of the other half in registers at a time
+      }
+    }
+    run_part_passes<kHalfLog + 1, kHalfLog, 0>(x, lds, t, h, tab, ar);
+    uint64_t* o = out + ((b * unsigned(P) + p) << (kHalfLog + 1)) + size_t(h) * kHalf;
+#pragma unroll
+    for (int j = 0; j < kE; j += 2)
+      *reinterpret_cast<ulonglong2*>(o + fwd_out_index<kHalfLog>(t, j)) =
+          make_ulonglong2(ar.to_u64_fwd(x[j]), ar.to_u64_fwd(x[j + 1]));
+    __syncthreads();  // the next half's first exchange reuses the LDS
+  }
+}
+
+template <class A, HalfInput IN>
+static hipError_t launch_lift_half(uint64_t* out, size_t blocks, const NttDevice& d, NttLift lift, hipStream_t s) {
+  static unsigned resident = 0;
+  if (!resident) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      cus = 256;
+    resident = unsigned(cus + 7) / 8 * 8 * 2;
+  }
+  const size_t total = (blocks + 7) / 8 * 8 * 2 * size_t(d.n_u64);
+  hipLaunchKernelGGL((ntt_lift_half_kernel<A, IN>), dim3(unsigned(std::min<size_t>(total, resident))),
+                     dim3(1 << (kHalfLog - kLogE)), 0, s, out, blocks, d.primes, d.tw_fwd_u, d.P, d.sel_u64, d.n_u64,
+                     lift);
+  return hipGetLastError();
+}
+
 template <int LOGN>
 static hipError_t launch_ntt_lift_n(const uint64_t* ring, size_t width, uint64_t* out, size_t limbs,
                                     const NttDevice& d, hipStream_t s) {
   const NttLift lift{ring, width};
   const auto go = [&](auto tag) {
-    return launch_subset<LOGN, false, typename decltype(tag)::type, true>(out, limbs, d, d.tw_fwd_u, d.sel_u64,
-                                                                          d.host_sel_u64, d.n_u64, s, lift);
+    if constexpr (LOGN == kHalfLog + 1) {
+      using A = typename decltype(tag)::type;
+      const size_t blocks = limbs / unsigned(d.P);
+      return !width ? launch_lift_half<A, kPlain>(out, blocks, d, lift, s)
+             : width > (size_t(1) << kHalfLog) ? launch_lift_half<A, kReversed>(out, blocks, d, lift, s)
+                                               : launch_lift_half<A, kReversedLow>(out, blocks, d, lift, s);
+    } else {
+      return launch_subset<LOGN, false, typename decltype(tag)::type, true>(out, limbs, d, d.tw_fwd_u, d.sel_u64,
+                                                                            d.host_sel_u64, d.n_u64, s, lift);
+    }
   };
   return d.pm_u64 ? go(TypeTag<ArPM>{}) : d.lazy_u64 ? go(TypeTag<ArU64L>{}) : go(TypeTag<ArU64>{});
 }
@@ -243,6 +373,40 @@ hipError_t launch_ntt_lift(const uint64_t* ring, size_t width, uint64_t* out, si
     case 12: return launch_ntt_lift_n<12>(ring, width, out, limbs, d, s);
     case 13: return launch_ntt_lift_n<13>(ring, width, out, limbs, d, s);
     case 14: return launch_ntt_lift_n<14>(ring, width, out, limbs, d, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int LOGN>
+static hipError_t launch_ntt_finish_n(uint64_t* data, size_t limbs, const NttDevice& d, NttFinish fin, hipStream_t s) {
+  hipError_t e = launch_subset<LOGN, true, ArF64T, false, true>(data, limbs, d, d.tw_inv_f, d.sel_f64, d.host_sel_f64,
+                                                                d.n_f64, s, {}, fin);
+  const auto go = [&](auto tag) {
+    return launch_subset<LOGN, true, typename decltype(tag)::type, false, true>(data, limbs, d, d.tw_inv_u, d.sel_u64,
+                                                                                d.host_sel_u64, d.n_u64, s, {}, fin);
+  };
+  if (e == hipSuccess && d.n_u64)
+    e = d.pm_u64 ? go(TypeTag<ArPM>{}) : d.lazy_u64 ? go(TypeTag<ArU64L>{}) : go(TypeTag<ArU64>{});
+  return e;
+}
+
+hipError_t launch_ntt_finish(uint64_t* data, const uint64_t* scaled, uint64_t* out, size_t slots, size_t width,
+                             const NttDevice& d, hipStream_t s) {
+  const size_t limbs = slots * 2 * size_t(d.P);
+  if (limbs == 0) return hipSuccess;
+  const NttFinish fin{out, scaled, unsigned(width - 1)};
+  switch (d.log_n) {
+    case 4: return launch_ntt_finish_n<4>(data, limbs, d, fin, s);
+    case 5: return launch_ntt_finish_n<5>(data, limbs, d, fin, s);
+    case 6: return launch_ntt_finish_n<6>(data, limbs, d, fin, s);
+    case 7: return launch_ntt_finish_n<7>(data, limbs, d, fin, s);
+    case 8: return launch_ntt_finish_n<8>(data, limbs, d, fin, s);
+    case 9: return launch_ntt_finish_n<9>(data, limbs, d, fin, s);
+    case 10: return launch_ntt_finish_n<10>(data, limbs, d, fin, s);
+    case 11: return launch_ntt_finish_n<11>(data, limbs, d, fin, s);
+    case 12: return launch_ntt_finish_n<12>(data, limbs, d, fin, s);
+    case 13: return launch_ntt_finish_n<13>(data, limbs, d, fin, s);
+    case 14: return launch_ntt_finish_n<14>(data, limbs, d, fin, s);
     default: return hipErrorInvalidValue;
   }
 }

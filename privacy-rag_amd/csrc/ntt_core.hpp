@@ -442,32 +442,34 @@ constexpr int pass_tw_count() {
   return pass_twiddles<R, LE>();
 }
 
-template <int LOGN, bool INV, int P, int LE, class TW>
+// LOGT > LOGN: the 2^LOGN coefficients are part `row` (the same in every lane) of
+// a transform of 2^LOGT whose table `tab` is.
+template <int LOGN, bool INV, int P, int LE, class TW, int LOGT = LOGN>
 __device__ __forceinline__ void load_pass_twiddles_e(TW (&w)[(pass_tw_count<LOGN, INV, P, LE>())], unsigned t,
-                                                     const TW* __restrict__ tab) {
+                                                     const TW* __restrict__ tab, unsigned row = 0) {
   using M = PassMap<LOGN, INV, P, LE>;
   constexpr int LO = M::LO, R = M::R, SUB = (1 << LE) >> R;
-  constexpr unsigned N = 1u << LOGN;
+  constexpr unsigned N = 1u << LOGT;
   int n = 0;
 #pragma unroll
   for (int b = 0; b < SUB; ++b) {
     // group index of the block: the coefficient bits above the gap bits.
     // When no lane bit lies there, all lanes of a wave share it and the
     // twiddle loads go through the scalar unit into SGPRs.
-    const unsigned hi_lane = M::elem(t, b << R) >> (LO + R);
+    const unsigned hi_lane = ((row << LOGN) | M::elem(t, b << R)) >> (LO + R);
     const unsigned hi = M::uniform_groups() ? __builtin_amdgcn_readfirstlane(hi_lane) : hi_lane;
     const auto ld = [&](unsigned x) { return M::uniform_groups() ? load_invariant(tab + x) : tab[x]; };
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       if (!INV) {
-        const int s = LOGN - LO - R + i;
+        const int s = LOGT - LO - R + i;
 #pragma unroll
         for (int k = 0; k < (1 << i); ++k) w[n++] = ld((1u << s) + (hi << i) + k);
       } else {
         const int l = LO + i;
 #pragma unroll
         for (int k = 0; k < (1 << (R - 1 - i)); ++k) {
-          if (l != LOGN - 1) w[n] = ld(N - (N >> l) + 1 + (hi << (R - 1 - i)) + k);
+          if (l != LOGT - 1) w[n] = ld(N - (N >> l) + 1 + (hi << (R - 1 - i)) + k);
           ++n;
         }
       }
@@ -618,6 +620,22 @@ __device__ __forceinline__ void run_passes(typename A::T (&v)[kE], typename A::T
       inv_pass<LOGN, LO, R, UNI>(v, w, ar, pr, [] {});
     else
       fwd_pass<LOGN, LO, R, UNI>(v, w, ar, [] {});
+  }
+}
+
+// Forward passes P .. NP - 1 of part `row` of a transform of 2^LOGT, the part's
+// 2^LOGN coefficients in registers; each pass's twiddles loaded when it starts.
+template <int LOGT, int LOGN, int P, class A>
+__device__ __forceinline__ void run_part_passes(typename A::T (&v)[kE], typename A::T* lds, unsigned t, unsigned row,
+                                                const typename A::TW* __restrict__ tab, const A& ar) {
+  using S = Passes<LOGN>;
+  constexpr int LO = S::lo(false, P), R = S::r(false, P);
+  typename A::TW w[pass_twiddles<R>()];
+  load_pass_twiddles_e<LOGN, false, P, kLogE, typename A::TW, LOGT>(w, t, tab, row);
+  fwd_pass<LOGT, LO, R, PassMap<LOGN, false, P>::uniform_groups()>(v, w, ar, [] {});
+  if constexpr (P + 1 < S::NP) {
+    exchange<LOGN, false, P>(v, lds, t);
+    run_part_passes<LOGT, LOGN, P + 1>(v, lds, t, row, tab, ar);
   }
 }
 

@@ -745,11 +745,11 @@ PrimeList token_primes(const praghip_token_plan* p) {
   pl.count = int(p->P);
   return pl;
 }
-// lift + NTT (one pass) -> sum over blocks -> (INTT) into p->output.  ev
+// lift + NTT (one pass) -> sum over blocks into p->output.  ev
 // (null: none) receives events after the lift (ev[0], only when the lift is a
 // kernel of its own, i.e. a prime is on the float path), after the transform
 // (ev[1]) and after the sum (ev[2]).
-hipError_t token_product(praghip_token_plan* p, const uint64_t* ring_dev, bool inverse, hipStream_t s,
+hipError_t token_product(praghip_token_plan* p, const uint64_t* ring_dev, hipStream_t s,
                          hipEvent_t* ev = nullptr) {
   Barrett m[kMaxKeyPrimes];
   for (size_t i = 0; i < p->P; ++i) m[i] = barrett_of(p->host_q[i]);
@@ -766,14 +766,13 @@ hipError_t token_product(praghip_token_plan* p, const uint64_t* ring_dev, bool i
   if (e == hipSuccess)
     e = launch_dyadic_mac(p->input, p->weight, p->output, p->blocks, limbs, int(p->log_n), p->P, m, int(p->P), s);
   if (e == hipSuccess && ev) e = hipEventRecord(ev[2], s);
-  if (e == hipSuccess && inverse) e = launch_ntt(true, p->output, limbs, p->d, s);
   return e;
 }
 // the whole evaluate_device path; residues [slots][P] device, or null for the
 // bound local shares
 hipError_t token_finished(praghip_token_plan* p, const uint64_t* ring_dev, const uint64_t* residues, uint64_t* out,
                           hipStream_t s, hipEvent_t* ev = nullptr) {
-  hipError_t e = token_product(p, ring_dev, true, s, ev);
+  hipError_t e = token_product(p, ring_dev, s, ev);
   if (e == hipSuccess && !residues) {
     Barrett m[kMaxKeyPrimes];
     for (size_t i = 0; i < p->P; ++i) m[i] = barrett_of(p->host_q[i]);
@@ -782,7 +781,7 @@ hipError_t token_finished(praghip_token_plan* p, const uint64_t* ring_dev, const
     residues = p->scaled;
   }
   if (e == hipSuccess)
-    e = launch_token_finish(p->output, residues, out, p->slots, token_primes(p), int(p->log_n), p->width, s);
+    e = launch_ntt_finish(p->output, residues, out, p->slots, p->width, p->d, s);
   return e;
 }
 // Delta_k = floor(Q / 2^59) mod q_k and r = Q mod 2^59, Q = prod q (the
@@ -942,7 +941,7 @@ int praghip_token_evaluate(praghip_token_plan* p, const uint64_t* ring, size_t w
   if (e == hipSuccess) e = hipEventRecord(p->ev[0], s);
   if (e == hipSuccess) e = hipMemcpyAsync(p->ring, ring, words * 8, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipEventRecord(p->ev[1], s);
-  if (e == hipSuccess) e = token_product(p, p->ring, false, s, p->ev + 2);
+  if (e == hipSuccess) e = token_product(p, p->ring, s, p->ev + 2);
   if (e == hipSuccess) e = hipEventRecord(p->ev[5], s);
   if (e == hipSuccess) e = hipMemcpyAsync(output, p->output, p->words * 8, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipEventRecord(p->ev[6], s);
@@ -1070,14 +1069,13 @@ int praghip_token_evaluate_device_batch(praghip_token_plan* p, const uint64_t* r
   if (e == hipSuccess) e = launch_ntt_lift(rings, p->width, p->bweight, coords * p->blocks, pl, p->d, s);
   if (e == hipSuccess)
     e = launch_token_mac(p->input, p->bweight, p->boutput, coords, p->blocks, limbs, int(p->log_n), m, int(p->P), s);
-  if (e == hipSuccess) e = launch_ntt(true, p->boutput, coords * limbs, p->d, s);
   if (e == hipSuccess && !residues) {
     e = launch_local_dot_scale(p->local_shares, rings, words, p->slots, p->delta.data(), p->r, m, int(p->P),
                                p->bscaled, p->bpartial, s, coords);
     residues = p->bscaled;
   }
   if (e == hipSuccess)
-    e = launch_token_finish(p->boutput, residues, output, coords * p->slots, pl, int(p->log_n), p->width, s);
+    e = launch_ntt_finish(p->boutput, residues, output, coords * p->slots, p->width, p->d, s);
   if (e != hipSuccess) return token_failure(p, e, "evaluate_device_batch");
   return PRAGHIP_OK;
 }

@@ -1,8 +1,5 @@
 // Element-wise kernels of the token-resident path and of the acyclic packing
 // tree:
-//   token_finish: the Delta-scaled local term added to coefficient
-//     block_width-1 of c0, then the product multiplied by x^-(block_width-1)
-//     (resident.cu:54-59 add_shift);
 //   pack_prepare: right * x^shift, then the sum and the Galois image of the
 //     difference of a packing pair (switch.cu:49-58 packing_prepare);
 //   pack_finish: the two switched halves added (switch.cu:59-61).
@@ -18,111 +15,186 @@ static unsigned elem_grid(size_t items) {
   return unsigned(std::min<size_t>(std::max<size_t>((items + 255) / 256, 1), 1u << 20));
 }
 
-// out[slot][c][p][d] = x^-(w-1) * (in[slot][c][p] + [c == 0] scaled[slot][p] x^(w-1)),
-// negacyclic: source j = d + w - 1 (kept) or d + w - 1 - N (negated).
-__global__ void __launch_bounds__(256)
-    token_finish_kernel(const uint64_t* __restrict__ in, const uint64_t* __restrict__ scaled,
-                        uint64_t* __restrict__ out, size_t slots, PrimeList pl, int log_n, size_t width) {
-  const size_t n = size_t(1) << log_n, P = size_t(pl.count), total = slots * 2 * P * n;
-  const size_t lift = width - 1;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += size_t(gridDim.x) * blockDim.x) {
-    const size_t d = i & (n - 1), limb = i >> log_n, p = limb % P, c = (limb / P) & 1, slot = limb / (2 * P);
-    const uint64_t q = pl.q[p];
-    const bool wrap = d + lift >= n;
-    const size_t j = wrap ? d + lift - n : d + lift;
-    uint64_t v = in[(limb << log_n) + j];
-    if (c == 0 && j == lift) v = add_mod(v, scaled[slot * P + p], q);
-    out[i] = (wrap && v) ? q - v : v;
+// Sum of products of a batch of weight columns against the resident inputs:
+//   out[c][l][z] = sum_b in[b][l][z] * w[c][b][l % P][z]  mod q_{l % P}
+// (resident.cu:38-45 accumulate), for every column c of the batch.
+//
+// For primes below 2^60 no product is reduced: with both words split
+// at 30 bits a product is four 32 x 32 multiply-adds into three sums (weights
+// 1, 2^30, 2^60), and the sums are brought below q once per sixteen blocks
+// (the middle sum takes two products a block and is carried into the upper one
+// after eight) - about 7
+// instructions per product at 19 blocks instead of 20 with a Shoup product
+// each.  A thread holds KL limbs (of one prime) x kMacCoords columns of one
+// coefficient; every input word then meets four columns and every weight word
+// KL limbs.
+//
+// What bounds it then is the memory, so workgroups are numbered for the L2:
+// the ones on one XCD (blockIdx % 8) that share a prime's 256 coefficients come
+// one after the other - every column group and limb tile of them - and the
+// input words (19 blocks x 8 limbs: 311 KB) are read from HBM once.
+// 64 columns, 19 blocks, 48 limbs at N = 16384 (1.5 GB): 796 us with Shoup
+// products and the columns walked over all of N, 448 here.
+//
+// MODE: kMacPm   - primes just below 2^60 (2^60 == c): the sums are brought
+//                  together by three multiply-adds;
+//       kMacNarrow - any primes below 2^60: by a Shoup product by 2^60;
+//       kMacWide - primes of 2^60 and more.
+//
+// Primes of 2^60 and more: a Shoup quotient per weight word (from the Barrett
+// ratio), Shoup products and canonical sums.
+constexpr int kMacCoords = 4;
+enum MacMode { kMacPm, kMacNarrow, kMacWide };
+constexpr uint64_t kMacLow = (1ull << 30) - 1;
+
+struct MacConst {
+  uint64_t q, one_q, c60, c60_q;  // q, Shoup quotient of 1, c60 = 2^60 mod q with its quotient
+  uint32_t c;                     // kMacPm: M = q 2^(60-b) = 2^60 - c (pm_bits b, c < 2^28)
+  int bits;
+};
+
+// s0 + s1 2^30 + s2 2^60 mod q as some word below 2^62.
+template <MacMode MODE>
+__device__ __forceinline__ uint64_t mac_fold(uint64_t s0, uint64_t s1, uint64_t s2, const MacConst& m) {
+  s1 += s0 >> 30;
+  s2 += s1 >> 30;
+  const uint64_t low = ((s1 & kMacLow) << 30) | (s0 & kMacLow);
+  if constexpr (MODE == kMacPm) {
+    // s2 2^60 == s2 c; u = (s2 >> 32) c < 2^60 stands at 2^32: its part from
+    // 2^60 on, below 2^32, meets c again
+    const uint64_t u = uint64_t(uint32_t(s2 >> 32)) * m.c;
+    return uint64_t(uint32_t(s2)) * m.c + uint64_t(uint32_t(u >> 28)) * m.c + low + ((u & 0xfffffffull) << 32);
+  } else {
+    return mul_shoup_lazy(s2, m.c60, m.c60_q, m.q) + low;
   }
 }
 
-hipError_t launch_token_finish(const uint64_t* in, const uint64_t* scaled, uint64_t* out, size_t slots,
-                               const PrimeList& pl, int log_n, size_t width, hipStream_t s) {
-  const size_t total = slots * 2 * size_t(pl.count) << log_n;
-  hipLaunchKernelGGL(token_finish_kernel, dim3(elem_grid(total)), dim3(256), 0, s, in, scaled, out, slots, pl, log_n,
-                     width);
-  return hipGetLastError();
-}
-
-// Sum of products of a batch of weight columns against the resident inputs:
-//   out[c][l][z] = sum_b in[b][l][z] * w[c][b][l % P][z]  mod q_{l % P}
-// (resident.cu:38-45 accumulate), for every column c of the batch.  One thread
-// per (coordinate group, prime p, coefficient z) walks all limbs l = p (mod P)
-// and kMacCoords columns: each weight word is read once and each input word
-// once per column group, instead of once per column.  A weight word meets up
-// to KL inputs (KL limb slots per thread: 8 for the token path's slots x 2P
-// limbs, 2 for a single ciphertext's 2P, so no slot multiplies zeros), so it
-// gets a Shoup quotient (from the Barrett ratio)
-// and the products are Shoup products: exact, like the reference's Barrett-128
-// products, with fewer 64-bit multiplies.  LAZY (every prime below 2^60): the
-// products are left in [0, 2q) and the sums reduced by 8q after every fourth
-// block, so they stay below 16q < 2^64, and made canonical once at the end.
-constexpr int kMacCoords = 4;
-template <bool LAZY, int KL>
+template <MacMode MODE, int KL>
 __global__ void __launch_bounds__(256)
     token_mac_kernel(const uint64_t* __restrict__ in, const uint64_t* __restrict__ w, uint64_t* __restrict__ out,
-                     size_t coords, size_t blocks, size_t limbs, int log_n, BarrettList bl) {
-  const size_t n = size_t(1) << log_n, P = size_t(bl.count), groups = (coords + kMacCoords - 1) / kMacCoords;
-  const size_t words = limbs << log_n, wcol = blocks * P << log_n, total = groups * P << log_n;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += size_t(gridDim.x) * blockDim.x) {
-    const size_t z = i & (n - 1), p = (i >> log_n) % P, c0 = ((i >> log_n) / P) * kMacCoords;
-    const Barrett m = bl.m[p];
-    const size_t cn = coords - c0 < size_t(kMacCoords) ? coords - c0 : size_t(kMacCoords);
-    for (size_t l0 = p; l0 < limbs; l0 += KL * P) {
-      uint64_t acc[kMacCoords][KL];
+                     unsigned coords, unsigned blocks, unsigned limbs, int log_n, BarrettList bl, unsigned tiles,
+                     unsigned groups, unsigned places) {
+  // blockIdx = ((place / 8) * groups * tiles + group * tiles + tile) * 8 + place % 8,
+  // place = (prime, 256 coefficients)
+  const unsigned x8 = blockIdx.x & 7u, y = blockIdx.x >> 3, inner = groups * tiles;
+  const unsigned place = (y / inner) * 8u + x8, gt = y % inner;
+  if (place >= places) return;
+  const unsigned P = unsigned(bl.count), n = 1u << log_n, zs = (n + 255u) / 256u;
+  const unsigned p = place / zs, z = (place % zs) * 256u + threadIdx.x;
+  if (z >= n) return;
+  const unsigned c0 = (gt / tiles) * unsigned(kMacCoords);
+  const unsigned l0 = p + (gt % tiles) * unsigned(KL) * P;  // limbs l0, l0 + P, ...
+  if (l0 >= limbs) return;
+  const Barrett m = bl.m[p];
+  const size_t words = size_t(limbs) << log_n, wcol = (size_t(blocks) * P) << log_n;
+  const unsigned cn = coords - c0 < unsigned(kMacCoords) ? coords - c0 : unsigned(kMacCoords);
+  // past the last limb or column a thread works on the last one again and
+  // does not store it: no branch in the loop
+  size_t xo[KL], wo[kMacCoords];
 #pragma unroll
-      for (int c = 0; c < kMacCoords; ++c)
+  for (int k = 0; k < KL; ++k) {
+    const unsigned l = l0 + unsigned(k) * P;
+    xo[k] = size_t(l < limbs ? l : l0) << log_n;
+  }
 #pragma unroll
-        for (int k = 0; k < KL; ++k) acc[c][k] = 0;
-      for (size_t b = 0; b < blocks; ++b) {
-        uint64_t x[KL];
+  for (int c = 0; c < kMacCoords; ++c)
+    wo[c] = (c0 + (unsigned(c) < cn ? unsigned(c) : 0u)) * wcol + (size_t(p) << log_n);
+  const auto store = [&](int c, int k, uint64_t v) {
+    const unsigned l = l0 + unsigned(k) * P;
+    if (unsigned(c) < cn && l < limbs) (out + (size_t(c0) + unsigned(c)) * words + (size_t(l) << log_n))[z] = v;
+  };
+  if constexpr (MODE != kMacWide) {
+    MacConst mc;
+    mc.q = m.q;
+    mc.one_q = m.r1;                                // floor(2^64 / q)
+    mc.c60 = (1ull << 60) - (m.r1 >> 4) * m.q;      // 2^60 mod q
+    mc.c60_q = shoup_quotient(mc.c60, m);
+    mc.bits = 64 - __clzll((long long)m.q);
+    mc.c = uint32_t((1ull << 60) - (m.q << (60 - mc.bits)));
+    uint64_t s0[kMacCoords][KL], s1[kMacCoords][KL], s2[kMacCoords][KL];
 #pragma unroll
-        for (int k = 0; k < KL; ++k) {
-          const size_t l = l0 + size_t(k) * P;
-          x[k] = l < limbs ? in[b * words + (l << log_n) + z] : 0;
-        }
+    for (int c = 0; c < kMacCoords; ++c)
 #pragma unroll
-        for (int c = 0; c < kMacCoords; ++c) {
-          if (size_t(c) >= cn) break;
-          const uint64_t wv = w[(c0 + c) * wcol + ((b * P + p) << log_n) + z];
-          const uint64_t wq = shoup_quotient(wv, m);
+      for (int k = 0; k < KL; ++k) s0[c][k] = s1[c][k] = s2[c][k] = 0;
+    // the next block's words are in flight while this block's are multiplied
+    uint64_t xn[KL], wn[kMacCoords];
+    const auto load = [&](unsigned b) {
+      const uint64_t* xb = in + size_t(b) * words;
+      const uint64_t* wb = w + ((size_t(b) * P) << log_n);
+#pragma unroll
+      for (int k = 0; k < KL; ++k) xn[k] = (xb + xo[k])[z];
+#pragma unroll
+      for (int c = 0; c < kMacCoords; ++c) wn[c] = (wb + wo[c])[z];
+    };
+    load(0);
+    for (unsigned b = 0; b < blocks; ++b) {
+      uint32_t x0[KL], x1[KL], w0[kMacCoords], w1[kMacCoords];
+#pragma unroll
+      for (int k = 0; k < KL; ++k) x0[k] = uint32_t(xn[k]) & uint32_t(kMacLow), x1[k] = uint32_t(xn[k] >> 30);
+#pragma unroll
+      for (int c = 0; c < kMacCoords; ++c) w0[c] = uint32_t(wn[c]) & uint32_t(kMacLow), w1[c] = uint32_t(wn[c] >> 30);
+      if (b + 1 < blocks) load(b + 1);
+      if (b && b % 8 == 0) {
+#pragma unroll
+        for (int c = 0; c < kMacCoords; ++c)
 #pragma unroll
           for (int k = 0; k < KL; ++k) {
-            if constexpr (LAZY) {
-              acc[c][k] += mul_shoup_lazy(x[k], wv, wq, m.q);
-            } else {
-              const uint64_t v = acc[c][k] + mul_shoup(x[k], wv, wq, m.q);
-              acc[c][k] = v >= m.q ? v - m.q : v;
+            if (b % 16) {
+              // sixteen products of s2 and both carries of s1 stay below 2^64:
+              // 16 (2^30 - 1)^2 + 2 (2^34 - 31) + 16 = 2^64 - 30
+              s2[c][k] += s1[c][k] >> 30;
+              s1[c][k] &= kMacLow;
+            } else {  // below 2^62: s1 restarts below 2^32
+              const uint64_t r = mac_fold<MODE>(s0[c][k], s1[c][k], s2[c][k], mc);
+              s0[c][k] = r & kMacLow;
+              s1[c][k] = r >> 30;
+              s2[c][k] = 0;
             }
           }
-        }
-        if constexpr (LAZY) {
-          if ((b & 3) == 3) {
-            const uint64_t q8 = 8 * m.q;
-#pragma unroll
-            for (int c = 0; c < kMacCoords; ++c)
-#pragma unroll
-              for (int k = 0; k < KL; ++k) acc[c][k] = acc[c][k] >= q8 ? acc[c][k] - q8 : acc[c][k];
-          }
-        }
       }
 #pragma unroll
-      for (int c = 0; c < kMacCoords; ++c) {
-        if (size_t(c) >= cn) break;
+      for (int k = 0; k < KL; ++k) {
 #pragma unroll
-        for (int k = 0; k < KL; ++k) {
-          const size_t l = l0 + size_t(k) * P;
-          uint64_t v = acc[c][k];
-          if constexpr (LAZY) {  // below 16q -> [0, q)
-            v = v >= 8 * m.q ? v - 8 * m.q : v;
-            v = v >= 4 * m.q ? v - 4 * m.q : v;
-            v = v >= 2 * m.q ? v - 2 * m.q : v;
-            v = v >= m.q ? v - m.q : v;
-          }
-          if (l < limbs) out[(c0 + c) * words + (l << log_n) + z] = v;
+        for (int c = 0; c < kMacCoords; ++c) {
+          s0[c][k] += uint64_t(x0[k]) * w0[c];
+          s1[c][k] += uint64_t(x0[k]) * w1[c];
+          s1[c][k] += uint64_t(x1[k]) * w0[c];
+          s2[c][k] += uint64_t(x1[k]) * w1[c];
         }
       }
     }
+#pragma unroll
+    for (int c = 0; c < kMacCoords; ++c)
+#pragma unroll
+      for (int k = 0; k < KL; ++k) {
+        const uint64_t r = mac_fold<MODE>(s0[c][k], s1[c][k], s2[c][k], mc);
+        if constexpr (MODE == kMacPm)
+          store(c, k, canon_pm(r, m.q, mc.c >> (60 - mc.bits), unsigned(mc.bits) - 32));
+        else
+          store(c, k, mul_shoup(r, 1, mc.one_q, m.q));
+      }
+  } else {
+    uint64_t acc[kMacCoords][KL];
+#pragma unroll
+    for (int c = 0; c < kMacCoords; ++c)
+#pragma unroll
+      for (int k = 0; k < KL; ++k) acc[c][k] = 0;
+    for (unsigned b = 0; b < blocks; ++b) {
+      uint64_t xv[KL];
+#pragma unroll
+      for (int k = 0; k < KL; ++k) xv[k] = (in + size_t(b) * words + xo[k])[z];
+#pragma unroll
+      for (int c = 0; c < kMacCoords; ++c) {
+        const uint64_t wv = (w + wo[c] + ((size_t(b) * P) << log_n))[z];
+        const uint64_t wq = shoup_quotient(wv, m);
+#pragma unroll
+        for (int k = 0; k < KL; ++k) acc[c][k] = add_mod(acc[c][k], mul_shoup(xv[k], wv, wq, m.q), m.q);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kMacCoords; ++c)
+#pragma unroll
+      for (int k = 0; k < KL; ++k) store(c, k, acc[c][k]);
   }
 }
 
@@ -131,19 +203,30 @@ hipError_t launch_token_mac(const uint64_t* in, const uint64_t* w, uint64_t* out
   BarrettList bl{};
   for (int i = 0; i < primes; ++i) bl.m[i] = m[i];
   bl.count = primes;
-  bool lazy = true;
-  for (int i = 0; i < primes; ++i) lazy = lazy && m[i].q < (1ull << 60);
-  const size_t total = ((coords + kMacCoords - 1) / kMacCoords * size_t(primes)) << log_n;
-  // limb slots per thread: the limbs of one prime, rounded up to 2, 4 or 8
-  const size_t per = (limbs + size_t(primes) - 1) / size_t(primes);
-  const int kl = per <= 2 ? 2 : (per <= 4 ? 4 : 8);
+  MacMode mode = kMacPm;
+  for (int i = 0; i < primes; ++i) {
+    const int b = pm_bits(m[i].q);
+    if (m[i].q >> 60)
+      mode = kMacWide;
+    else if (mode == kMacPm && (!b || ((1ull << 60) - (m[i].q << (60 - b))) >> 28))
+      mode = kMacNarrow;
+  }
+  // limbs of one prime: 2 per thread for a single ciphertext's, else 4 (24
+  // 64-bit sums are 96 registers; 8 limbs would leave two waves per SIMD)
+  const unsigned per = unsigned((limbs + size_t(primes) - 1) / size_t(primes)), kl = per <= 2 ? 2 : 4;
+  const unsigned tiles = (per + kl - 1) / kl, groups = unsigned((coords + kMacCoords - 1) / kMacCoords);
+  const unsigned places = unsigned(primes) * unsigned(((size_t(1) << log_n) + 255) / 256);
+  const dim3 grid((places + 7) / 8 * 8 * groups * tiles);
   const auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(elem_grid(total)), dim3(256), 0, s, in, w, out, coords, blocks, limbs, log_n, bl);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, w, out, unsigned(coords), unsigned(blocks), unsigned(limbs),
+                       log_n, bl, tiles, groups, places);
   };
-  if (lazy)
-    kl == 2 ? go(token_mac_kernel<true, 2>) : kl == 4 ? go(token_mac_kernel<true, 4>) : go(token_mac_kernel<true, 8>);
+  if (mode == kMacPm)
+    kl == 2 ? go(token_mac_kernel<kMacPm, 2>) : go(token_mac_kernel<kMacPm, 4>);
+  else if (mode == kMacNarrow)
+    kl == 2 ? go(token_mac_kernel<kMacNarrow, 2>) : go(token_mac_kernel<kMacNarrow, 4>);
   else
-    kl == 2 ? go(token_mac_kernel<false, 2>) : kl == 4 ? go(token_mac_kernel<false, 4>) : go(token_mac_kernel<false, 8>);
+    kl == 2 ? go(token_mac_kernel<kMacWide, 2>) : go(token_mac_kernel<kMacWide, 4>);
   return hipGetLastError();
 }
 

@@ -218,3 +218,32 @@ def test_enc0_batch(gpu):
         z.reserve(count + 1)
     c = z.close()
     assert c.closed and c.wipe_synchronized_bytes == c.freed_bytes > 0
+
+
+@pytest.mark.parametrize("primes", ["locked", "50bit", "59bit", "62bit"])
+@pytest.mark.parametrize("blocks,groups", [(1, 1), (8, 5), (9, 4), (16, 3), (17, 2), (33, 1)])
+def test_matrix_batch_largest_sums(gpu, primes, blocks, groups):
+    """The column product's sums at their largest: every transformed input and
+    weight word q - 1 (a constant polynomial -1 is -1 at every point), over
+    block counts on both sides of the sums' carries and folds, ragged column
+    groups, and primes on each way of folding; exact."""
+    import torch
+    n, log_n = 1 << 10, 10
+    q = {"locked": cf.LOCKED_PRIMES[:3], "50bit": cf.primes_below(50, n, 3), "62bit": cf.primes_below(62, n, 3),
+         "59bit": [v for v in range((3 << 57) + 1, (3 << 57) + 400 * 2 * n, 2 * n) if cf.is_prime(v)][:3]}[primes]
+    print(f"[matrix-sums] {primes} blocks={blocks} groups={groups}", flush=True)
+    ct = np.zeros((blocks, 2, 3, n), dtype=np.uint64)
+    ct[:, :, :, 0] = np.array(q, dtype=np.uint64) - np.uint64(1)
+    ct[:, 1, :, 1:] = oracle.fill_residues(blocks * 3, n, q, 9).reshape(blocks, 3, n)[:, :, 1:]
+    rings = np.zeros((groups, blocks, n), dtype=np.uint64)
+    rings[:, :, 0] = T59
+    rings[groups // 2:, :, 1:] = oracle.fill_u64(blocks * n, 10).reshape(blocks, n)[:, 1:] & np.uint64(T59)
+    m = praghip.Matrix(q, log_n, ct)
+    m.reserve(groups)
+    out = to_dev(np.zeros((groups, 2, 3, n), dtype=np.uint64))
+    m.evaluate_device_batch(to_dev(rings), out)
+    torch.cuda.synchronize()
+    got = from_dev(out)
+    for g in sorted({0, groups - 1}):
+        np.testing.assert_array_equal(got[g], oracle.matrix_product(ct, rings[g], q, log_n), err_msg=f"group {g}")
+    m.close()

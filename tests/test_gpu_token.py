@@ -378,3 +378,32 @@ def test_token_batch(gpu, log_n, P, blocks, slots, width, coords, locked):
         tw.evaluate_device_batch(to_dev(np.concatenate([rings, rings[:1]])),
                                  torch.zeros((coords + 1) * slots * 2 * P * n, dtype=torch.int64, device="cuda"))
     tw.close()
+
+
+@pytest.mark.parametrize("primes", ["locked", "offpower", "62bit"])
+@pytest.mark.parametrize("width,blocks", [(1, 1), (100, 9), (8191, 2), (8192, 8), (8193, 3), (16384, 2)])
+def test_token_half_limb_lift(gpu, primes, width, blocks):
+    """The lifted transform by half limbs (N = 16384) and the finish in the
+    inverse transform's stores: widths on both sides of half a limb, block
+    counts off a multiple of eight, each integer form, words at both signs'
+    largest; exact."""
+    import torch
+    log_n, n, slots, coords = 14, 1 << 14, 1, 2
+    q = {"locked": cf.LOCKED_PRIMES[:2], "62bit": cf.primes_below(62, n, 2),
+         "offpower": [v for v in range((3 << 57) + 1, (3 << 57) + 400 * 2 * n, 2 * n) if cf.is_prime(v)][:2]}[primes]
+    print(f"[token-half] {primes} width={width} blocks={blocks}", flush=True)
+    ct = _inputs(q, n, blocks, slots, 41)
+    bound = 1 << 20
+    rings = (oracle.fill_u64(coords * blocks * width, 42) % np.uint64(2 * bound + 1)).astype(np.int64) - bound
+    rings = (rings.reshape(coords, blocks, width) & ((1 << 59) - 1)).astype(np.uint64)
+    rings[0, 0, 0], rings[0, 0, -1] = (1 << 59) - bound, bound
+    local = [[int(v) & MASK59 for v in oracle.fill_u64(slots, 43 + c)] for c in range(coords)]
+    plan = praghip.TokenWeights(q, log_n, ct, width)
+    plan.reserve(coords)
+    scaled = np.stack([oracle.token_scaled(local[c], q) for c in range(coords)])
+    out = to_dev(np.zeros((coords, slots, 2, 2, n), dtype=np.uint64))
+    plan.evaluate_device_batch(to_dev(rings), out, residues=to_dev(scaled))
+    torch.cuda.synchronize()
+    got = from_dev(out)
+    for c in range(coords):
+        np.testing.assert_array_equal(got[c], oracle.token_finished(ct, rings[c], scaled[c], q, log_n, width))
