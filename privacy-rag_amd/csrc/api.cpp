@@ -703,8 +703,10 @@ int build_ks_const(const uint64_t* q, size_t L, size_t dnum, unsigned log_n, KsC
     kc.last_r[t] = Shoup{lr, shoup_q(lr, q[t])};
   }
   kc.pm = kc.lazy && pm_plan(q, K) ? 1 : 0;
+  kc.pm_sums = kc.pm;
   for (size_t t = 0; kc.pm && t < K; ++t) {
     if (!pm_bits(q[t])) continue;  // a float-path prime
+    kc.pm_sums &= (((1ull << 60) - (q[t] << (60 - pm_bits(q[t])))) >> 28) == 0 ? 1 : 0;
     for (Shoup* c : {&kc.ninv_r[t], &kc.last_r[t]}) {
       const ulonglong2 w = pm_pair(c->w, c->wq, q[t]);
       *c = Shoup{w.x, w.y};

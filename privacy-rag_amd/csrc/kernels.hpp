@@ -57,6 +57,7 @@ struct KsConst {
   Shoup ninv_r[kMaxKeyPrimes];           // N^-1 2^64 mod q_t
   Shoup last_r[kMaxKeyPrimes];           // w_last N^-1 2^64 mod q_t (w_last = inv[N-1])
   int pm;                                // ArPM on the integer path (ninv_r, last_r in its form)
+  int pm_sums;                           // and 2^60 - M < 2^28 for every prime: unreduced key-product sums (sum_pm)
 };
 
 struct KsArgs {

@@ -62,6 +62,7 @@ struct KsRows {
   int moddown_f64;  // every data prime in (2^32, 2^50): ModDown in FP64 too
   int narrow;       // every key prime below twice every other: x mod q_t by one subtraction
   unsigned big;     // digits of the larger size (the first ones)
+  int mont;         // the products lack the factor 2^64 of Montgomery key products
   unsigned b0, cts;  // chunk: ciphertexts b0 .. b0 + cts - 1
 };
 
@@ -499,13 +500,12 @@ __device__ __forceinline__ void row_passes_e(typename A::T (&v)[E], typename A::
 // every digit's forward passes read them there, so no vector-memory load
 // stands between a digit's row and key loads and their use.
 constexpr unsigned kRowTw = (1u << kRowLog) - 1;
-constexpr int kRowKeyPass = 3;
 
-template <int LOG, class TW>
+template <int LOG, unsigned TH, class TW>
 __device__ __forceinline__ void row_twiddles_fill(TW* ltw, const TW* __restrict__ tab, unsigned row, unsigned t2) {
 #pragma unroll
-  for (unsigned i = 0; i < (kRowTw + kRow2Threads - 1) / kRow2Threads; ++i) {
-    const unsigned e = t2 + i * kRow2Threads;
+  for (unsigned i = 0; i < (kRowTw + TH - 1) / TH; ++i) {
+    const unsigned e = t2 + i * TH;
     if (e < kRowTw) {
       const unsigned m = e + 1, sl = 31u - unsigned(__builtin_clz(m));  // s - kColLog
       ltw[e] = tab[(1u << (sl + kColLog<LOG>)) + (row << sl) + (m - (1u << sl))];
@@ -569,14 +569,16 @@ __device__ __forceinline__ void row_passes_fwd_lds(typename A::T (&v)[E], typena
 // g, g + groups, ... on its own exchange buffer lds (of the array all_lds), the
 // pairs' sums meet in LDS, and pairs 0 and 1 transform one sum each (the other
 // pairs run the same passes on what they hold, for the barriers in them).
-template <int LOG, class A, bool SPLIT>
+template <int LOG, class A, bool SPLIT, bool SUMS>
 __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, unsigned bl, unsigned t,
                                           unsigned row, unsigned t2, typename A::T* lds, typename A::TW* ltw,
                                           unsigned g = 0, unsigned groups = 1, typename A::T* all_lds = nullptr) {
   using T = typename A::T;
-  constexpr int E = 1 << kRowLE;
+  constexpr int LE = SUMS ? 2 : kRowLE, E = 1 << LE;
+  constexpr unsigned TH = 1u << (kRowLog - LE);  // threads of the item
+  constexpr int KP = Passes<kRowLog, LE>::NP - 1;  // the pass at whose start the key words are loaded
   constexpr bool kF64 = std::is_same<T, double>::value;
-  constexpr bool kMont = mont_keys<A>;
+  constexpr bool kSums = SUMS && std::is_same<A, ArPM>::value, kMont = mont_keys<A> && !kSums;
   const unsigned dnum = unsigned(kc.dnum), K = unsigned(kc.K);
   const unsigned b = f.b0 + bl;
   const NttPrime pr = f.primes[t];
@@ -590,15 +592,22 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
   // twiddle loads are issued first, so their wait before the LDS writes
   // leaves the row's loads in flight)
   if constexpr (SPLIT) {
-    if (g == 0) row_twiddles_fill<LOG>(ltw, fwd_table<LOG, A>(f, int(t)), row, t2);
+    if (g == 0) row_twiddles_fill<LOG, TH>(ltw, fwd_table<LOG, A>(f, int(t)), row, t2);
   } else {
-    row_twiddles_fill<LOG>(ltw, fwd_table<LOG, A>(f, int(t)), row, t2);
+    row_twiddles_fill<LOG, TH>(ltw, fwd_table<LOG, A>(f, int(t)), row, t2);
   }
   uint64_t en[E];
 #pragma unroll
-  for (int k = 0; k < E; ++k) en[k] = __builtin_nontemporal_load(&e0[g * e_step + fwd_in_index<kRowLog, kRowLE>(t2, k)]);
+  for (int k = 0; k < E; ++k) en[k] = __builtin_nontemporal_load(&e0[g * e_step + fwd_in_index<kRowLog, LE>(t2, k)]);
   __syncthreads();
   T a0[E], a1[E];
+  uint64_t s0[2][kSums ? E : 1], s1[2][kSums ? E : 1], s2[2][kSums ? E : 1];
+  if constexpr (kSums) {
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) s0[c][k] = s1[c][k] = s2[c][k] = 0;
+  }
   if constexpr (kMont || kF64) {
 #pragma unroll
     for (int k = 0; k < E; ++k) a0[k] = a1[k] = 0;
@@ -614,19 +623,19 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
     if (j + groups < dnum) {  // the next digit's row, in flight during this digit's passes
       const uint64_t* src = e0 + (j + groups) * e_step;
 #pragma unroll
-      for (int k = 0; k < E; ++k) en[k] = __builtin_nontemporal_load(&src[fwd_in_index<kRowLog, kRowLE>(t2, k)]);
+      for (int k = 0; k < E; ++k) en[k] = __builtin_nontemporal_load(&src[fwd_in_index<kRowLog, LE>(t2, k)]);
     }
-    // the digit's key words, issued at the start of forward pass kRowKeyPass:
+    // the digit's key words, issued at the start of forward pass KP:
     // registers r, r + 1 hold adjacent coefficients after the last forward
     // pass, so one 16-byte load per key limb and pair
     const uint64_t* k0 = kb + ((size_t(j) * 2 * K) << LOG);
     const uint64_t* k1 = k0 + (size_t(K) << LOG);
     ulonglong2 kav[E / 2], kkv[E / 2];
-    row_passes_fwd_lds<LOG, 0, kRowKeyPass>(v, lds, t2, ltw, ar, [&] {
+    row_passes_fwd_lds<LOG, 0, KP>(v, lds, t2, ltw, ar, [&] {
       if (SPLIT && j >= dnum) return;
 #pragma unroll
       for (int r = 0; r < E; r += 2) {
-        const unsigned pos = (row << kRowLog) | fwd_out_index<kRowLog, kRowLE>(t2, r);
+        const unsigned pos = (row << kRowLog) | fwd_out_index<kRowLog, LE>(t2, r);
         if (own_keys) {
           const u64x2 a = __builtin_nontemporal_load(reinterpret_cast<const u64x2*>(k0 + pos));
           const u64x2 c = __builtin_nontemporal_load(reinterpret_cast<const u64x2*>(k1 + pos));
@@ -653,6 +662,18 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
           // q/2 + 1 + 4 (1.8 q) < 8 q < 2^53
           a0[rr] += ar.mul(v[rr], ArF64::from_u64(w0));
           a1[rr] += ar.mul(v[rr], ArF64::from_u64(w1));
+        } else if constexpr (kSums) {
+          const uint64_t x = fold_pm(v[rr], ar.c1);  // below 2^60 + 2^35
+          const uint32_t x0 = uint32_t(x) & uint32_t(kLow30), x1 = uint32_t(x >> 30);
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const uint64_t w = c ? w1 : w0;
+            const uint32_t k0 = uint32_t(w) & uint32_t(kLow30), k1 = uint32_t(w >> 30);
+            s0[c][rr] += uint64_t(x0) * k0;
+            s1[c][rr] += uint64_t(x0) * k1;
+            s1[c][rr] += uint64_t(x1) * k0;
+            s2[c][rr] += uint64_t(x1) * k1;
+          }
         } else if constexpr (kMont) {
           // any x < 2^64, canonical key words: each product < 2q
           a0[rr] += mul_mont(v[rr], w0, ar.q, kc.neg_qinv[t]);
@@ -666,7 +687,17 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
         }
       }
     }
-    if constexpr (kMont) {
+    if constexpr (kSums) {
+      if ((n & 3) == 3) {  // eight products of 2^60 in s1, at most 15 in s2
+#pragma unroll
+        for (int k = 0; k < E; ++k)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            s2[c][k] += s1[c][k] >> 30;
+            s1[c][k] &= kLow30;
+          }
+      }
+    } else if constexpr (kMont) {
       if ((n & 3) == 3) {  // sums below 16q: reduced by 8q every fourth digit
 #pragma unroll
         for (int k = 0; k < E; ++k) {
@@ -685,6 +716,13 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
     }
     // the next digit's first exchange writes the LDS this digit's last one
     // read, and crosses the waves: it starts with a workgroup barrier
+  }
+  if constexpr (kSums) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      a0[k] = sum_pm(s0[0][k], s1[0][k], s2[0][k], ar.c1);  // below 4M, the inverse's input bound
+      a1[k] = sum_pm(s0[1][k], s1[1][k], s2[1][k], ar.c1);
+    }
   }
   if constexpr (kF64) {  // re-centred, |x| <= q/2 + 1: the inverse passes' input bound
 #pragma unroll
@@ -709,7 +747,7 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
       __syncthreads();  // earlier reads of the buffers are over
       if (g != c) {
 #pragma unroll
-        for (int k = 0; k < E; ++k) lds[unsigned(k) * kRow2Threads + t2] = a[k];
+        for (int k = 0; k < E; ++k) lds[unsigned(k) * TH + t2] = a[k];
       }
       __syncthreads();
       if (g == c) {
@@ -718,7 +756,7 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
           const T* src = all_lds + o * kRowLds;
 #pragma unroll
           for (int k = 0; k < E; ++k) {
-            const T x = src[unsigned(k) * kRow2Threads + t2];
+            const T x = src[unsigned(k) * TH + t2];
             if constexpr (kF64) {
               a[k] += x;  // at most six re-centred sums: below 4 q
             } else if constexpr (kMont) {
@@ -755,13 +793,13 @@ __device__ __forceinline__ void row_item2(const KsRows& f, const KsConst& kc, un
   row_passes_e<LOG, true, 0>(a0, lds, t2, row, ti, ari, pr);
   if (SPLIT && g > 1) return;
 #pragma unroll
-  for (int k = 0; k < E; ++k) pb[inv_out_index<kRowLog, kRowLE>(t2, k)] = store_form<A>(a0[k]);
+  for (int k = 0; k < E; ++k) pb[inv_out_index<kRowLog, LE>(t2, k)] = store_form<A>(a0[k]);
   if constexpr (SPLIT) return;
   __syncthreads();  // the second transform's first exchange reuses the LDS
   row_passes_e<LOG, true, 0>(a1, lds, t2, row, ti, ari, pr);
   uint64_t* pc = pb + (size_t(K) << LOG);
 #pragma unroll
-  for (int k = 0; k < E; ++k) pc[inv_out_index<kRowLog, kRowLE>(t2, k)] = store_form<A>(a1[k]);
+  for (int k = 0; k < E; ++k) pc[inv_out_index<kRowLog, LE>(t2, k)] = store_form<A>(a1[k]);
 }
 
 // One workgroup (two waves) per item; items [0, u64_items) are the
@@ -780,13 +818,32 @@ __global__ void __launch_bounds__(kRow2Threads) __attribute__((amdgpu_waves_per_
   if (item >= f.cts * K * rows) return;
   if (item < u64_items) {
     const unsigned row = item % rows, t = t_u64 + (item / rows) % n_u64, bl = item / (rows * n_u64);
-    row_item2<LOG, AU, false>(f, kc, bl, t, row, t2, lds, ltw);
+    row_item2<LOG, AU, false, false>(f, kc, bl, t, row, t2, lds, ltw);
   } else {
     const unsigned x = item - u64_items;
     const unsigned row = x % rows, t = (x / rows) % t_u64, bl = x / (rows * t_u64);
-    row_item2<LOG, ArF64Lean, false>(f, kc, bl, t, row, t2, reinterpret_cast<double*>(lds),
+    row_item2<LOG, ArF64Lean, false, false>(f, kc, bl, t, row, t2, reinterpret_cast<double*>(lds),
                                      reinterpret_cast<double*>(ltw));
   }
+}
+
+// Every key prime on ArPM: four coefficients per lane on four waves, and the key
+// products of the digits in three unreduced sums each (words split at 30 bits,
+// four multiply-adds a product, one reduction at the end) instead of a
+// Montgomery product per digit - about 32 issue cycles a product against 85.
+// The sums take three times the registers, which four coefficients per lane
+// hold at four waves per SIMD.  64 ciphertexts with six one-prime digits and a
+// shared key, N = 16384: 225 us with Montgomery products, 210 here (233 with
+// eight coefficients per lane, two waves per SIMD).
+template <int LOG>
+__global__ void __launch_bounds__(4 * 64) __attribute__((amdgpu_waves_per_eu(4))) ks_rows4_kernel(KsRows f) {
+  __shared__ __attribute__((aligned(16))) uint64_t lds[kRowLds];
+  __shared__ ulonglong2 ltw[kRowTw];
+  const KsConst& kc = *f.kc;
+  const unsigned K = unsigned(kc.K), item = blockIdx.x;
+  constexpr unsigned rows = kLen<LOG> >> kRowLog;
+  const unsigned row = item % rows, t = (item / rows) % K, bl = item / (rows * K);
+  row_item2<LOG, ArPM, false, true>(f, kc, bl, t, row, threadIdx.x, lds, ltw);
 }
 
 // The same items with the digits of each spread over `groups` (2..6) pairs of
@@ -807,10 +864,10 @@ __global__ void __launch_bounds__(kRow2Threads * kRowGroupsMax) ks_rows_split_ke
   constexpr unsigned rows = kLen<LOG> >> kRowLog;
   const unsigned row = blockIdx.x % rows, t = (blockIdx.x / rows) % K, bl = blockIdx.x / (rows * K);
   if (t >= t_u64) {
-    row_item2<LOG, AU, true>(f, kc, bl, t, row, t2, lds + g * kRowLds, ltw, g, groups, lds);
+    row_item2<LOG, AU, true, false>(f, kc, bl, t, row, t2, lds + g * kRowLds, ltw, g, groups, lds);
   } else {
     double* l = reinterpret_cast<double*>(lds);
-    row_item2<LOG, ArF64Lean, true>(f, kc, bl, t, row, t2, l + g * kRowLds, reinterpret_cast<double*>(ltw), g, groups, l);
+    row_item2<LOG, ArF64Lean, true, false>(f, kc, bl, t, row, t2, l + g * kRowLds, reinterpret_cast<double*>(ltw), g, groups, l);
   }
 }
 
@@ -840,7 +897,7 @@ __device__ __forceinline__ void top_inv(typename A::T (&v)[kColE<LOG>], const ty
 template <class A>
 __device__ __forceinline__ NttPrime product_prime(const KsRows& f, const KsConst& kc, int t) {
   NttPrime r = f.primes[t];
-  if constexpr (mont_keys<A>) {
+  if (mont_keys<A> && f.mont) {
     r.ninv = kc.ninv_r[t].w;
     r.ninv_q = kc.ninv_r[t].wq;
     r.last = kc.last_r[t].w;
@@ -1010,7 +1067,7 @@ void launch_cols_fwd(const KsRows& f, unsigned dnum, unsigned K, hipStream_t s) 
 // One chunk of ciphertexts through its launches, the integer-path primes on
 // policy AU.
 template <int LOG, class AU>
-void launch_chunk(const KsRows& f, const KsConst& kc, hipStream_t s, hipEvent_t* ev) {
+void launch_chunk(KsRows f, const KsConst& kc, hipStream_t s, hipEvent_t* ev) {
   const auto mark = [&](int i) {
     if (ev) (void)hipEventRecord(ev[i], s);
   };
@@ -1028,9 +1085,13 @@ void launch_chunk(const KsRows& f, const KsConst& kc, hipStream_t s, hipEvent_t*
   mark(0);
   const unsigned items = f.cts * K * rows;
   const unsigned groups = std::min(dnum, kRowGroupsMax / ((items + 255) / 256));
+  const bool sums = groups < 2 && !f.data_f64 && kc.pm_sums;
+  f.mont = !sums;
   if (groups >= 2)
     hipLaunchKernelGGL((ks_rows_split_kernel<LOG, AU>), dim3(items), dim3(kRow2Threads * groups),
                        groups * kRowLds * sizeof(uint64_t), s, f, t_u64);
+  else if (sums)
+    hipLaunchKernelGGL((ks_rows4_kernel<LOG>), dim3(items), dim3(256), 0, s, f);
   else
     hipLaunchKernelGGL((ks_rows2_kernel<LOG, AU>), dim3(items), dim3(kRow2Threads), 0, s, f, t_u64);
   mark(1);
@@ -1070,6 +1131,7 @@ hipError_t run_keyswitch_rows(const KsArgs& a, const KsConst* kc_dev, const KsCo
   f.tw_inv_f = d.tw_inv_f;
   f.ginv = a.galois_inv;
   f.data_f64 = 1;
+  f.mont = 1;
   f.moddown_f64 = 1;
   for (int i = 0; i < kc.L; ++i) {
     f.data_f64 &= kc.q[i] < (1ull << 50) ? 1 : 0;

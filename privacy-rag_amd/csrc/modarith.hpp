@@ -187,6 +187,19 @@ PH_HD uint64_t mul_pm(uint64_t a, uint64_t w, uint64_t v, uint32_t c2) {
 PH_HD uint64_t fold_pm(uint64_t x, uint32_t c1) {
   return uint64_t(uint32_t(x >> 32) >> 28) * c1 + (x & 0x0fffffffffffffffull);
 }
+// s0 + s1 2^30 + s2 2^60 mod q for sums of products of words split at 30 bits
+// (s1 + (s0 >> 30) and s2 + (s1 >> 30) without a carry out), for c' < 2^28:
+// s2 2^60 == s2 c', whose upper half u = (s2 >> 32) c' < 2^60 stands at 2^32 and
+// meets c' again with its part from 2^60 on.  Each of the four terms is below
+// 2^60 and the two products below 2^60 - 2^32: the result is below 2^62 - 2^33 < 4M.
+constexpr uint64_t kLow30 = (1ull << 30) - 1;
+PH_HD uint64_t sum_pm(uint64_t s0, uint64_t s1, uint64_t s2, uint32_t c1) {
+  s1 += s0 >> 30;
+  s2 += s1 >> 30;
+  const uint64_t u = uint64_t(uint32_t(s2 >> 32)) * c1;
+  return uint64_t(uint32_t(s2)) * c1 + uint64_t(uint32_t(u >> 28)) * c1 + (((s1 & kLow30) << 30) | (s0 & kLow30)) +
+         ((u & 0xfffffffull) << 32);
+}
 // Canonical residue of any x < 2^64: x mod 2^b + (x >> b) c < q + 2^32.
 PH_HD uint64_t canon_pm(uint64_t x, uint64_t q, uint32_t c, unsigned sh) {  // sh = b - 32
   const uint32_t hi = uint32_t(x >> 32);

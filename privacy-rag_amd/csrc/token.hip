@@ -45,7 +45,6 @@ static unsigned elem_grid(size_t items) {
 // ratio), Shoup products and canonical sums.
 constexpr int kMacCoords = 4;
 enum MacMode { kMacPm, kMacNarrow, kMacWide };
-constexpr uint64_t kMacLow = (1ull << 30) - 1;
 
 struct MacConst {
   uint64_t q, one_q, c60, c60_q;  // q, Shoup quotient of 1, c60 = 2^60 mod q with its quotient
@@ -56,17 +55,10 @@ struct MacConst {
 // s0 + s1 2^30 + s2 2^60 mod q as some word below 2^62.
 template <MacMode MODE>
 __device__ __forceinline__ uint64_t mac_fold(uint64_t s0, uint64_t s1, uint64_t s2, const MacConst& m) {
+  if constexpr (MODE == kMacPm) return sum_pm(s0, s1, s2, m.c);
   s1 += s0 >> 30;
   s2 += s1 >> 30;
-  const uint64_t low = ((s1 & kMacLow) << 30) | (s0 & kMacLow);
-  if constexpr (MODE == kMacPm) {
-    // s2 2^60 == s2 c; u = (s2 >> 32) c < 2^60 stands at 2^32: its part from
-    // 2^60 on, below 2^32, meets c again
-    const uint64_t u = uint64_t(uint32_t(s2 >> 32)) * m.c;
-    return uint64_t(uint32_t(s2)) * m.c + uint64_t(uint32_t(u >> 28)) * m.c + low + ((u & 0xfffffffull) << 32);
-  } else {
-    return mul_shoup_lazy(s2, m.c60, m.c60_q, m.q) + low;
-  }
+  return mul_shoup_lazy(s2, m.c60, m.c60_q, m.q) + (((s1 & kLow30) << 30) | (s0 & kLow30));
 }
 
 template <MacMode MODE, int KL>
@@ -130,9 +122,9 @@ __global__ void __launch_bounds__(256)
     for (unsigned b = 0; b < blocks; ++b) {
       uint32_t x0[KL], x1[KL], w0[kMacCoords], w1[kMacCoords];
 #pragma unroll
-      for (int k = 0; k < KL; ++k) x0[k] = uint32_t(xn[k]) & uint32_t(kMacLow), x1[k] = uint32_t(xn[k] >> 30);
+      for (int k = 0; k < KL; ++k) x0[k] = uint32_t(xn[k]) & uint32_t(kLow30), x1[k] = uint32_t(xn[k] >> 30);
 #pragma unroll
-      for (int c = 0; c < kMacCoords; ++c) w0[c] = uint32_t(wn[c]) & uint32_t(kMacLow), w1[c] = uint32_t(wn[c] >> 30);
+      for (int c = 0; c < kMacCoords; ++c) w0[c] = uint32_t(wn[c]) & uint32_t(kLow30), w1[c] = uint32_t(wn[c] >> 30);
       if (b + 1 < blocks) load(b + 1);
       if (b && b % 8 == 0) {
 #pragma unroll
@@ -143,10 +135,10 @@ __global__ void __launch_bounds__(256)
               // sixteen products of s2 and both carries of s1 stay below 2^64:
               // 16 (2^30 - 1)^2 + 2 (2^34 - 31) + 16 = 2^64 - 30
               s2[c][k] += s1[c][k] >> 30;
-              s1[c][k] &= kMacLow;
+              s1[c][k] &= kLow30;
             } else {  // below 2^62: s1 restarts below 2^32
               const uint64_t r = mac_fold<MODE>(s0[c][k], s1[c][k], s2[c][k], mc);
-              s0[c][k] = r & kMacLow;
+              s0[c][k] = r & kLow30;
               s1[c][k] = r >> 30;
               s2[c][k] = 0;
             }
