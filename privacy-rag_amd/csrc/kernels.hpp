@@ -28,6 +28,13 @@ struct NttDevice {
 };
 
 hipError_t launch_ntt(bool inverse, uint64_t* data, size_t limbs, const NttDevice& d, hipStream_t s);
+// Products of a batch of encryptions of zero in coefficient form (every prime on
+// ArPM): prod[e][c][t] = INTT(NTT(samples + e stride + t N) (.) pk[c][t]); pk in
+// ArPM's pairs (launch_pm_pairs), work [count][P][N].
+hipError_t launch_enc0_products(const uint64_t* samples, size_t stride, const ulonglong2* pk, uint64_t* work,
+                                uint64_t* prod, size_t count, const NttDevice& d, hipStream_t s);
+hipError_t launch_pm_pairs(const uint64_t* in, ulonglong2* out, size_t words, int log_n, const Barrett* m, int primes,
+                           hipStream_t s);
 // Inverse transform of [slots][2][P][N] with the token path's finish on the way
 // to out: scaled[slot][p] added to coefficient width - 1 of component 0, then
 // the limb times x^-(width-1).  data is used up.

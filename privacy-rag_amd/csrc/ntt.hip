@@ -429,6 +429,110 @@ hipError_t launch_ntt(bool inverse, uint64_t* data, size_t limbs, const NttDevic
   }
 }
 
+// Products of a batch of small polynomials u with both components of a
+// resident public key, in coefficient form (enc0.cu:99-114 before its ModDown):
+//   prod[e][c][t] = INTT(NTT(u[e][t]) (.) pk[c][t]),  u[e][t] at samples + e stride + t N.
+// One workgroup per (encryption, prime): the forward transform's registers are
+// the inverse transform's, position by position, so the product happens in
+// registers and the transform of u goes to memory only to be read again for the
+// second component (`work`, each thread its own words).  The key is held as
+// ArPM's pairs, and the forward values need no reduction before the product.
+// 64 encryptions at N = 16384, seven 60-bit primes, us: a copy of u, its
+// transform, the products and the inverse as launches of their own 211, 162 here.
+template <int LOGN>
+__global__ void __launch_bounds__(ntt_threads<LOGN>())
+    enc0_products_kernel(const uint64_t* __restrict__ samples, size_t stride, const ulonglong2* __restrict__ pk,
+                         uint64_t* __restrict__ work, uint64_t* __restrict__ prod, size_t count,
+                         const NttPrime* __restrict__ primes, const ulonglong2* __restrict__ tw_fwd,
+                         const ulonglong2* __restrict__ tw_inv, unsigned K) {
+  __shared__ __attribute__((aligned(16))) uint64_t lds[(1 << LOGN) + (1 << LOGN) / 16];
+  constexpr unsigned TH = ntt_threads<LOGN>();
+  for (size_t v = blockIdx.x; v < count * K; v += gridDim.x) {
+    const unsigned t = threadIdx.x + unsigned(v >> 40);  // recomputed per item: no index kept across the loop
+    const size_t e = v / K;
+    const unsigned p = unsigned(v % K);
+    const NttPrime pr = primes[p];
+    const ArPM ar(pr);
+    uint64_t x[kE];
+    const uint64_t* u = samples + e * stride + (size_t(p) << LOGN);
+#pragma unroll
+    for (int j = 0; j < kE; ++j) x[j] = u[fwd_in_index<LOGN>(t, j)];
+    ntt_regs<LOGN, false>(x, lds, t, tw_fwd + (size_t(p) << LOGN), ar, pr);
+    uint64_t* own = work + (v << LOGN) + t;
+#pragma unroll
+    for (int j = 0; j < kE; ++j) own[unsigned(j) * TH] = x[j];
+#pragma unroll 1
+    for (unsigned c = 0; c < 2; ++c) {
+      const unsigned t2 = t + unsigned((v + c) >> 40);
+      if (c) {
+#pragma unroll
+        for (int j = 0; j < kE; ++j) x[j] = own[unsigned(j) * TH];
+      }
+      const ulonglong2* k = pk + (size_t(c * K + p) << LOGN);
+#pragma unroll
+      for (int j = 0; j < kE; ++j) {
+        const ulonglong2 w = k[fwd_out_index<LOGN>(t2, j)];
+        x[j] = mul_pm(x[j], w.x, w.y, ar.c2);  // below 3M, the inverse's input bound is 4M
+        if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four pairs in registers at a time
+      }
+      // no barrier between the transforms: the forward one's last exchanges and
+      // the inverse one's first stay in the same wave's part of the LDS, and an
+      // exchange across waves begins and ends with one
+      ntt_regs<LOGN, true>(x, lds, t2, tw_inv + (size_t(p) << LOGN), ar, pr);
+      uint64_t* out = prod + (((e * 2 + c) * K + p) << LOGN);
+#pragma unroll
+      for (int j = 0; j < kE; ++j) out[inv_out_index<LOGN>(t2, j)] = ar.to_u64_inv(x[j]);
+    }
+  }
+}
+
+template <int LOGN>
+static hipError_t launch_enc0_products_n(const uint64_t* samples, size_t stride, const ulonglong2* pk, uint64_t* work,
+                                         uint64_t* prod, size_t count, const NttDevice& d, hipStream_t s) {
+  const unsigned grid = unsigned(std::min<size_t>(count * size_t(d.P), persistent_grid<LOGN, true, ArPM, false, false>()));
+  hipLaunchKernelGGL((enc0_products_kernel<LOGN>), dim3(grid), dim3(ntt_threads<LOGN>()), 0, s, samples, stride, pk,
+                     work, prod, count, d.primes, d.tw_fwd_u, d.tw_inv_u, unsigned(d.P));
+  return hipGetLastError();
+}
+
+hipError_t launch_enc0_products(const uint64_t* samples, size_t stride, const ulonglong2* pk, uint64_t* work,
+                                uint64_t* prod, size_t count, const NttDevice& d, hipStream_t s) {
+  if (count == 0) return hipSuccess;
+  switch (d.log_n) {
+    case 4: return launch_enc0_products_n<4>(samples, stride, pk, work, prod, count, d, s);
+    case 5: return launch_enc0_products_n<5>(samples, stride, pk, work, prod, count, d, s);
+    case 6: return launch_enc0_products_n<6>(samples, stride, pk, work, prod, count, d, s);
+    case 7: return launch_enc0_products_n<7>(samples, stride, pk, work, prod, count, d, s);
+    case 8: return launch_enc0_products_n<8>(samples, stride, pk, work, prod, count, d, s);
+    case 9: return launch_enc0_products_n<9>(samples, stride, pk, work, prod, count, d, s);
+    case 10: return launch_enc0_products_n<10>(samples, stride, pk, work, prod, count, d, s);
+    case 11: return launch_enc0_products_n<11>(samples, stride, pk, work, prod, count, d, s);
+    case 12: return launch_enc0_products_n<12>(samples, stride, pk, work, prod, count, d, s);
+    case 13: return launch_enc0_products_n<13>(samples, stride, pk, work, prod, count, d, s);
+    case 14: return launch_enc0_products_n<14>(samples, stride, pk, work, prod, count, d, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// ArPM's pairs of `words` residues [..][P][N] (a plan's resident key).
+__global__ void pm_pairs_kernel(const uint64_t* __restrict__ in, ulonglong2* __restrict__ out, BarrettList bl,
+                                int log_n, size_t words) {
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += size_t(gridDim.x) * blockDim.x) {
+    const uint64_t w = in[i];
+    out[i] = make_ulonglong2(pm_split(w), pm_split(mul_barrett(w, 1ull << 32, bl.m[(i >> log_n) % unsigned(bl.count)])));
+  }
+}
+
+hipError_t launch_pm_pairs(const uint64_t* in, ulonglong2* out, size_t words, int log_n, const Barrett* m, int primes,
+                           hipStream_t s) {
+  BarrettList bl{};
+  for (int i = 0; i < primes; ++i) bl.m[i] = m[i];
+  bl.count = primes;
+  const unsigned blocks = unsigned(std::min<size_t>((words + 255) / 256, 4096));
+  hipLaunchKernelGGL(pm_pairs_kernel, dim3(blocks), dim3(256), 0, s, in, out, bl, log_n, words);
+  return hipGetLastError();
+}
+
 // Pointwise product with a per-prime operand in Shoup form (client_dyadic,
 // ntt.cu:55-57): data[l][k] = data[l][k] * key[l % P][k] mod q.
 __global__ void dyadic_shoup_kernel(uint64_t* __restrict__ data, const ulonglong2* __restrict__ key,

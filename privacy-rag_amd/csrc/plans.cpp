@@ -277,6 +277,7 @@ struct praghip_enc0_plan {
   Enc0Const kc{};
   uint64_t *pk = nullptr, *samples = nullptr, *expanded = nullptr, *prod = nullptr, *out = nullptr;
   size_t batch_cap = 0;
+  ulonglong2* pk_pairs = nullptr;  // the key as ArPM's pairs (every prime on ArPM), with the batch's scratch
   uint64_t *bu = nullptr, *bprod = nullptr;  // [batch_cap][K][N] NTT(u), [batch_cap][2][K][N] products
   hipStream_t stream = nullptr;
   hipEvent_t ev[1] = {};
@@ -401,12 +402,21 @@ int praghip_enc0_reserve(praghip_enc0_plan* p, size_t count) {
   hipError_t e = scope.status();
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->bu, count * p->K * limb, true);
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->bprod, count * 2 * p->K * limb, true);
+  if (e == hipSuccess && p->d.pm_u64 && !p->d.n_f64) {
+    Barrett m[kMaxKeyPrimes];
+    for (size_t i = 0; i < p->K; ++i) m[i] = barrett_of(p->host_q[i]);
+    e = p->buf.alloc((void**)&p->pk_pairs, 4 * p->K * limb, true);
+    if (e == hipSuccess)
+      e = launch_pm_pairs(p->pk, p->pk_pairs, (2 * p->K) << p->log_n, int(p->log_n), m, int(p->K), p->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
+  }
   if (e != hipSuccess) return enc0_failure(p, e, "reserve");
   p->batch_cap = count;
   return PRAGHIP_OK;
 }
 
-// Many encryptions per call: every u transformed in one launch, the products
+// Many encryptions per call: with every prime on ArPM both transforms and the
+// key products in one launch, else every u transformed in one launch, the products
 // with both key components as one column-batched product (the public key is
 // the single resident block), one inverse transform, one noise-add + ModDown.
 int praghip_enc0_evaluate_device_batch(praghip_enc0_plan* p, const uint64_t* samples, uint64_t* output, size_t count,
@@ -424,6 +434,13 @@ int praghip_enc0_evaluate_device_batch(praghip_enc0_plan* p, const uint64_t* sam
   const hipStream_t s = pick(stream);
   DeviceScope scope(p->device);
   hipError_t e = scope.status();
+  if (p->pk_pairs) {
+    if (e == hipSuccess)
+      e = launch_enc0_products(samples, sample_words, p->pk_pairs, p->bu, p->bprod, count, p->d, s);
+    if (e == hipSuccess) e = launch_enc0_moddown(p->bprod, samples + K * n, output, p->kc, s, count, sample_words);
+    if (e != hipSuccess) return enc0_failure(p, e, "evaluate_device_batch");
+    return PRAGHIP_OK;
+  }
   // u of every encryption: rows of K N words, sample_words apart
   if (e == hipSuccess)
     e = hipMemcpy2DAsync(p->bu, K * n * 8, samples, sample_words * 8, K * n * 8, count, hipMemcpyDeviceToDevice, s);

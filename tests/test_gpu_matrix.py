@@ -247,3 +247,28 @@ def test_matrix_batch_largest_sums(gpu, primes, blocks, groups):
     for g in sorted({0, groups - 1}):
         np.testing.assert_array_equal(got[g], oracle.matrix_product(ct, rings[g], q, log_n), err_msg=f"group {g}")
     m.close()
+
+
+@pytest.mark.parametrize("log_n,count,L", [(4, 5, 2), (9, 3, 1), (11, 300, 3), (12, 7, 6), (13, 90, 6), (14, 1, 6),
+                                           (14, 41, 6)])
+def test_enc0_batch_integer_primes(gpu, log_n, count, L):
+    """The one-launch products (every prime just below a power of two) over
+    sizes and over counts on both sides of the resident workgroups, with the
+    largest key and sample words; exact."""
+    import torch
+    n = 1 << log_n
+    q = list(cf.LOCKED_PRIMES[:L]) + [cf.LOCKED_PRIMES[6]]
+    print(f"[enc0-integer] log_n={log_n} count={count} L={L}", flush=True)
+    pk = oracle.fill_residues(2 * (L + 1), n, q, 620).reshape(2, L + 1, n)
+    pk[0] = np.array(q, dtype=np.uint64)[:, None] - np.uint64(1)
+    z = praghip.PublicZero(q, log_n, pk)
+    z.reserve(count)
+    samples = oracle.fill_residues(count * 3 * (L + 1), n, q, 621).reshape(count, 3, L + 1, n)
+    samples[0, 0] = np.array(q, dtype=np.uint64)[:, None] - np.uint64(1)
+    out = to_dev(np.zeros((count, 2, L, n), dtype=np.uint64))
+    z.evaluate_device_batch(to_dev(samples), out)
+    torch.cuda.synchronize()
+    got = from_dev(out)
+    for e in sorted({0, count // 2, count - 1}):
+        np.testing.assert_array_equal(got[e], oracle.enc0(samples[e], pk, q, log_n), err_msg=f"oracle {e}")
+    z.close()
