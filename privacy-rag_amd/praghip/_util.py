@@ -1,7 +1,7 @@
 """Pointer and stream hand-off helpers (torch tensors and numpy arrays)."""
 from __future__ import annotations
 
-import ctypes
+import functools
 
 import numpy as np
 
@@ -35,10 +35,13 @@ def stream_handle(stream) -> int | None:
     """hipStream_t of a torch stream (None -> the caller's current stream)."""
     import torch
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream).value
+        # the current stream's handle without building a Stream object (2.7 us
+        # of the 10 that a small call took)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
+    return stream.cuda_stream or None
 
 
+@functools.lru_cache(maxsize=None)
 def u64_dtypes():
     import torch
     return (torch.int64, torch.uint64)
