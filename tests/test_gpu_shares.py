@@ -170,3 +170,16 @@ def test_share_storage_round_trip_and_clear(gpu):
         st.read(0, 1)
     with pytest.raises(praghip.PraghipError, match="E_CUDA_SHAPE"):
         ls.allocate(0)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 2048, 2049])
+@pytest.mark.parametrize("cols", [1, 64, 65, 255, 1023, 1024, 1025])
+def test_ring_sum_rows_wave_split(gpu, rows, cols):
+    """One wave or four per row: both sides of the rule and of a lane's group of
+    four loads; exact."""
+    print(f"[ring] sum_rows split {rows}x{cols}", flush=True)
+    a = oracle.fill_u64(rows * cols, 0x61 + cols).reshape(rows, cols)
+    a[0] = np.uint64(2**64 - 1)
+    np.testing.assert_array_equal(from_dev(praghip.ring_sum_rows(to_dev(a), cols)), oracle.ring_sum_rows(a, cols))
+    np.testing.assert_array_equal(from_dev(praghip.ring_sum_rows(to_dev(a), cols, mask_bits=64)),
+                                  a.sum(axis=1, dtype=np.uint64))
