@@ -81,6 +81,7 @@ struct KsArgs {
   unsigned* queue;       // scratch [kQueueWords], zero before the first launch (the kernel leaves it zero)
   uint64_t* inter = nullptr;  // scratch [inter_cts][dnum][K][N]: expanded digits of the three-phase path
   size_t inter_cts = 0;       // ciphertexts per three-phase chunk (0: whole-limb path only)
+  int accumulate = 0;         // three-phase path: add to out instead of passing component 0 of `in` on
   // four events recorded on the stream after the ModUp + forward columns, the
   // rows, the special prime's inverse columns and the ModDown columns (the
   // whole-limb path records the first at its start, the next two after its
@@ -156,7 +157,7 @@ hipError_t launch_token_mac(const uint64_t* in, const uint64_t* w, uint64_t* out
                             size_t limbs, int log_n, const Barrett* m, int primes, hipStream_t s);
 hipError_t launch_pack_prepare(const uint64_t* left, const uint64_t* right, uint64_t* sum, uint64_t* diff,
                                size_t count, size_t first, size_t group, size_t stride, const PrimeList& pl,
-                               int log_n, size_t shift, uint32_t ginv, hipStream_t s);
+                               int log_n, size_t shift, uint32_t ginv, bool merge, hipStream_t s);
 // Selective batch output: c0 of each group [groups][2][primes][2^log_n] zero
 // outside the `count` (<= kMaxTargets) sorted target coefficients idx[], and
 // the targets gathered into selected [groups][primes][count] (if non-null).

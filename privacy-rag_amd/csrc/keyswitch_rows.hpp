@@ -62,6 +62,7 @@ struct KsRows {
   int moddown_f64;  // every data prime in (2^32, 2^50): ModDown in FP64 too
   int narrow;       // every key prime below twice every other: x mod q_t by one subtraction
   unsigned big;     // digits of the larger size (the first ones)
+  int accumulate;   // ModDown adds to what out holds (both components) instead of component 0 of in
   int mont;         // the products lack the factor 2^64 of Montgomery key products
   unsigned b0, cts;  // chunk: ciphertexts b0 .. b0 + cts - 1
 };
@@ -961,8 +962,12 @@ __global__ void __launch_bounds__(256)
   const unsigned i = w % L, comp = (w / L) & 1u, b = f.b0 + w / (2 * L);
   const uint64_t* pc = f.prod + ((size_t(b) * 2 + comp) * K << LOG) + c;
   const uint64_t qi = kc.q[i];
-  const uint64_t* c0 = f.in + ((size_t(b) * 2 * L + i) << LOG);
   uint64_t* o = f.out + (((size_t(b) * 2 + comp) * L + i) << LOG) + c;
+  // what is added to the quotient: component 0 of the input (for component 0),
+  // or the output's own words
+  const bool addend = f.accumulate || comp == 0;
+  const uint64_t* c0 = f.accumulate ? o - c : f.in + ((size_t(b) * 2 * L + i) << LOG);
+  const uint32_t add_ginv = f.accumulate ? 1u : f.ginv;
   // [P_p + floor(p/2)]_p of this column
   uint64_t lastv[kColE<LOG>];
   const auto special = [&] {
@@ -992,8 +997,8 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
         for (int k = 0; k < kColE<LOG>; ++k) lastv[k] = pc[(size_t(L) << LOG) + (unsigned(k) << kRowLog)];
       }
-      if (comp == 0) {
-        gather_column<LOG>(c0v, c0, c, f.ginv, qi);
+      if (addend) {
+        gather_column<LOG>(c0v, c0, c, add_ginv, qi);
       } else {
 #pragma unroll
         for (int k = 0; k < kColE<LOG>; ++k) c0v[k] = 0;
@@ -1017,12 +1022,12 @@ __global__ void __launch_bounds__(256)
   uint64_t x[kColE<LOG>], c0v[kColE<LOG>];
   if constexpr (SELF) {
     // registers to spare: c0's loads in flight during the two transforms
-    if (comp == 0) gather_column<LOG>(c0v, c0, c, f.ginv, qi);
+    if (addend) gather_column<LOG>(c0v, c0, c, add_ginv, qi);
     special();
   }
   column_residues<LOG, A>(x, pc + (size_t(i) << LOG), inv_table<LOG, A>(f, int(i)), product_prime<A>(f, kc, int(i)));
   if constexpr (!SELF) {
-    if (comp == 0) gather_column<LOG>(c0v, c0, c, f.ginv, qi);
+    if (addend) gather_column<LOG>(c0v, c0, c, add_ginv, qi);
   }
 #pragma unroll
   for (int k = 0; k < kColE<LOG>; ++k) {
@@ -1030,7 +1035,7 @@ __global__ void __launch_bounds__(256)
     const uint64_t reduced = reduce_to(last, kc, int(i), f.narrow);  // last mod q_i
     const uint64_t corr = sub_mod(reduced, kc.half_mod[i], qi);
     uint64_t val = mul_shoup(sub_mod(x[k], corr, qi), kc.invp[i].w, kc.invp[i].wq, qi);
-    if (comp == 0) val = add_mod(val, c0v[k], qi);
+    if (addend) val = add_mod(val, c0v[k], qi);
     __builtin_nontemporal_store(val, &o[unsigned(k) << kRowLog]);
   }
 }
@@ -1132,6 +1137,7 @@ hipError_t run_keyswitch_rows(const KsArgs& a, const KsConst* kc_dev, const KsCo
   f.ginv = a.galois_inv;
   f.data_f64 = 1;
   f.mont = 1;
+  f.accumulate = a.accumulate;
   f.moddown_f64 = 1;
   for (int i = 0; i < kc.L; ++i) {
     f.data_f64 &= kc.q[i] < (1ull << 50) ? 1 : 0;

@@ -231,6 +231,9 @@ hipError_t launch_token_mac(const uint64_t* in, const uint64_t* w, uint64_t* out
 // outputs are written in coefficient order: diff at d takes the source
 // coefficient u = d g^-1 mod 2N (negated when u >= N), gathered from inside
 // the same limb, so no write is scattered.
+// MERGE: the switched halves of a pair are added, and so are their components 0,
+// which the switches only pass on: component 0 of sum takes both and that of
+// diff is not written (a quarter of the writes less, and of the switches' reads).
 __device__ __forceinline__ uint64_t shifted_diff(const uint64_t* __restrict__ l, const uint64_t* __restrict__ r,
                                                  size_t j, size_t n, size_t shift, uint64_t q, uint64_t& sum) {
   uint64_t v = r[(j + n - shift) & (n - 1)];
@@ -240,6 +243,7 @@ __device__ __forceinline__ uint64_t shifted_diff(const uint64_t* __restrict__ l,
   return sub_mod(a, v, q);
 }
 
+template <bool MERGE>
 __global__ void __launch_bounds__(256)
     pack_prepare_kernel(const uint64_t* __restrict__ left, const uint64_t* __restrict__ right,
                         uint64_t* __restrict__ sum, uint64_t* __restrict__ diff, size_t count, size_t first,
@@ -254,20 +258,30 @@ __global__ void __launch_bounds__(256)
     const uint64_t* r = right + src;
     uint64_t s0;
     (void)shifted_diff(l, r, d, n, shift, q, s0);
-    sum[i * ct + w] = s0;
+    if constexpr (!MERGE) sum[i * ct + w] = s0;
     const size_t u = (d * size_t(ginv)) & (2 * n - 1);
     uint64_t unused;
     const uint64_t delta = shifted_diff(l, r, u & (n - 1), n, shift, q, unused);
-    diff[i * ct + w] = (u >= n && delta) ? q - delta : delta;
+    const uint64_t mapped = (u >= n && delta) ? q - delta : delta;
+    if constexpr (MERGE) {
+      const bool first_half = w < ct / 2;  // component 0
+      sum[i * ct + w] = first_half ? add_mod(s0, mapped, q) : s0;
+      if (!first_half) diff[i * ct + w] = mapped;
+    } else {
+      diff[i * ct + w] = mapped;
+    }
   }
 }
 
 hipError_t launch_pack_prepare(const uint64_t* left, const uint64_t* right, uint64_t* sum, uint64_t* diff,
                                size_t count, size_t first, size_t group, size_t stride, const PrimeList& pl,
-                               int log_n, size_t shift, uint32_t ginv, hipStream_t s) {
+                               int log_n, size_t shift, uint32_t ginv, bool merge, hipStream_t s) {
   const size_t total = count * 2 * size_t(pl.count) << log_n;
-  hipLaunchKernelGGL(pack_prepare_kernel, dim3(elem_grid(total)), dim3(256), 0, s, left, right, sum, diff, count,
-                     first, group, stride, pl, log_n, shift, ginv);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(elem_grid(total)), dim3(256), 0, s, left, right, sum, diff, count, first, group,
+                       stride, pl, log_n, shift, ginv);
+  };
+  merge ? go(pack_prepare_kernel<true>) : go(pack_prepare_kernel<false>);
   return hipGetLastError();
 }
 

@@ -407,3 +407,35 @@ def test_token_half_limb_lift(gpu, primes, width, blocks):
     got = from_dev(out)
     for c in range(coords):
         np.testing.assert_array_equal(got[c], oracle.token_finished(ct, rings[c], scaled[c], q, log_n, width))
+
+
+@pytest.mark.parametrize("primes,dnum", [("locked", 2), ("50bit", 1), ("offpower", 2)])
+@pytest.mark.parametrize("count,max_pairs", [(31, 64), (32, 64), (33, 64), (97, 64), (70, 40)])
+def test_pack_pairs_merged(gpu, primes, dnum, count, max_pairs):
+    """Pairs on both sides of the merged form (sums switched into the output,
+    differences added to it), over chunks; equal to the pairs one by one, and
+    the tree in place over the same leaves."""
+    import torch
+    print(f"[pack-merged] {primes} count={count} max_pairs={max_pairs}", flush=True)
+    log_n, n, L, levels = 12, 1 << 12, 2, 7
+    q = {"locked": list(cf.LOCKED_PRIMES[:2]), "50bit": cf.primes_below(50, n, 2),
+         "offpower": [v for v in range((3 << 57) + 1, (3 << 57) + 400 * 2 * n, 2 * n) if cf.is_prime(v)][:2]}[primes]
+    q = q + [cf.LOCKED_PRIMES[6]]
+    keys = _pack_keys(q, n, dnum, levels, 770)
+    pk = praghip.Packing(q, log_n, keys, dnum=dnum, max_pairs=max_pairs)
+    lr = oracle.fill_residues(2 * count * 2 * L, n, q[:L], 771).reshape(2, count, 2, L, n)
+    lr[:, 0] = np.array(q[:L], dtype=np.uint64)[None, :, None] - np.uint64(1)
+    left, right = to_dev(lr[0]), to_dev(lr[1])
+    got = pk.pair_device(left, right, 1)
+    torch.cuda.synchronize()
+    got = from_dev(got).reshape(count, 2, L, n)
+    for i in range(count):
+        one = pk.pair_device(left[i].contiguous(), right[i].contiguous(), 1)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(got[i], from_dev(one).reshape(2, L, n), err_msg=f"pair {i}")
+    if count == 32:  # 64 leaves: the first level is merged, in place
+        lv = lr.reshape(64, 1, 2, L, n)
+        roots = pk.tree_device(to_dev(lv), slots=1)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(from_dev(roots).reshape(1, 2, L, n), oracle.pack_tree(lv, keys, q, dnum, log_n))
+    pk.close()
