@@ -183,6 +183,64 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
   }
 }
 
+// Few limbs (no more than CUs): one workgroup per limb on twice the threads of
+// ntt_kernel, eight coefficients each.  A limb alone on its CU is bound by
+// latency: with sixteen coefficients per thread a SIMD holds one wave at
+// N = 4096, which issues a multiply-add every 8.8 cycles; two waves issue one
+// every 4.4, and the next pass's twiddles are on their way during a pass.
+// 32 limbs at N = 4096, forward and inverse: 15.9 -> 12.6 us.  Not at N = 8192, whose
+// sixteen waves would name coefficient bits that the second pass needs.
+constexpr int kFewLE = 3;
+template <int LOGN, bool INV, class A>
+__global__ void __launch_bounds__((ntt_threads<LOGN, kFewLE>()))
+    ntt_few_kernel(uint64_t* __restrict__ data, size_t count, const NttPrime* __restrict__ primes,
+                   const typename A::TW* __restrict__ tw, int P, const int* __restrict__ sel, int C) {
+  constexpr int E = 1 << kFewLE;
+  // the second pass's gap bits end where the wave bits begin
+  static_assert(LOGN - kFewLE <= LOGN - Passes<LOGN, kFewLE>::WAVE_BITS);
+  __shared__ __attribute__((aligned(16))) uint64_t lds[(1 << LOGN) + (1 << LOGN) / 16];
+  using T = typename A::T;
+  const unsigned t = threadIdx.x, v = blockIdx.x;
+  if (v >= count) return;
+  const size_t limb = size_t(v / unsigned(C)) * unsigned(P) + unsigned(sel[v % unsigned(C)]);
+  const int p = int(limb % unsigned(P));
+  const typename A::TW* tab = tw + (size_t(p) << LOGN);
+  uint64_t* d = data + (limb << LOGN);
+  uint64_t raw[E];
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    raw[j] = d[INV ? inv_in_index<LOGN, kFewLE>(t, j) : fwd_in_index<LOGN, kFewLE>(t, j)];
+  typename A::TW w0[(pass_tw_count<LOGN, INV, 0, kFewLE>())];
+  load_pass_twiddles_e<LOGN, INV, 0, kFewLE>(w0, t, tab);
+  const NttPrime pr = primes[p];
+  const A ar(pr);
+  T x[E];
+#pragma unroll
+  for (int j = 0; j < E; ++j) x[j] = ar.from_u64(raw[j]);
+  run_passes_wide<LOGN, INV, 0>(x, reinterpret_cast<T*>(lds), t, tab, ar, pr, w0);
+  if constexpr (!INV) {
+#pragma unroll
+    for (int j = 0; j < E; j += 2)
+      *reinterpret_cast<ulonglong2*>(d + fwd_out_index<LOGN, kFewLE>(t, j)) =
+          make_ulonglong2(ar.to_u64_fwd(x[j]), ar.to_u64_fwd(x[j + 1]));
+  } else {
+#pragma unroll
+    for (int j = 0; j < E; ++j) d[inv_out_index<LOGN, kFewLE>(t, j)] = ar.to_u64_inv(x[j]);
+  }
+}
+
+static unsigned device_cus() {
+  static unsigned cached = 0;
+  if (!cached) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+      cus = 256;
+    cached = unsigned(cus);
+  }
+  return cached;
+}
+
 // Resident workgroups per CU times the CU count, cached per kernel.
 template <int LOGN, bool INV, class A, bool LIFT, bool FINISH>
 static unsigned persistent_grid() {
@@ -217,6 +275,13 @@ static hipError_t launch_subset(uint64_t* data, size_t limbs, const NttDevice& d
   if (!C) return hipSuccess;
   const size_t count = subset_count(limbs, d.P, sel_host, C);
   if (!count) return hipSuccess;
+  if constexpr (!LIFT && !FINISH && LOGN >= 10 && LOGN <= 12) {
+    if (count <= device_cus()) {
+      hipLaunchKernelGGL((ntt_few_kernel<LOGN, INV, A>), dim3(unsigned(count)), dim3(ntt_threads<LOGN, kFewLE>()), 0, s,
+                         data, count, d.primes, tw, d.P, sel_dev, C);
+      return hipGetLastError();
+    }
+  }
   const dim3 block{unsigned(ntt_threads<LOGN>())};
   const dim3 grid{unsigned(std::min<size_t>(count, persistent_grid<LOGN, INV, A, LIFT, FINISH>()))};
   hipLaunchKernelGGL((ntt_kernel<LOGN, INV, A, LIFT, FINISH>), grid, block, 0, s, data, count, d.primes, tw, d.P,
@@ -315,14 +380,7 @@ __global__ void __launch_bounds__(1 << (kHalfLog - kLogE)) __attribute__((amdgpu
 
 template <class A, HalfInput IN>
 static hipError_t launch_lift_half(uint64_t* out, size_t blocks, const NttDevice& d, NttLift lift, hipStream_t s) {
-  static unsigned resident = 0;
-  if (!resident) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
-    resident = unsigned(cus + 7) / 8 * 8 * 2;
-  }
+  const unsigned resident = (device_cus() + 7) / 8 * 8 * 2;
   const size_t total = (blocks + 7) / 8 * 8 * 2 * size_t(d.n_u64);
   hipLaunchKernelGGL((ntt_lift_half_kernel<A, IN>), dim3(unsigned(std::min<size_t>(total, resident))),
                      dim3(1 << (kHalfLog - kLogE)), 0, s, out, blocks, d.primes, d.tw_fwd_u, d.P, d.sel_u64, d.n_u64,
@@ -439,7 +497,10 @@ hipError_t launch_ntt(bool inverse, uint64_t* data, size_t limbs, const NttDevic
 // ArPM's pairs, and the forward values need no reduction before the product.
 // 64 encryptions at N = 16384, seven 60-bit primes, us: a copy of u, its
 // transform, the products and the inverse as launches of their own 211, 162 here.
-template <int LOGN>
+// SPLIT: a workgroup per component as well, each transforming u for itself - two
+// transforms in series instead of three, while even that leaves CUs idle (two
+// encryptions, us: launches of their own 61, three in series 64, SPLIT 43).
+template <int LOGN, bool SPLIT>
 __global__ void __launch_bounds__(ntt_threads<LOGN>())
     enc0_products_kernel(const uint64_t* __restrict__ samples, size_t stride, const ulonglong2* __restrict__ pk,
                          uint64_t* __restrict__ work, uint64_t* __restrict__ prod, size_t count,
@@ -447,9 +508,9 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
                          const ulonglong2* __restrict__ tw_inv, unsigned K) {
   __shared__ __attribute__((aligned(16))) uint64_t lds[(1 << LOGN) + (1 << LOGN) / 16];
   constexpr unsigned TH = ntt_threads<LOGN>();
-  for (size_t v = blockIdx.x; v < count * K; v += gridDim.x) {
-    const unsigned t = threadIdx.x + unsigned(v >> 40);  // recomputed per item: no index kept across the loop
-    const size_t e = v / K;
+  for (size_t i = blockIdx.x; i < (SPLIT ? 2 : 1) * count * K; i += gridDim.x) {
+    const unsigned t = threadIdx.x + unsigned(i >> 40);  // recomputed per item: no index kept across the loop
+    const size_t v = SPLIT ? i / 2 : i, e = v / K;
     const unsigned p = unsigned(v % K);
     const NttPrime pr = primes[p];
     const ArPM ar(pr);
@@ -459,12 +520,15 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
     for (int j = 0; j < kE; ++j) x[j] = u[fwd_in_index<LOGN>(t, j)];
     ntt_regs<LOGN, false>(x, lds, t, tw_fwd + (size_t(p) << LOGN), ar, pr);
     uint64_t* own = work + (v << LOGN) + t;
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int j = 0; j < kE; ++j) own[unsigned(j) * TH] = x[j];
+      for (int j = 0; j < kE; ++j) own[unsigned(j) * TH] = x[j];
+    }
+    const unsigned c_first = SPLIT ? unsigned(i & 1) : 0u, c_end = SPLIT ? c_first + 1 : 2u;
 #pragma unroll 1
-    for (unsigned c = 0; c < 2; ++c) {
+    for (unsigned c = c_first; c < c_end; ++c) {
       const unsigned t2 = t + unsigned((v + c) >> 40);
-      if (c) {
+      if (!SPLIT && c) {
 #pragma unroll
         for (int j = 0; j < kE; ++j) x[j] = own[unsigned(j) * TH];
       }
@@ -489,9 +553,15 @@ __global__ void __launch_bounds__(ntt_threads<LOGN>())
 template <int LOGN>
 static hipError_t launch_enc0_products_n(const uint64_t* samples, size_t stride, const ulonglong2* pk, uint64_t* work,
                                          uint64_t* prod, size_t count, const NttDevice& d, hipStream_t s) {
-  const unsigned grid = unsigned(std::min<size_t>(count * size_t(d.P), persistent_grid<LOGN, true, ArPM, false, false>()));
-  hipLaunchKernelGGL((enc0_products_kernel<LOGN>), dim3(grid), dim3(ntt_threads<LOGN>()), 0, s, samples, stride, pk,
-                     work, prod, count, d.primes, d.tw_fwd_u, d.tw_inv_u, unsigned(d.P));
+  const size_t items = count * size_t(d.P);
+  const bool split = 2 * items <= device_cus();
+  const unsigned grid =
+      unsigned(std::min<size_t>((split ? 2 : 1) * items, persistent_grid<LOGN, true, ArPM, false, false>()));
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(ntt_threads<LOGN>()), 0, s, samples, stride, pk, work, prod, count,
+                       d.primes, d.tw_fwd_u, d.tw_inv_u, unsigned(d.P));
+  };
+  split ? go(enc0_products_kernel<LOGN, true>) : go(enc0_products_kernel<LOGN, false>);
   return hipGetLastError();
 }
 

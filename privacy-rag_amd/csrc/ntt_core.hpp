@@ -639,6 +639,33 @@ __device__ __forceinline__ void run_part_passes(typename A::T (&v)[kE], typename
   }
 }
 
+// Passes P .. NP - 1 of a limb on 2^LE coefficients per thread, the twiddles of a
+// pass loaded before the pass in front of it.
+template <int LOGN, bool INV, int P, class A, int E>
+__device__ __forceinline__ void run_passes_wide(
+    typename A::T (&v)[E], typename A::T* lds, unsigned t, const typename A::TW* __restrict__ tab, const A& ar,
+    const NttPrime& pr, const typename A::TW (&w)[(pass_tw_count<LOGN, INV, P, ilog2(E)>())]) {
+  constexpr int LE = ilog2(E);
+  using S = Passes<LOGN, LE>;
+  constexpr int LO = S::lo(INV, P), R = S::r(INV, P);
+  constexpr bool UNI = PassMap<LOGN, INV, P, LE>::uniform_groups();
+  const auto pass = [&] {
+    if constexpr (INV)
+      inv_pass<LOGN, LO, R, UNI>(v, w, ar, pr, [] {});
+    else
+      fwd_pass<LOGN, LO, R, UNI>(v, w, ar, [] {});
+  };
+  if constexpr (P + 1 < S::NP) {
+    typename A::TW wn[(pass_tw_count<LOGN, INV, P + 1, LE>())];
+    load_pass_twiddles_e<LOGN, INV, P + 1, LE>(wn, t, tab);
+    pass();
+    exchange<LOGN, INV, P>(v, lds, t);
+    run_passes_wide<LOGN, INV, P + 1>(v, lds, t, tab, ar, pr, wn);
+  } else {
+    pass();
+  }
+}
+
 // Whole-limb transform on register data (v holds the input layout on entry
 // and the output layout on exit; values stay in the policy's lazy form).
 template <int LOGN, bool INV, class A, class F>

@@ -239,3 +239,13 @@ def test_ntt_integer_prime_forms(gpu, log_n, bits):
         top = (3 << 57) // (2 * n) * 2 * n + 1
         q = [v for v in range(top - 600 * 2 * n, top, 2 * n) if cf.is_prime(v)][-2:]
     _roundtrip_case(q, log_n, 7, 0x98 + log_n, gpu)
+
+
+@pytest.mark.parametrize("log_n", [9, 10, 11, 12, 13])
+@pytest.mark.parametrize("bits,limbs", [(50, 1), (50, 255), (54, 3), (60, 256), (60, 257), (62, 5), (0, 2)])
+def test_ntt_few_limbs(gpu, log_n, bits, limbs):
+    """One workgroup per limb on eight coefficients per thread: both sides of
+    the limb count it ends at, its sizes and the neighbours', each arithmetic."""
+    n = 1 << log_n
+    q = cf.primes_below(bits, n, 3) if bits else cf.primes_below(50, n, 1) + cf.primes_below(60, n, 1)
+    _roundtrip_case(q, log_n, limbs, 0xa0 + limbs, gpu)
