@@ -1055,12 +1055,20 @@ constexpr unsigned kSpreadBlocks() {
 // itself up to this many workgroups (batch 1, 48: 40.9 / 47.6 us; batch 16, 768:
 // 143 / 150; batch 32, 1536: 253 / 257 and, 50-bit primes, 153.6 / 152.8).
 constexpr unsigned kSelfBlocks = 1024;
+// Threads of a column workgroup of these small launches: one wave, spread over
+// the CUs, while the inverse columns as workgroups of four would leave half of
+// them without one (`c_blocks`: the latter's count).  us, 64 / 256 threads: six
+// one-prime digits, N = 16384, batch 1 (48) 36.0 / 37.6, 2 (96) 41.4 / 42.7, 4 (192)
+// 62.6 / 58.7; three two-prime digits of 50-bit primes, batch 1 29.2 / 30.7, 4 47.3 /
+// 46.7.
+inline unsigned column_threads(unsigned c_blocks) { return c_blocks <= 128 ? 64 : 256; }
 
 template <int LOG, int D, bool MIX, class AU>
 void launch_cols_fwd(const KsRows& f, unsigned dnum, unsigned K, hipStream_t s) {
   const unsigned blocks = f.cts * dnum * kCols / 256;  // (ciphertext, digit, 256 columns)
   if (blocks <= kSpreadBlocks<D, MIX>()) {
-    hipLaunchKernelGGL((ks_cols_fwd_spread<LOG, D, MIX, AU>), dim3(blocks * K), dim3(256), 0, s, f);
+    const unsigned th = column_threads(f.cts * 2 * (K - 1) * kCols / 256);
+    hipLaunchKernelGGL((ks_cols_fwd_spread<LOG, D, MIX, AU>), dim3(blocks * K * (256 / th)), dim3(th), 0, s, f);
   } else if (!f.data_f64) {  // every prime on the integer path
     constexpr unsigned G = (D == 1 && !MIX) ? kColTargets<ArU64, 1>() : 1u;
     hipLaunchKernelGGL((ks_cols_fwd_kernel<LOG, D, MIX, AU, G>), dim3(blocks * ((K + G - 1) / G)), dim3(256), 0, s, f);
@@ -1105,7 +1113,10 @@ void launch_chunk(KsRows f, const KsConst& kc, hipStream_t s, hipEvent_t* ev) {
   if (!self)
     hipLaunchKernelGGL((ks_cols_special_kernel<LOG, AU>), dim3(f.cts * 2 * kCols / 256), dim3(256), 0, s, f);
   mark(2);
-  const auto inv = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(c_blocks), dim3(256), 0, s, f); };
+  const auto inv = [&](auto kernel) {
+    const unsigned th = self ? column_threads(c_blocks) : 256;
+    hipLaunchKernelGGL(kernel, dim3(c_blocks * (256 / th)), dim3(th), 0, s, f);
+  };
   if (f.data_f64)
     self ? inv(ks_cols_inv_kernel<LOG, ArF64, AU, true>) : inv(ks_cols_inv_kernel<LOG, ArF64, AU, false>);
   else
