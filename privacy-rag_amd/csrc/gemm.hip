@@ -1023,7 +1023,7 @@ constexpr size_t kFewBytes = size_t(128) << 20;
 static int few_rb(int w_bits, int M) { return M <= 4 ? 1 : (M <= 8 || w_bits != 8) ? 2 : 4; }
 static size_t few_bytes(int w_bits, int M, int K, int N) {
   const size_t rb = size_t(few_rb(w_bits, M)), wgs = (size_t(M) + 4 * rb - 1) / (4 * rb) * ((size_t(N) + 31) / 32);
-  return wgs * size_t(K) * 32 * (rb + (w_bits == 8 ? 1 : w_bits == 24 ? 3 : 4));
+  return wgs * size_t(std::max(K, kFewWaves * kFewChunk)) * 32 * (rb + (w_bits == 8 ? 1 : w_bits == 24 ? 3 : 4));
 }
 
 // Which kernel a product takes, and how its K is split.
