@@ -1020,6 +1020,9 @@ __global__ void __launch_bounds__(256) gemm_clear_list_kernel(GemmClearList l) {
 // planes: 64x3072x1024 15.3 / 18.2 (126 MB), 77x3072x1024 28.2 / 21.2 (157 MB);
 // int32: 13x1024x3001 12.7 / 18.7 (37 MB), 13x3072x4096 32.9 / 29.5 (151 MB).
 constexpr size_t kFewBytes = size_t(128) << 20;
+// K counts as at least the eight waves' 1024 words: below it some of them have no
+// chunk.  us, few-row / tiles: int8 486x90x1131 27.8 / 9.3, 200x130x4000 34.2 / 9.4,
+// 700x500x700 24.2 / 12.6; int32 486x90x1131 61.2 / 24.8, 40x700x5000 46.0 / 24.4.
 static int few_rb(int w_bits, int M) { return M <= 4 ? 1 : (M <= 8 || w_bits != 8) ? 2 : 4; }
 static size_t few_bytes(int w_bits, int M, int K, int N) {
   const size_t rb = size_t(few_rb(w_bits, M)), wgs = (size_t(M) + 4 * rb - 1) / (4 * rb) * ((size_t(N) + 31) / 32);
