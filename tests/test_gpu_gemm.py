@@ -273,3 +273,31 @@ def test_gemm_batch_forms(gpu):
         torch.cuda.synchronize()
         for i, (_, _, _, y) in enumerate(keep):
             np.testing.assert_array_equal(from_dev(y), want[i], err_msg=f"product {i} {rows[i]}")
+
+
+@pytest.mark.parametrize("m,n", [(3, 40), (512, 512), (1024, 2048)])
+@pytest.mark.parametrize("bits", [8, 24, 32])
+def test_gemm_empty_sum(gpu, m, n, bits):
+    """K = 0 through the C ABI: y is zeroed, alone and in a batch beside a
+    product with terms, whatever the output's size."""
+    import ctypes
+
+    import torch
+    from praghip._lib import GemmDesc, check, lib
+    print(f"[gemm] k=0 m={m} n={n} bits={bits}", flush=True)
+    x = torch.ones(16, dtype=torch.int64, device="cuda")
+    w = torch.ones(16, dtype=torch.int32, device="cuda")
+    y = torch.full((m, n), -1, dtype=torch.int64, device="cuda")
+    check(lib().praghip_share_gemm(0, x.data_ptr(), w.data_ptr(), bits, None, y.data_ptr(), m, 0, n, 59, None))
+    torch.cuda.synchronize()
+    assert not y.any()
+    x1, w1 = oracle.fill_u64(600 * 128, 18000).reshape(600, 128), oracle.fill_i8(1000 * 128, 18001).reshape(1000, 128)
+    tx, tw = to_dev(x1), torch.from_numpy(w1).cuda()
+    y.fill_(-1)
+    y1 = torch.full((600, 1000), -1, dtype=torch.int64, device="cuda")
+    arr = (GemmDesc * 2)(GemmDesc(x.data_ptr(), w.data_ptr(), 0, y.data_ptr(), m, 0, n, bits, 64),
+                         GemmDesc(tx.data_ptr(), tw.data_ptr(), 0, y1.data_ptr(), 600, 128, 1000, 8, 64))
+    check(lib().praghip_share_gemm_batch(0, ctypes.cast(arr, ctypes.c_void_p), 2, None))
+    torch.cuda.synchronize()
+    assert not y.any()
+    np.testing.assert_array_equal(from_dev(y1), oracle.share_gemm(x1, w1))
