@@ -453,16 +453,14 @@ __device__ __forceinline__ void tile_of(int& tm, int& tn, int TN, int TM, int t)
   tn = in / rows;
 }
 
-// Epilogue of one accumulator tile of a wave: rows row0 .. row0 + 3 (this lane
-// writes rows row0 + 2 khalf and row0 + 2 khalf + 1), column col.  The lane
-// holds, for its column, digits 4 khalf .. 4 khalf + 3 of the four rows in
-// register groups g (rows row0 + g); the halves of the wave add their digit
+// Digit sums of one accumulator tile of a wave: rows r0 .. r0 + 3, of which this
+// lane takes r0 + 2 khalf (sum[0]) and r0 + 2 khalf + 1 (sum[1]) of its column.
+// The lane holds, for its column, digits 4 khalf .. 4 khalf + 3 of the four rows
+// in register groups g (rows r0 + g); the halves of the wave add their digit
 // sums with v_permlane32_swap: swapping lanes 32-63 of part[g] with lanes 0-31
 // of part[g + 2] leaves every lane with its own half's value and the other
-// half's for the row it writes, one in each register.  corr is the
-// offset-binary correction of the column, sh its shift.
-__device__ __forceinline__ void store_tile(const v16i& a, int row0, int col, int khalf, uint64_t corr, int sh,
-                                           bool split, uint64_t mask, uint64_t* __restrict__ y, int M, int N) {
+// half's for the row it takes, one in each register.
+__device__ __forceinline__ void tile_sums(const v16i& a, int khalf, uint64_t (&sum)[2]) {
   uint64_t part[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -470,13 +468,20 @@ __device__ __forceinline__ void store_tile(const v16i& a, int row0, int col, int
     const int64_t v = mad_i64(a[4 * g + 3], 16777216, mad_i64(a[4 * g + 2], 65536, mad_i64(a[4 * g + 1], 256, int64_t(a[4 * g]))));
     part[g] = uint64_t(v) << (32 * khalf);
   }
-  uint64_t sum[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const auto lo = __builtin_amdgcn_permlane32_swap(uint32_t(part[h]), uint32_t(part[h + 2]), false, false);
     const auto hi = __builtin_amdgcn_permlane32_swap(uint32_t(part[h] >> 32), uint32_t(part[h + 2] >> 32), false, false);
     sum[h] = ((uint64_t(hi[0]) << 32) | lo[0]) + ((uint64_t(hi[1]) << 32) | lo[1]);
   }
+}
+
+// Epilogue of one accumulator tile of a wave: rows row0 .. row0 + 3, column col;
+// corr is the offset-binary correction of the column, sh its shift.
+__device__ __forceinline__ void store_tile(const v16i& a, int row0, int col, int khalf, uint64_t corr, int sh,
+                                           bool split, uint64_t mask, uint64_t* __restrict__ y, int M, int N) {
+  uint64_t sum[2];
+  tile_sums(a, khalf, sum);
   if (col >= N) return;  // the same for lanes l and l ^ 32
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -734,6 +739,12 @@ __device__ __forceinline__ uint4 load_w4(const int32_t* row, int k, int K) {
 // written to the other of two LDS stages, in the DMA path's swizzled layout;
 // the MFMA part is the same.  One barrier per step: a stage is rewritten two
 // steps after it was read.  Workgroup z as in the DMA kernel.
+//
+// FUSED: the workgroup takes the three planes one after the other and keeps the
+// outputs' sums in registers, so that y is written once: no clear, no atomics and
+// no mask pass, which move y nine times.  They are the cost where K is short:
+// three planes 1000x16x3072 71 -> 24 us, int32 78 -> 34.  Each step's words are
+// loaded as it starts (the sums take the registers that the next step's would).
 template <int WT>
 struct RegTile {
   uint4 x[4], w[WT == kW32 ? 8 : 2];
@@ -763,7 +774,7 @@ __device__ __forceinline__ uint32_t digit4(uint4 w, uint32_t sel) {
   return __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ 0x80808080u;
 }
 
-template <int WT>
+template <int WT, bool FUSED = false>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
     share_gemm_reg_kernel(const uint64_t* __restrict__ x, const void* __restrict__ wv,
                           const int8_t* __restrict__ shifts, uint64_t* __restrict__ y, int M, int K, int N,
@@ -771,7 +782,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   constexpr int CB = 2;
   __shared__ __attribute__((aligned(16))) uint8_t raw[2][kBM * kRawRow];
   __shared__ __attribute__((aligned(16))) uint8_t wt[2][kBN * kBK];
-  const int plane = int(blockIdx.z) / splits, k_begin = (int(blockIdx.z) % splits) * k_split;
+  const int first = FUSED ? 0 : int(blockIdx.z) / splits, k_begin = (int(blockIdx.z) % splits) * k_split;
   const int k_end = min(k_begin + k_split, K);
   int tm, tn;
   tile_of(tm, tn, int(gridDim.x), int(gridDim.y), int(blockIdx.y * gridDim.x + blockIdx.x));
@@ -793,48 +804,94 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const int row = 16 * (2 * c.wave + j) + (lane >> 2);
     const size_t off = size_t(min(n0 + row, N - 1)) * K;
     wrow[j] = WT == kW32 ? static_cast<const void*>(static_cast<const int32_t*>(wv) + off)
-                         : static_cast<const void*>(static_cast<const int8_t*>(wv) + off + size_t(plane) * N * K);
+                         : static_cast<const void*>(static_cast<const int8_t*>(wv) + off + size_t(first) * N * K);
     w_at[j] = row * kBK + ((wc ^ wt_swizzle(row)) << 4);
   }
-  const uint32_t sel = 0x0c0c0400u + 0x0101u * unsigned(plane);
+  // the K loop of weight plane `plane`
+  const auto products = [&](int plane, int (&colsum)[CB], v16i (&acc)[4][CB]) {
+    const uint32_t sel = 0x0c0c0400u + 0x0101u * unsigned(plane);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      colsum[cb] = 0;
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = v16i{0};
+    }
+    RegTile<WT> r;
+    if constexpr (!FUSED) reg_load<WT>(r, xrow, wrow, k_begin + 2 * xc, k_begin + 16 * wc, k_end);
+    const auto step = [&](uint8_t* rs, uint8_t* ws, int k) {
+      if constexpr (FUSED) reg_load<WT>(r, xrow, wrow, k + 2 * xc, k + 16 * wc, k_end);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(rs + x_at[j]) = r.x[j];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (WT == kW32)
+          *reinterpret_cast<uint4*>(ws + w_at[j]) = make_uint4(digit4(r.w[4 * j], sel), digit4(r.w[4 * j + 1], sel),
+                                                               digit4(r.w[4 * j + 2], sel), digit4(r.w[4 * j + 3], sel));
+        else
+          *reinterpret_cast<uint4*>(ws + w_at[j]) = r.w[j];
+      }
+      __syncthreads();
+      const int kn = k + kBK;
+      if (!FUSED && kn < k_end) reg_load<WT>(r, xrow, wrow, kn + 2 * xc, kn + 16 * wc, k_end);
+      mfma_step<CB>(c, static_cast<const uint8_t*>(rs), static_cast<const uint8_t*>(ws), colsum, acc);
+    };
+    for (int k = k_begin; k < k_end; k += 2 * kBK) {
+      step(raw[0], wt[0], k);
+      if (k + kBK < k_end) step(raw[1], wt[1], k + kBK);
+    }
+  };
   int colsum[CB];
   v16i acc[4][CB];
+  if constexpr (!FUSED) {
+    products(first, colsum, acc);
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    colsum[cb] = 0;
+    for (int cb = 0; cb < CB; ++cb) {
+      const int col = n0 + c.wn * 32 * CB + cb * 32 + c.i;
+      const uint64_t corr = column_correction(colsum[cb]);
+      const int sh = 8 * first + (shifts && col < N ? int(shifts[col]) : 0);
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = v16i{0};
-  }
-  RegTile<WT> r;
-  reg_load<WT>(r, xrow, wrow, k_begin + 2 * xc, k_begin + 16 * wc, k_end);
-  const auto step = [&](uint8_t* rs, uint8_t* ws, int k) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(rs + x_at[j]) = r.x[j];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if constexpr (WT == kW32)
-        *reinterpret_cast<uint4*>(ws + w_at[j]) = make_uint4(digit4(r.w[4 * j], sel), digit4(r.w[4 * j + 1], sel),
-                                                             digit4(r.w[4 * j + 2], sel), digit4(r.w[4 * j + 3], sel));
-      else
-        *reinterpret_cast<uint4*>(ws + w_at[j]) = r.w[j];
+      for (int rb = 0; rb < 4; ++rb)
+        store_tile(acc[rb][cb], m0 + c.wm * 16 + rb * 4, col, c.khalf, corr, sh, gridDim.z > 1, mask, y, M, N);
     }
-    __syncthreads();
-    const int kn = k + kBK;
-    if (kn < k_end) reg_load<WT>(r, xrow, wrow, kn + 2 * xc, kn + 16 * wc, k_end);
-    mfma_step<CB>(c, static_cast<const uint8_t*>(rs), static_cast<const uint8_t*>(ws), colsum, acc);
-  };
-  for (int k = k_begin; k < k_end; k += 2 * kBK) {
-    step(raw[0], wt[0], k);
-    if (k + kBK < k_end) step(raw[1], wt[1], k + kBK);
-  }
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    const int col = n0 + c.wn * 32 * CB + cb * 32 + c.i;
-    const uint64_t corr = column_correction(colsum[cb]);
-    const int sh = 8 * plane + (shifts && col < N ? int(shifts[col]) : 0);
+  } else {
+    uint64_t total[4][CB][2];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
-      store_tile(acc[rb][cb], m0 + c.wm * 16 + rb * 4, col, c.khalf, corr, sh, gridDim.z > 1, mask, y, M, N);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) total[rb][cb][0] = total[rb][cb][1] = 0;
+#pragma unroll 1
+    for (int plane = 0; plane < 3; ++plane) {
+      products(plane, colsum, acc);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
+        const uint64_t corr = column_correction(colsum[cb]);
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          uint64_t sum[2];
+          tile_sums(acc[rb][cb], c.khalf, sum);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) total[rb][cb][h] += (corr + sum[h]) << (8 * plane);
+        }
+      }
+      if constexpr (WT == kWPlanes) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wrow[j] = static_cast<const int8_t*>(wrow[j]) + size_t(N) * K;
+      }
+      __syncthreads();  // both stages are read: the next plane writes them
+    }
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      const int col = n0 + c.wn * 32 * CB + cb * 32 + c.i;
+      if (col >= N) continue;
+      const int sh = shifts ? int(shifts[col]) : 0;
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int row = m0 + c.wm * 16 + rb * 4 + 2 * c.khalf + h;
+          if (row < M) y[size_t(row) * N + col] = (sh < 64 ? total[rb][cb][h] << sh : 0) & mask;
+        }
+    }
   }
 }
 
@@ -1047,12 +1104,14 @@ static hipError_t run_share_gemm(const uint64_t* x, const void* w, int w_bits, c
     if (e != hipSuccess || c.kernel == kGemmZero) return e;
   }
   const dim3 block(kThreads);
-  const unsigned gy = unsigned((M + kBM - 1) / kBM), gz = unsigned(c.splits * c.planes);
+  const unsigned gy = unsigned((M + kBM - 1) / kBM), gz = c.kernel == kGemmRegFused ? 1u : unsigned(c.splits * c.planes);
   const dim3 grid2(unsigned((N + kBN - 1) / kBN), gy, gz);
   const auto reg = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid2, block, 0, s, x, w, shifts, y, M, K, N, mask, c.k_split, c.splits);
   };
-  if (c.kernel == kGemmReg)
+  if (c.kernel == kGemmRegFused)
+    w_bits == 32 ? reg(share_gemm_reg_kernel<kW32, true>) : reg(share_gemm_reg_kernel<kWPlanes, true>);
+  else if (c.kernel == kGemmReg)
     w_bits == 32 ? reg(share_gemm_reg_kernel<kW32>) : reg(share_gemm_reg_kernel<kW8>);
   else if (c.kernel == kGemmDma2)
     hipLaunchKernelGGL(share_gemm_dma_kernel<2>, grid2, block, 0, s, x, static_cast<const int8_t*>(w), shifts, y, M, K,

@@ -28,8 +28,9 @@ inline size_t few_bytes(int w_bits, int M, int K, int N) {
   return wgs * size_t(std::max(K, kFewWaves * kFewChunk)) * 32 * (rb + (w_bits == 8 ? 1 : w_bits == 24 ? 3 : 4));
 }
 
+// kGemmRegFused: the register-staged tile with the three planes in one workgroup;
 // kGemmZero: K = 0, the empty sum; y is zeroed.
-enum GemmKernel { kGemmFew, kGemmDma2, kGemmDma3, kGemmReg, kGemmZero };
+enum GemmKernel { kGemmFew, kGemmDma2, kGemmDma3, kGemmReg, kGemmRegFused, kGemmZero };
 struct GemmChoice {
   GemmKernel kernel;
   int rb;               // kGemmFew: 4-row blocks per workgroup
@@ -70,6 +71,19 @@ inline GemmChoice gemm_choice(const void* x, const void* w, int w_bits, int M, i
   c.kernel = !dma ? kGemmReg : (splits == 1 && c.planes == 1 && wg2 > 256 && wg2 < 512 && tiles3 <= 256) ? kGemmDma3 : kGemmDma2;
   c.k_split = (ksteps + splits - 1) / splits * kBK;
   c.splits = (K + c.k_split - 1) / c.k_split;
+  // Three planes in one workgroup: a third of the workgroups, but no clear, atomics
+  // and mask over y, which cost most while K is short.  us, planes apart /
+  // together - three planes: 1000x16x1024 (256 tiles, 1 step) 29.4 / 11.9,
+  // 1000x700x1024 (256, 11) 51.3 / 41.4, 1000x200x512 (128, 4) 20.6 / 20.0,
+  // 1000x300x512 (128, 5) 21.4 / 23.1, 200x47x1024 (56, 1) 11.9 / 12.1; int32:
+  // 1000x200x1024 (256, 4) 41.7 / 31.6, 1000x512x1024 (256, 8) 45.8 / 45.8,
+  // 1000x100x512 (128, 2) 21.9 / 21.3, 1000x200x512 (128, 4) 24.0 / 29.8.
+  const int most = w_bits == 24 ? (tiles2 >= 256 ? 15 : tiles2 >= 128 ? 4 : tiles2 >= 64 ? 1 : 0)
+                                : (tiles2 >= 256 ? 4 : tiles2 >= 128 ? 2 : 0);
+  if (c.kernel == kGemmReg && c.planes == 3 && ksteps <= most) {
+    c.kernel = kGemmRegFused;
+    return c;
+  }
   c.adds = c.splits * c.planes > 1;
   return c;
 }

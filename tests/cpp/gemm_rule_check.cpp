@@ -4,7 +4,7 @@
 #include "gemm_rule.hpp"
 
 int main() {
-  static const char* names[] = {"few", "dma2", "dma3", "reg", "zero"};
+  static const char* names[] = {"few", "dma2", "dma3", "reg", "fused", "zero"};
   unsigned long long x, w;
   int bits, m, k, n;
   while (std::scanf("%llu %llu %d %d %d %d", &x, &w, &bits, &m, &k, &n) == 6) {

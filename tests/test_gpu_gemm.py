@@ -301,3 +301,35 @@ def test_gemm_empty_sum(gpu, m, n, bits):
     torch.cuda.synchronize()
     assert not y.any()
     np.testing.assert_array_equal(from_dev(y1), oracle.share_gemm(x1, w1))
+
+
+@pytest.mark.parametrize("wdt,m,k,n,want", [
+    ("i32split", 1455, 47, 1057, "fused"), ("i32split", 1024, 1, 1024, "fused"), ("i32split", 1030, 65, 1030, "fused"),
+    ("i32split", 1000, 700, 1024, "fused"), ("i32split", 300, 200, 6500, "fused"), ("i32split", 2100, 64, 130, "fused"),
+    ("i32", 1455, 47, 1057, "fused"), ("i32", 702, 19, 3032, "fused"), ("i32", 1001, 255, 1023, "fused"),
+    ("i32", 1001, 257, 1023, "reg"), ("i32split", 1000, 300, 512, "reg")])
+def test_gemm_planes_in_one_workgroup(gpu, wdt, m, k, n, want):
+    """Three-plane products of short K keep the outputs' sums in registers over
+    the planes: rows and columns off the tile, K about a step, odd and even
+    step counts, extreme weights, shifts and the 59-bit ring; the two that the
+    rule leaves to planes of their own beside them.  Exact."""
+    import gemm_rule
+    import torch
+    print(f"[gemm] m={m} k={k} n={n} {wdt} {want}", flush=True)
+    x = oracle.fill_u64(m * k, 19000 + m).reshape(m, k)
+    w = ((oracle.fill_u64(n * k, 19100 + n) % np.uint64(0x7F7F7F + 0x808080 + 1)).astype(np.int64)
+         - 0x808080).astype(np.int32).reshape(n, k)
+    w.flat[0], w.flat[-1] = 0x7F7F7F, -0x808080
+    sh = oracle.fill_shift(n, 19200 + k)
+    tx, tw = to_dev(x), torch.from_numpy(w).cuda()
+    if wdt == "i32split":  # one byte off 16, so that no K takes the LDS DMA
+        off = torch.zeros(3 * n * k + 1, dtype=torch.int8, device="cuda")[1:].view(3, n, k)
+        off.copy_(praghip.split_weights(tw))
+        tw = off
+    assert gemm_rule.kernel(wdt, m, k, n, tx.data_ptr(), tw.data_ptr())[0] == want
+    for shifts, mask in ((None, 64), (sh, 59)):
+        ts = None if shifts is None else torch.from_numpy(shifts).cuda()
+        y = torch.full((m, n), -1, dtype=torch.int64, device="cuda")
+        praghip.share_gemm(tx, tw, y=y, shifts=ts, mask_bits=mask)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(from_dev(y), oracle.share_gemm(x, w, shifts, mask))
