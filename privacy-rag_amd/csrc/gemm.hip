@@ -1152,7 +1152,7 @@ hipError_t launch_share_gemm_group(const praghip_gemm_desc* list, size_t count, 
     if (d.m == 0 || d.n == 0) continue;
     GemmChoice c = gemm_choice(d.x, d.w, d.w_bits, int(d.m), int(d.k), int(d.n));
     if (d.w_bits == 8 && c.kernel == kGemmFew && d.m > 4 && moved > kFewBytes) {
-      const GemmChoice t = gemm_choice(d.x, d.w, 8, int(d.m), int(d.k), int(d.n), 0);
+      const GemmChoice t = gemm_choice(d.x, d.w, 8, int(d.m), int(d.k), int(d.n), false);
       if (t.kernel == kGemmDma2 || t.kernel == kGemmDma3) c = t;
     }
     const size_t tiles = ((d.m + 3) / 4) * ((d.n + kFewCols - 1) / kFewCols);
