@@ -36,9 +36,10 @@ inline size_t few_bytes(int w_bits, int M, int K, int N) {
 //   64x64x3072 11.8 / 5.6 (384).  Three and more: 1000x100x300 16.8 / 8.4 (630),
 //   1000x64x300 17.1 / 5.7 (630), 400x64x1024 21.7 / 5.8 (800);
 //   three planes: 64x64x1024 6.8 / 9.0 (256), 16x3072x1024 15.2 / 15.8, but 8x4096x1024
-//   19.4 / 17.1 where the DMA tiles' splits still fit one round (1x3804x308 13.5 / 18.8); 200x128x512 8.3 /
-//   10.2 (400), 200x1024x512 13.7 / 15.0 (400), but 32x2048x3072 23.5 / 19.1 (384),
-//   64x64x3072 17.2 / 10.4 (768);
+//   19.4 / 17.1 where the DMA tiles' splits still fit one round (1x3804x308, on no
+//   DMA, 13.5 / 18.8); 200x128x512 8.3 / 10.2 (400), 200x1024x512 13.7 / 15.0 (400),
+//   406x28x178 11.0 / 13.0 (306), but 32x2048x3072 23.5 / 19.1 (384), 64x64x3072 17.2 /
+//   10.4 (768);
 //   int32, whose tiles split the digits at every use: 13x3072x1024 20.8 / 23.3,
 //   200x512x512 13.4 / 19.5 (400), 1024x800x100 22.8 / 25.7 (512), but 400x64x300 15.7 /
 //   11.6 (500), 400x1024x300 27.3 / 21.2 (500: from 1024 on the tiles split K).
@@ -51,7 +52,7 @@ inline bool few_pays(int w_bits, bool dma, long tile_groups, int M, int K, int N
   if (w_bits == 8)
     return near && (rounds == 1 ? !(dma && K <= kBK && M > 8) : rounds == 2 && K >= 448 && K <= 1024);
   if (w_bits == 24)
-    return rounds == 1 ? K <= 3072 || !dma || M <= 4 || tile_groups > 256 : rounds == 2 && near && K > kBK && K <= 1024;
+    return rounds == 1 ? K <= 3072 || !dma || M <= 4 || tile_groups > 256 : rounds == 2 && near && (K > kBK || !dma) && K <= 1024;
   return rounds == 1 || (K >= 100 && ((rounds == 2 && (K < 1024 || N <= 64)) || (rounds <= 4 && K <= 600)));
 }
 

@@ -31,7 +31,7 @@ def test_k_splits_cover_k(w_bits):
     ("i8", [(1, 1024, 4096), (64, 1024, 1024), (64, 63, 1024), (8, 64, 8000), (400, 512, 512), (200, 1024, 1024), (1000, 3072, 64)],
      [(64, 64, 1024), (64, 64, 3072), (400, 64, 1024), (1000, 64, 300), (1000, 100, 300), (4000, 100, 70), (100, 128, 3072),
       (400, 300, 512), (512, 64, 512), (1000, 128, 300), (1000, 3072, 128), (512, 1024, 3072)]),
-    ("i32split", [(64, 64, 1024), (16, 3072, 1024), (200, 128, 512), (200, 1024, 512), (4000, 1024, 32), (64, 3072, 1024), (1, 3804, 308)],
+    ("i32split", [(64, 64, 1024), (16, 3072, 1024), (200, 128, 512), (200, 1024, 512), (4000, 1024, 32), (64, 3072, 1024), (1, 3804, 308), (406, 28, 178)],
      [(200, 64, 1024), (64, 64, 3072), (400, 47, 512), (32, 2048, 3072), (8, 4096, 1024), (77, 3072, 1024)]),
     ("i32", [(13, 3072, 1024), (200, 512, 512), (200, 700, 512), (1024, 800, 100), (4000, 1024, 32)],
      [(400, 64, 300), (400, 1024, 300), (702, 19, 3032), (13, 3072, 4096)])])
