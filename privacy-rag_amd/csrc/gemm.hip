@@ -1132,16 +1132,21 @@ hipError_t launch_share_gemm(const uint64_t* x, const void* w, int w_bits, const
   return run_share_gemm(x, w, w_bits, shifts, y, M, K, N, mask_bits, s, false);
 }
 
-// Products whose order does not matter: the int8 ones in launches of up to
-// kGroupMax, those of few rows by their row blocks and the DMA path's as
+// Products whose order does not matter: those of few rows in launches of up to
+// kGroupMax by their weight form and row blocks, the DMA path's int8 ones as
 // 128-column tiles, longest K first (the last round of tiles is then one of
 // short ones); the rest one by one, the outputs they add into zeroed together.
 // A grid of many products fills the chip with either kernel, and then the bytes
 // per product decide: for every 32 columns and k a tile moves 96, the few-row
 // kernel 64 (up to 4 rows), 96 or 160.  56 products of 16 rows: tiles 85 us,
 // few-row 142 us; of one row: 77 and 60 us.
+// A grid of tiles has no need of K splits, but one product alone may: where the
+// split saves 16 K steps and more it takes its own path.  us, unsplit / split with
+// its clear and mask: 200x3072x1024 (48 steps to 12) 31.0 / 18.4, 512x3072x1024 (48 to
+// 24) 31.8 / 28.4, 200x1024x3072 (16 to 8) 13.9 / 20.4.  Four three-plane products
+// 16x3072x1024 64 us one after the other (64 workgroups each), 17 together.
 hipError_t launch_share_gemm_group(const praghip_gemm_desc* list, size_t count, hipStream_t s) {
-  std::vector<const praghip_gemm_desc*> few[3], dma, rest, adds;
+  std::vector<const praghip_gemm_desc*> few[3][3], dma, rest;
   hipError_t e = hipSuccess;
   size_t moved = 0;
   for (size_t i = 0; i < count; ++i)
@@ -1156,15 +1161,23 @@ hipError_t launch_share_gemm_group(const praghip_gemm_desc* list, size_t count, 
       if (t.kernel == kGemmDma2 || t.kernel == kGemmDma3) c = t;
     }
     const size_t tiles = ((d.m + 3) / 4) * ((d.n + kFewCols - 1) / kFewCols);
-    if (d.w_bits == 8 && c.kernel == kGemmFew && tiles < (1u << 24))
-      few[c.rb >> 1].push_back(&d);
+    if (c.kernel == kGemmFew && tiles < (1u << 24))
+      few[d.w_bits == 8 ? 0 : d.w_bits == 24 ? 1 : 2][c.rb >> 1].push_back(&d);
     else if (d.w_bits == 8 && (c.kernel == kGemmDma2 || c.kernel == kGemmDma3) && tiles < (1u << 24))
       dma.push_back(&d);
-    else {
+    else
       rest.push_back(&d);
-      if (c.adds) adds.push_back(&d);
+  }
+  if (dma.size() == 1) {
+    const praghip_gemm_desc& d = *dma[0];
+    if (int(d.k) - gemm_choice(d.x, d.w, 8, int(d.m), int(d.k), int(d.n), false).k_split >= 16 * kBK) {
+      rest.push_back(dma[0]);
+      dma.clear();
     }
   }
+  std::vector<const praghip_gemm_desc*> adds;
+  for (const praghip_gemm_desc* d : rest)
+    if (gemm_choice(d->x, d->w, d->w_bits, int(d->m), int(d->k), int(d->n)).adds) adds.push_back(d);
   const bool together = adds.size() > 1;
   for (size_t a0 = 0; together && a0 < adds.size() && e == hipSuccess; a0 += kGemmClearMax) {
     GemmClearList l{};
@@ -1193,10 +1206,11 @@ hipError_t launch_share_gemm_group(const praghip_gemm_desc* list, size_t count, 
       e = launch(g, tiles);
     }
   };
-  for (int i = 0; i < 3; ++i) {
-    const int rb = 1 << i;
-    run(few[i], 4 * rb, kFewCols, [&](const GemmGroup& g, unsigned tiles) { return launch_few(g, rb, 8, tiles, s); });
-  }
+  for (int f = 0; f < 3; ++f)
+    for (int i = 0; i < 3; ++i) {
+      const int bits = f == 0 ? 8 : f == 1 ? 24 : 32, rb = 1 << i;
+      run(few[f][i], 4 * rb, kFewCols, [&](const GemmGroup& g, unsigned tiles) { return launch_few(g, rb, bits, tiles, s); });
+    }
   run(dma, kBM, kBN, [&](const GemmGroup& g, unsigned tiles) {
     hipLaunchKernelGGL(share_gemm_group_kernel, dim3(tiles), dim3(kThreads), 0, s, g);
     return hipGetLastError();

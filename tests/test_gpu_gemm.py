@@ -333,3 +333,52 @@ def test_gemm_planes_in_one_workgroup(gpu, wdt, m, k, n, want):
         praghip.share_gemm(tx, tw, y=y, shifts=ts, mask_bits=mask)
         torch.cuda.synchronize()
         np.testing.assert_array_equal(from_dev(y), oracle.share_gemm(x, w, shifts, mask))
+
+
+def _mixed_batch(specs, seed, stale=-1):
+    """specs: (m, k, n, wdt, mask); runs them as one batch with operands of
+    their own and compares each output exactly."""
+    import ctypes
+
+    import gemm_rule
+    import torch
+    from praghip._lib import GemmDesc, check, lib
+    descs, keep, want = [], [], []
+    for i, (m, k, n, wdt, mask) in enumerate(specs):
+        x = oracle.fill_u64(m * k, seed + 4 * i).reshape(m, k)
+        if wdt == "i8":
+            w = oracle.fill_i8(n * k, seed + 4 * i + 1).reshape(n, k)
+        else:
+            w = ((oracle.fill_u64(n * k, seed + 4 * i + 1) % np.uint64(1 << 21)).astype(np.int64)
+                 - (1 << 20)).astype(np.int32).reshape(n, k)
+        tw = torch.from_numpy(w).cuda()
+        if wdt == "i32split":
+            tw = praghip.split_weights(tw)
+        sh = oracle.fill_shift(n, seed + 4 * i + 2)
+        tx, ts = to_dev(x), torch.from_numpy(sh).cuda()
+        y = torch.full((m, n), stale, dtype=torch.int64, device="cuda")
+        keep.append((tx, tw, ts, y))
+        want.append(oracle.share_gemm(x, w, sh, mask))
+        descs.append(GemmDesc(tx.data_ptr(), tw.data_ptr(), ts.data_ptr(), y.data_ptr(), m, k, n,
+                              gemm_rule.W_BITS[wdt], mask))
+    arr = (GemmDesc * len(descs))(*descs)
+    check(lib().praghip_share_gemm_batch(0, ctypes.cast(arr, ctypes.c_void_p), len(descs),
+                                         torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    for i, (_, _, _, y) in enumerate(keep):
+        np.testing.assert_array_equal(from_dev(y), want[i], err_msg=f"product {i} {specs[i]}")
+
+
+def test_gemm_batch_lone_tile_product_and_grouped_planes(gpu):
+    """One tiled product among products of few rows keeps its K split; the
+    three-plane and int32 products of few rows run in one launch per form."""
+    import gemm_rule
+    tiled = (200, 3072, 1024, "i8", 59)
+    assert gemm_rule.kernel("i8", *tiled[:3])[:3] == ("dma2", 768, 4)
+    few = [(16, 3072, 256, "i32split", 59), (3, 1000, 70, "i32split", 64), (9, 129, 300, "i32split", 59),
+           (13, 700, 90, "i32", 59), (4, 64, 33, "i32", 64), (16, 1024, 256, "i32", 59), (5, 100, 40, "i8", 64)]
+    assert all(gemm_rule.kernel(wdt, m, k, n)[0] == "few" for m, k, n, wdt, _ in few)
+    print("[gemm] batch: one tiled product, few rows of every form", flush=True)
+    _mixed_batch(few[:3] + [tiled] + few[3:], 20000)
+    print("[gemm] batch: few rows alone, more than one launch holds", flush=True)
+    _mixed_batch(few * 6, 21000)
