@@ -70,16 +70,18 @@ typedef struct praghip_timing {
 
 /* Switch::Timing (switch.hpp:10): the phases of the last host-buffer keyswitch
  * (apply / evaluate), from events on the plan's stream between its launches.
- * At N = 16384 (digits of one to three primes) the keyswitch runs in three
- * kernel phases, whose boundaries are not the reference's:
- *   rns_ntt_ms  - ModUp (decompose, base conversion) and forward stages 0-3
- *                 of every expanded digit limb (the column kernel);
- *   product_ms  - forward stages 4-13, the key inner product and inverse
- *                 stages 0-9 of both sums (the row kernel);
- *   inverse_ms  - inverse stages 10-13 of the special prime's limbs;
- *   moddown_ms  - inverse stages 10-13 of the data primes' limbs with ModDown.
+ * At N = 4096, 8192 and 16384 (digits of one to three primes; below 16384 with
+ * every prime below 2^60) the keyswitch runs in three kernel phases, whose
+ * boundaries are not the reference's; C = log2 N - 10:
+ *   rns_ntt_ms  - ModUp (decompose, base conversion) and forward stages
+ *                 0 .. C-1 of every expanded digit limb (the column kernel);
+ *   product_ms  - the other ten forward stages, the key inner product and
+ *                 inverse stages 0-9 of both sums (the row kernel);
+ *   inverse_ms  - inverse stages 10 and on of the special prime's limbs;
+ *   moddown_ms  - the same stages of the data primes' limbs with ModDown.
  * At other sizes the whole-limb kernel (ModUp, transforms and product) is
- * product_ms, its ModDown moddown_ms, and rns_ntt_ms = inverse_ms = 0.
+ * product_ms, its ModDown moddown_ms, and rns_ntt_ms and inverse_ms are no
+ * more than the time between two events.
  * setup_upload_ms is the plan's table, constant and key upload at creation.
  * The phases sum to kernel_ms of praghip_switch_timing. */
 typedef struct praghip_switch_phases {

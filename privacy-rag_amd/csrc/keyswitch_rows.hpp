@@ -1109,7 +1109,8 @@ void launch_chunk(KsRows f, const KsConst& kc, hipStream_t s, hipEvent_t* ev) {
     hipLaunchKernelGGL((ks_rows2_kernel<LOG, AU>), dim3(items), dim3(kRow2Threads), 0, s, f, t_u64);
   mark(1);
   const unsigned c_blocks = f.cts * 2 * L * kCols / 256;
-  const bool self = c_blocks <= kSelfBlocks;
+  // timed phases keep the special prime's columns apart: its time is a phase
+  const bool self = c_blocks <= kSelfBlocks && !ev;
   if (!self)
     hipLaunchKernelGGL((ks_cols_special_kernel<LOG, AU>), dim3(f.cts * 2 * kCols / 256), dim3(256), 0, s, f);
   mark(2);

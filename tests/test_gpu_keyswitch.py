@@ -331,3 +331,28 @@ def test_keyswitch_primes_off_a_power_of_two(gpu, log_n, L, dnum, batch):
     got = from_dev(tout)
     for b in sorted({0, batch - 1}):
         np.testing.assert_array_equal(got[b], oracle.keyswitch(ct[b:b + 1], key, q, dnum, log_n, 3)[0])
+
+
+def _phase_medians(q, log_n, dnum, calls=25):
+    n, L = 1 << log_n, len(q) - 1
+    ct = oracle.fill_residues(2 * L, n, q[:L], 0x7b + log_n).reshape(2, L, n)
+    key = oracle.fill_residues(dnum * 2 * (L + 1), n, q, 0x7c + log_n).reshape(dnum, 2, L + 1, n)
+    sw = praghip.Switch(q, log_n, dnum, key=key, element=3)
+    want = oracle.keyswitch(ct[None], key, q, dnum, log_n, 3)[0]
+    rows = []
+    for _ in range(calls):
+        np.testing.assert_array_equal(sw.apply(ct), want)
+        ph = sw.phase_timing()
+        rows.append([1e3 * x for x in (ph.rns_ntt_ms, ph.product_ms, ph.inverse_ms, ph.moddown_ms)])
+    return np.median(np.array(rows), axis=0)
+
+
+def test_keyswitch_phases_time_the_special_prime(gpu):
+    """inverse_ms is the special prime's inverse columns, a kernel of its own in
+    a timed call: clearly longer than the gap between two events, which is what
+    the whole-limb path leaves in that field."""
+    gap = _phase_medians(list(cf.LOCKED_PRIMES[:3]) + [cf.LOCKED_PRIMES[6]], 11, 3)[2]
+    for log_n, dnum in ((14, 6), (14, 3), (13, 6), (12, 2)):
+        ph = _phase_medians(list(cf.LOCKED_PRIMES), log_n, dnum)
+        print(f"[ks] phases N={1 << log_n} dnum={dnum} us {np.round(ph, 1).tolist()} gap {gap:.1f}", flush=True)
+        assert ph[2] > 1.15 * gap
