@@ -7,6 +7,8 @@
 // is a single HBM pass; one thread per output coefficient, contiguous in the
 // coefficient index so reads and writes coalesce except the Galois-permuted
 // reads, which stay inside one 2^log_n-word limb.
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace praghip {
@@ -42,7 +44,9 @@ static unsigned elem_grid(size_t items) {
 //       kMacWide - primes of 2^60 and more.
 //
 // Primes of 2^60 and more: a Shoup quotient per weight word (from the Barrett
-// ratio), Shoup products and canonical sums.
+// ratio), Shoup products and canonical sums; one or two columns in a loop of their
+// own (one column of two 62-bit primes, 19 blocks and 2 slots, N = 4096, the whole
+// evaluation, us: 61 with four columns formed and one stored, 42 so).
 constexpr int kMacCoords = 4;
 enum MacMode { kMacPm, kMacNarrow, kMacWide };
 
@@ -80,7 +84,7 @@ __global__ void __launch_bounds__(256)
   const Barrett m = bl.m[p];
   const size_t words = size_t(limbs) << log_n, wcol = (size_t(blocks) * P) << log_n;
   const unsigned cn = coords - c0 < unsigned(kMacCoords) ? coords - c0 : unsigned(kMacCoords);
-  // past the last limb or column a thread works on the last one again and
+  // past the last limb or column a thread works on the first one again and
   // does not store it: no branch in the loop
   size_t xo[KL], wo[kMacCoords];
 #pragma unroll
@@ -166,27 +170,37 @@ __global__ void __launch_bounds__(256)
           store(c, k, mul_shoup(r, 1, mc.one_q, m.q));
       }
   } else {
-    uint64_t acc[kMacCoords][KL];
+    // the products bound this loop, so one or two columns get a loop of their own
+    const auto wide = [&](auto columns) {
+      constexpr int C = decltype(columns)::value;
+      uint64_t acc[C][KL];
 #pragma unroll
-    for (int c = 0; c < kMacCoords; ++c)
+      for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int k = 0; k < KL; ++k) acc[c][k] = 0;
-    for (unsigned b = 0; b < blocks; ++b) {
-      uint64_t xv[KL];
+        for (int k = 0; k < KL; ++k) acc[c][k] = 0;
+      for (unsigned b = 0; b < blocks; ++b) {
+        uint64_t xv[KL];
 #pragma unroll
-      for (int k = 0; k < KL; ++k) xv[k] = (in + size_t(b) * words + xo[k])[z];
+        for (int k = 0; k < KL; ++k) xv[k] = (in + size_t(b) * words + xo[k])[z];
 #pragma unroll
-      for (int c = 0; c < kMacCoords; ++c) {
-        const uint64_t wv = (w + wo[c] + ((size_t(b) * P) << log_n))[z];
-        const uint64_t wq = shoup_quotient(wv, m);
+        for (int c = 0; c < C; ++c) {
+          const uint64_t wv = (w + wo[c] + ((size_t(b) * P) << log_n))[z];
+          const uint64_t wq = shoup_quotient(wv, m);
 #pragma unroll
-        for (int k = 0; k < KL; ++k) acc[c][k] = add_mod(acc[c][k], mul_shoup(xv[k], wv, wq, m.q), m.q);
+          for (int k = 0; k < KL; ++k) acc[c][k] = add_mod(acc[c][k], mul_shoup(xv[k], wv, wq, m.q), m.q);
+        }
       }
-    }
 #pragma unroll
-    for (int c = 0; c < kMacCoords; ++c)
+      for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int k = 0; k < KL; ++k) store(c, k, acc[c][k]);
+        for (int k = 0; k < KL; ++k) store(c, k, acc[c][k]);
+    };
+    if (cn > 2)
+      wide(std::integral_constant<int, kMacCoords>{});
+    else if (cn == 2)
+      wide(std::integral_constant<int, 2>{});
+    else
+      wide(std::integral_constant<int, 1>{});
   }
 }
 
