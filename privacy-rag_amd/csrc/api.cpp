@@ -777,7 +777,7 @@ int praghip_switch_plan_create(int device, const uint64_t* q, size_t data_primes
   if (e == hipSuccess && fused) e = hipMemsetAsync(p->queue, 0, kQueueWords * 4, p->stream);
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->prod, max_batch * 2 * K * n * 8, true);
   if (e == hipSuccess && keyswitch_rows_supported(p->kc)) {
-    p->inter_cts = std::min(max_batch, kKsRowsChunk);
+    p->inter_cts = std::min(max_batch, keyswitch_rows_chunk(p->kc));
     e = p->buf.alloc((void**)&p->inter, p->inter_cts * dnum * K * n * 8, true);
   }
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->in, 2 * L * n * 8, true);

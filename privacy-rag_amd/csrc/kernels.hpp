@@ -172,13 +172,14 @@ hipError_t launch_keyswitch(const KsArgs& a, const KsConst* kc_dev, const KsCons
 // Workgroups of the fused keyswitch kernel for 2^log_n (the acc slots a plan
 // allocates); 0 for an unsupported size.
 unsigned ks_acc_slots(int log_n);
-// Three-phase keyswitch (columns, rows, columns) for N = 16384 with digits of
-// equal size 1..3; hipErrorNotSupported for any other shape or without the
-// `inter` scratch.  launch_keyswitch takes it when it applies.
+// Three-phase keyswitch (columns, rows, columns) at N = 4096, 8192 and 16384 with
+// digits of up to three primes, the first ones the largest; hipErrorNotSupported
+// for any other shape or without the `inter` scratch.  launch_keyswitch takes it
+// when it applies.
 bool keyswitch_rows_supported(const KsConst& kc);
 hipError_t launch_keyswitch_rows(const KsArgs& a, const KsConst* kc_dev, const KsConst& kc, const NttDevice& d,
                                  hipStream_t s);
 // Ciphertexts per three-phase chunk a plan sizes its `inter` scratch for.
-constexpr size_t kKsRowsChunk = 64;
+size_t keyswitch_rows_chunk(const KsConst& kc);
 
 }  // namespace praghip

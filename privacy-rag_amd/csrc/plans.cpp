@@ -622,7 +622,7 @@ int praghip_pack_plan_create(int device, const uint64_t* q, size_t data_primes, 
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->ksout, 2 * max_pairs * ct * 8, true);
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->prod, 2 * max_pairs * 2 * K * n * 8, true);
   if (e == hipSuccess && keyswitch_rows_supported(p->kc)) {
-    p->inter_cts = std::min(2 * max_pairs, kKsRowsChunk);
+    p->inter_cts = std::min(2 * max_pairs, keyswitch_rows_chunk(p->kc));
     e = p->buf.alloc((void**)&p->inter, p->inter_cts * dnum * K * n * 8, true);
   }
   if (e == hipSuccess) e = p->buf.alloc((void**)&p->host_in, 2 * ct * 8, true);

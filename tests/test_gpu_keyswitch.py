@@ -356,3 +356,25 @@ def test_keyswitch_phases_time_the_special_prime(gpu):
         ph = _phase_medians(list(cf.LOCKED_PRIMES), log_n, dnum)
         print(f"[ks] phases N={1 << log_n} dnum={dnum} us {np.round(ph, 1).tolist()} gap {gap:.1f}", flush=True)
         assert ph[2] > 1.15 * gap
+
+
+@pytest.mark.parametrize("log_n,kind,L,dnum,chunk,over", [(12, "50", 1, 1, 1024, 6), (12, "50", 2, 2, 341, 0),
+                                                          (13, "locked", 2, 1, 341, 3), (13, "50", 6, 3, 64, 1)])
+def test_keyswitch_chunks_of_the_scratch(gpu, log_n, kind, L, dnum, chunk, over):
+    """Below N = 16384 a chunk is as many ciphertexts as expand to 64 MiB (64 at
+    least): the plan holds scratch for one chunk, and batches that fill it or
+    pass it are exact on both sides of the bound."""
+    n, batch = 1 << log_n, chunk + over
+    q = (cf.primes_below(50, n, L) + cf.primes_below(60, n, 1)) if kind == "50" else \
+        list(cf.LOCKED_PRIMES[:L]) + [cf.LOCKED_PRIMES[6]]
+    print(f"[ks] chunk N={n} {kind} L={L} dnum={dnum} batch={batch}", flush=True)
+    ct = oracle.fill_residues(batch * 2 * L, n, q[:L], 0x7d + batch).reshape(batch, 2, L, n)
+    key = oracle.fill_residues(dnum * 2 * (L + 1), n, q, 0x7e + L).reshape(dnum, 2, L + 1, n)
+    one = praghip.Switch(q, log_n, dnum, max_batch=chunk).timing().device_bytes
+    sw = praghip.Switch(q, log_n, dnum, max_batch=batch)
+    assert sw.timing().device_bytes - one == over * 2 * (L + 1) * n * 8  # products only, no more expanded digits
+    tin, tout = to_dev(ct), to_dev(np.zeros_like(ct))
+    sw.keyswitch(tin, tout, keys=to_dev(key), key_stride=0, galois=3)
+    got = from_dev(tout)
+    for b in sorted({0, chunk - 1, min(chunk, batch - 1), batch - 1}):
+        np.testing.assert_array_equal(got[b], oracle.keyswitch(ct[b:b + 1], key, q, dnum, log_n, 3)[0])
