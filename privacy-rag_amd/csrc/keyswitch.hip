@@ -437,7 +437,12 @@ unsigned ks_acc_slots(int log_n) {
 
 template <int LOGN, class AU>
 static hipError_t launch_fused_n(KsFused f, hipStream_t s) {
-  const unsigned blocks = std::min(f.items, std::min(fused_grid<LOGN, AU>(), f.acc_slots));
+  // at N = 1024 ArPM's registers let a SIMD hold three waves, ArU64's two; on the
+  // third wave's workgroups large batches were slower (us, 3,072 / 2,048
+  // workgroups: 512 ciphertexts of three 50-bit digits, 3,584 items, 244 / 204; 900 of
+  // one digit of two, 2,700 items, 164 / 136)
+  const unsigned grid = std::min(fused_grid<LOGN, AU>(), LOGN == 10 ? fused_grid<LOGN, ArU64>() : ~0u);
+  const unsigned blocks = std::min(f.items, std::min(grid, f.acc_slots));
   f.xcd = (f.batch % kQueueGroups == 0 && blocks % kQueueGroups == 0) ? 1 : 0;
   hipLaunchKernelGGL((ks_fused_kernel<LOGN, AU>), dim3(blocks), dim3(ntt_threads<LOGN>()), 0, s, f);
   return hipGetLastError();
