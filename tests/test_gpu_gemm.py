@@ -162,11 +162,11 @@ def _batch(descs):
 
 
 def test_gemm_batch_split_k_outputs_cleared_together(gpu):
-    """praghip_share_gemm_batch zeroes the outputs of its split-K products in
-    one launch before the first product (the Qwen3 o and down shapes here,
-    with and without the 59-bit mask), and falls back to a clear per product
-    when such an output is also an earlier product's input: product 1 reads
-    buffer B as its shares, then product 2 (split K) writes B."""
+    """praghip_share_gemm_batch on outputs that hold stale values: products that
+    would split K alone run together (the Qwen3 o and down shapes here, with
+    and without the 59-bit mask), and one after the other, each with its own
+    clear, when such an output is also an earlier product's input: product 1
+    reads buffer B as its shares, then product 2 (split K) writes B."""
     import torch
     specs = [(512, 2048, 1024, None, 64), (512, 3072, 1024, 7001, 59), (64, 1024, 512, None, 64),
              (512, 2048, 1024, 7002, 64)]
@@ -205,11 +205,11 @@ def test_gemm_batch_split_k_outputs_cleared_together(gpu):
                                    (129, 130, 1)])
 @pytest.mark.parametrize("wdt", ["i8", "i32", "i32split"])
 def test_gemm_any_k_and_alignment(gpu, m, k, n, wdt):
-    """Few-row and register-staged kernels around their edges: rows about the
-    4-row blocks and the 32-row tile, K about the 128-wide chunks and 64-wide
-    steps (odd K puts every weight row at another alignment), columns about 32
-    and 128; the operands start 8 bytes (x) and one element (w) off 16 bytes.
-    Whole-number arithmetic: exact."""
+    """Small products, most of them on the few-row kernel, around its edges: rows
+    about the 4-row blocks and the 32-row tile, K about the 128-wide chunks and
+    64-wide steps (odd K puts every weight row at another alignment), columns
+    about 32 and 128; the operands start 8 bytes (x) and one element (w) off 16
+    bytes.  Whole-number arithmetic: exact."""
     import torch
     print(f"[gemm] m={m} k={k} n={n} {wdt}", flush=True)
     x = oracle.fill_u64(m * k, 11000 + m).reshape(m, k)
@@ -382,3 +382,59 @@ def test_gemm_batch_lone_tile_product_and_grouped_planes(gpu):
     _mixed_batch(few[:3] + [tiled] + few[3:], 20000)
     print("[gemm] batch: few rows alone, more than one launch holds", flush=True)
     _mixed_batch(few * 6, 21000)
+
+
+def _off(t, elements=1):
+    """The tensor's values in memory that starts `elements` past an aligned address."""
+    import torch
+    flat = torch.zeros(t.numel() + elements, dtype=t.dtype, device="cuda")[elements:]
+    return flat.view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("wdt,m,k,n,x_off,w_off,want", [
+    ("i8", 486, 90, 1131, 0, 0, ("reg", 1)), ("i8", 700, 500, 700, 0, 0, ("reg", 1)),
+    ("i8", 1001, 31, 1025, 0, 0, ("reg", 1)), ("i8", 512, 1024, 1024, 1, 0, ("reg", 2)),
+    ("i8", 512, 1024, 1024, 0, 1, ("reg", 2)), ("i8", 300, 2047, 1025, 0, 0, ("reg", 4)),
+    ("i32split", 512, 2047, 1024, 0, 0, ("reg", 2)), ("i32split", 130, 4095, 500, 0, 0, ("reg", 4)),
+    ("i32", 512, 2047, 1024, 0, 0, ("reg", 2)), ("i32", 130, 4097, 520, 0, 0, ("reg", 4)),
+    ("i32", 1000, 640, 1024, 0, 0, ("reg", 1))])
+def test_gemm_register_staged_tiles(gpu, wdt, m, k, n, x_off, w_off, want):
+    """The register-staged tile: ragged K with the tail that a split or the row
+    cuts, odd and even step counts through its two LDS stages, K splits and planes
+    that add into y, operands off 16 bytes; exact."""
+    import gemm_rule
+    import torch
+    print(f"[gemm] m={m} k={k} n={n} {wdt} off {x_off} {w_off}", flush=True)
+    x = oracle.fill_u64(m * k, 22000 + m).reshape(m, k)
+    if wdt == "i8":
+        w = oracle.fill_i8(n * k, 22100 + n).reshape(n, k)
+        w.flat[-1] = -128
+    else:
+        w = ((oracle.fill_u64(n * k, 22200 + n) % np.uint64(0x7F7F7F + 0x808080 + 1)).astype(np.int64)
+             - 0x808080).astype(np.int32).reshape(n, k)
+        w.flat[0], w.flat[-1] = 0x7F7F7F, -0x808080
+    sh = oracle.fill_shift(n, 22300 + k)
+    tw = torch.from_numpy(w).cuda()
+    if wdt == "i32split":
+        tw = praghip.split_weights(tw)
+    tx, tw = _off(to_dev(x), x_off), _off(tw, w_off)
+    assert gemm_rule.kernel(wdt, m, k, n, tx.data_ptr(), tw.data_ptr())[0:3:2] == want
+    for shifts, mask in ((None, 64), (sh, 59)):
+        ts = None if shifts is None else torch.from_numpy(shifts).cuda()
+        y = torch.full((m, n), -1, dtype=torch.int64, device="cuda")
+        praghip.share_gemm(tx, tw, y=y, shifts=ts, mask_bits=mask)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(from_dev(y), oracle.share_gemm(x, w, shifts, mask))
+
+
+def test_gemm_batch_clears_added_outputs_together(gpu):
+    """Products of a batch that add into their outputs (planes and K splits on the
+    tiles) have them zeroed in one launch: stale outputs, with and without the
+    59-bit mask, beside products that store; exact."""
+    import gemm_rule
+    specs = [(512, 2047, 1024, "i32split", 59), (300, 2047, 1025, "i8", 59), (512, 1024, 1024, "i32", 64),
+             (77, 3072, 1024, "i32split", 64), (5, 100, 40, "i8", 59), (600, 128, 1000, "i8", 59), (600, 128, 900, "i8", 64)]
+    rule = [gemm_rule.kernel(wdt, m, k, n) for m, k, n, wdt, _ in specs]
+    assert [r[4] for r in rule] == [True, True, True, True, False, False, False]
+    print("[gemm] batch: outputs that are added into, cleared together", flush=True)
+    _mixed_batch(specs, 23000, stale=0x1234)
