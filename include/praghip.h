@@ -241,11 +241,13 @@ int praghip_share_gemm_valu(int device, const uint64_t *x, const int8_t *w, cons
  * quantize_weights.py:91,102).  Weights outside the range are not detected. */
 int praghip_weights_split(int device, const int32_t *w, int8_t *planes, size_t count, void *stream);
 
-/* A list of share GEMMs launched in order on one stream, for the per-layer
- * projections of Transformer::project_many / project_joint_many
- * (model.hpp:66-126): the joint q/k/v and gate/up products, o and down.  Each
- * entry has the meaning of praghip_share_gemm's arguments; the whole list is
- * validated before the first launch. */
+/* A list of share GEMMs on one stream, for the per-layer projections of
+ * Transformer::project_many / project_joint_many (model.hpp:66-126): the joint
+ * q/k/v and gate/up products, o and down.  Each entry has the meaning of
+ * praghip_share_gemm's arguments; the whole list is validated before the first
+ * launch.  The results are those of the products in list order: where an output
+ * overlaps another operand of the list they run in that order, otherwise together
+ * and in any. */
 typedef struct praghip_gemm_desc {
   const uint64_t *x;
   const void *w;

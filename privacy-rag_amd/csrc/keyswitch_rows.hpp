@@ -8,7 +8,8 @@
 //               0 .. C-1 (gaps N/2 .. 1024): thread c holds coefficients
 //               c + 1024 k, k < 2^C, and every twiddle is the same for all
 //               threads.  Out: E[b][j][t][N] (lazy, per-policy form).
-//   B  rows     two waves per (ciphertext, prime t, row r): forward stages
+//   B  rows     two waves (four on unreduced key-product sums, pairs of waves
+//               for few items) per (ciphertext, prime t, row r): forward stages
 //               C .. C+9 of each digit's row, the key product summed over the
 //               digits in registers, inverse stages 0-9 of both sums.
 //               Out: the products' rows, [b][2][K][N] (lazy).
@@ -86,7 +87,7 @@ __device__ __forceinline__ uint64_t gather(const uint64_t* __restrict__ limb, un
   return ((i >> LOG) && v) ? q - v : v;
 }
 
-// Column c (coefficients c + 1024 k, k < 16) of a limb after the Galois
+// Column c (coefficients c + 1024 k, k < kColE) of a limb after the Galois
 // gather; a plain strided read when the element is the identity (ginv is a
 // launch argument, so the branch is uniform).
 template <int LOG>
@@ -431,9 +432,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 1
 // ------------------------------------------------------------------ phase B
 // One item = (ciphertext, key prime t, row of 1024 coefficients) on the two
 // waves of a workgroup, 8 coefficients per lane (radix-8 register passes, one
-// exchange crossing the two waves, the others within a wave): forward stages
-// 4-13 of each digit's row, the key products summed over the digits in
-// registers, inverse stages 0-9 of both sums.  Eight coefficients per lane
+// exchange crossing the two waves, the others within a wave): the forward
+// stages from C on of each digit's row, the key products summed over the digits
+// in registers, inverse stages 0-9 of both sums (ks_rows4_kernel and
+// ks_rows_split_kernel are its other forms).  Eight coefficients per lane
 // keep a wave within 168 VGPRs, so a SIMD holds three waves.  The row's
 // forward twiddles are staged in LDS once per item (16 KiB beside the 8.5 KiB
 // exchange buffer: six items fit a CU's 160 KiB), so the digits' passes issue
@@ -553,8 +555,8 @@ __device__ __forceinline__ void row_passes_fwd_lds(typename A::T (&v)[E], typena
   }
 }
 
-// Item (ciphertext bl, prime t, row) on the two waves of the workgroup
-// (thread t2 < 128).  Policy A:
+// Item (ciphertext bl, prime t, row) on threads t2 < TH of the workgroup: two
+// waves with eight coefficients per lane, or four with four (SUMS).  Policy A:
 //   ArPM, ArU64L - every key prime below 2^60: Montgomery key products x k 2^-64
 //               of the transformed digit word (any x < 2^64) and
 //               the canonical key words (x k < q 2^64, each product

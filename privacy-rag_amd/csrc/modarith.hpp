@@ -200,7 +200,8 @@ PH_HD uint64_t sum_pm(uint64_t s0, uint64_t s1, uint64_t s2, uint32_t c1) {
   return uint64_t(uint32_t(s2)) * c1 + uint64_t(uint32_t(u >> 28)) * c1 + (((s1 & kLow30) << 30) | (s0 & kLow30)) +
          ((u & 0xfffffffull) << 32);
 }
-// Canonical residue of any x < 2^64: x mod 2^b + (x >> b) c < q + 2^32.
+// Canonical residue of any x < 2^64: x mod 2^b + (x >> b) c < q + c + 2^35 < 2q (pm_bits:
+// c 2^(60-b) < 2^31).
 PH_HD uint64_t canon_pm(uint64_t x, uint64_t q, uint32_t c, unsigned sh) {  // sh = b - 32
   const uint32_t hi = uint32_t(x >> 32);
   const uint64_t r = uint64_t(hi >> sh) * c + ((uint64_t(hi & ((1u << sh) - 1)) << 32) | uint32_t(x));

@@ -469,8 +469,10 @@ void praghip_enc0_destroy(praghip_enc0_plan* p) { delete p; }
 // 2 x levels switching keys of the acyclic packing tree held on the device.
 // A pair at level l is  ks_{l,0}(L + x^s R) + ks_{l,1}(sigma_g(L - x^s R)),
 // s = N >> (l + 1), g = 2^(l+1) + 1 (switch.cu:49-61, 157-185).  Both switches
-// of every pair in a call run as ONE batched keyswitch: the prepared sums
-// first, then the Galois-mapped differences, each half sharing its key.
+// of fewer than 32 pairs run as one batched keyswitch - the prepared sums first,
+// then the Galois-mapped differences, each half sharing its key - and their
+// outputs are added; from 32 pairs on (pack_run) the sums are switched into the
+// output and the differences, in a second keyswitch, added to it.
 struct praghip_pack_plan {
   int device = -1;
   unsigned log_n = 0;

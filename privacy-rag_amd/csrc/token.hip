@@ -136,8 +136,10 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
           for (int k = 0; k < KL; ++k) {
             if (b % 16) {
-              // sixteen products of s2 and both carries of s1 stay below 2^64:
-              // 16 (2^30 - 1)^2 + 2 (2^34 - 31) + 16 = 2^64 - 30
+              // sixteen products of s2 and both carries of s1 stay below 2^64: s1
+              // restarts below 2^32 after a fold, so this carry is at most 2^34 - 28
+              // and the fold's (with s0's) at most 2^34 - 16, and
+              // 16 (2^30 - 1)^2 + 2^35 - 44 = 2^64 - 28
               s2[c][k] += s1[c][k] >> 30;
               s1[c][k] &= kLow30;
             } else {  // below 2^62: s1 restarts below 2^32
@@ -217,7 +219,7 @@ hipError_t launch_token_mac(const uint64_t* in, const uint64_t* w, uint64_t* out
     else if (mode == kMacPm && (!b || ((1ull << 60) - (m[i].q << (60 - b))) >> 28))
       mode = kMacNarrow;
   }
-  // limbs of one prime: 2 per thread for a single ciphertext's, else 4 (24
+  // limbs of one prime: 2 per thread for a single ciphertext's, else 4 (their 48
   // 64-bit sums are 96 registers; 8 limbs would leave two waves per SIMD)
   const unsigned per = unsigned((limbs + size_t(primes) - 1) / size_t(primes)), kl = per <= 2 ? 2 : 4;
   const unsigned tiles = (per + kl - 1) / kl, groups = unsigned((coords + kMacCoords - 1) / kMacCoords);

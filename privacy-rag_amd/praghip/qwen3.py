@@ -85,7 +85,8 @@ class Qwen3LocalGemms:
         return self.shape.layers * self.shape.ops_per_layer(self.rows)
 
     def forward(self, stream=None):
-        """Every local product of the forward, in layer order, on one stream."""
+        """Every local product of the forward, as one batch on one stream (their
+        operands are apart, so they run together and in any order)."""
         check(lib().praghip_share_gemm_batch(self.device.index or 0, ctypes.cast(self._descs, ctypes.c_void_p),
                                              len(self._descs), stream_handle(stream)))
 
