@@ -44,7 +44,7 @@ TRAFFIC_SOURCES = {
     "keyswitch_reference": ("keyswitch_n16384_locked_dnum6_batch64.md", r"ks_", 1),
     "gemm": ("share_gemm_512x1024x3072_i8.md", r"share_gemm_dma_kernel", 1),
     "gemm_f12": ("share_gemm_512x1024x3072_f12.md", r"share_gemm_dma_kernel|gemm_clear_kernel", 1),
-    "qwen3": ("qwen3_0.6b_local_gemms_28_layers.md", r"share_gemm_dma_kernel", None),
+    "qwen3": ("qwen3_0.6b_local_gemms_28_layers.md", r"share_gemm_group_kernel", 28),  # 112 products in 4 launches
 }
 
 
@@ -266,7 +266,7 @@ def bench_qwen3(torch, praghip, steps, warmup):
             "ops_per_forward": m.ops,
             "roofline": {"bound": "mfma", "achieved": round(8 * tops, 2), "peak": I8_PEAK_TOPS, "unit": "TFLOP/s",
                          "frac": round(8 * tops / I8_PEAK_TOPS, 4), "traffic": measured_traffic("qwen3"),
-                         "kernel": "share_gemm_dma_kernel over the 112 products (i8 MFMA ops executed); "
+                         "kernel": "share_gemm_group_kernel over the 112 products (i8 MFMA ops executed); "
                                    "traffic is the average per product"},
             "_model": m}
 
