@@ -83,7 +83,7 @@ def test_gemm_c4_full_shape(gpu):
 def test_gemm_split_k_shapes(gpu, m, k, n):
     """Shapes whose tiles leave most workgroup slots empty run split-K (64-bit
     atomic accumulation into a zeroed y, then the 59-bit mask): the Qwen3 o
-    and down products, and a long-K thin case."""
+    and down products; and a long-K thin case, on the few-row kernel."""
     print(f"[gemm] split-K m={m} k={k} n={n}", flush=True)
     x = oracle.fill_u64(m * k, 5000 + k).reshape(m, k)
     w = oracle.fill_i8(n * k, 6000 + k).reshape(n, k)
